@@ -1,0 +1,627 @@
+"""The work a user of phybs_amd has it do, as measurable cases, each through the public binding.
+
+A case is a dict of plain values; listed() gives the standing ones, draw(rng) one more of the same
+ranges.  prepare(case, seed) builds what a program holds before the call (mesh, solver handle,
+initial state, samples), run(state) is one call, work(case) the bytes and operations it cannot do
+without, exact(case, seed) the same result in 64 bits from plain torch.
+
+Meshes are bars of nx x ny x nz cubes, 6 tets per cube, clamped on the face x = 0, whose interior
+rest positions are moved by up to 8 % of the edge so that no two tets are alike.  The state a step
+starts from is a bar in motion: a twist about the long axis, a smooth displacement and a smooth
+velocity field of random phases.
+"""
+import itertools
+import math
+
+import numpy as np
+import torch
+
+import phybs_amd as P
+
+EDGE = 0.05
+DT = 1.0 / 30.0
+GRAV = (0.0, -9.8, 0.0)
+
+
+# ---- the cases ----
+def listed():
+    return [
+        # one frame of an interactive session on a small model: external forces in, positions out,
+        # the solver's default 96 iterations; launches and latency are everything
+        dict(name="frame-1.5k-f32", kind="descent", nx=4, ny=4, nz=16, precision=32, material=0, iterations=96, ext=True),
+        # a step solved to a gradient tolerance at the smaller of the two headline sizes
+        dict(name="relgrad-43k-f64", kind="relgrad", nx=12, ny=12, nz=50, material=0, mixed=0.0),
+        # the same at the larger headline size (6,291,456 tets)
+        dict(name="relgrad-6.3m-f64", kind="relgrad", nx=64, ny=64, nz=256, material=0, mixed=0.0),
+        # a fixed-iteration step of the large bar in the default precision, as a simulation loop runs it
+        dict(name="step-6.3m-f32", kind="descent", nx=64, ny=64, nz=256, precision=32, material=0, iterations=64, ext=False),
+        # the stretch material on a ragged middle-sized mesh
+        dict(name="step-stretch-1.3m-f32", kind="descent", nx=37, ny=41, nz=149, precision=32, material=1, iterations=64, ext=True),
+        # many small bars of different sizes and materials stepped together
+        dict(name="batch-64-bars-f32", kind="batch", instances=64, lo=8, hi=16, zlo=24, zhi=64, precision=32, iterations=32),
+        # one backward-Euler step: assembly and conjugate gradients
+        dict(name="implicit-1.5m-f32", kind="implicit", nx=40, ny=40, nz=160, precision=32, material=0),
+        # one projective-dynamics step on a ragged mesh
+        dict(name="pd-0.7m-f32", kind="pd", nx=33, ny=29, nz=127, precision=32),
+        # the material calls a host-side integrator makes: forces, energies, stiffness diagonal
+        dict(name="material-200k-f32", kind="material", nx=24, ny=23, nz=61, precision=32, material=0),
+        # one epoch of training the warm-start network on collected samples
+        dict(name="train-64k", kind="train", samples=65536, batch=8192, steps=8),
+        # loss and gradient of one ragged mini-batch
+        dict(name="lossgrad-5k", kind="lossgrad", samples=5003),
+        # the network's predictions for the nodes of a middle-sized mesh
+        dict(name="forward-250k", kind="forward", samples=250007),
+    ]
+
+
+def _dims(rng, lo, hi):
+    """A bar of about exp(uniform(log lo, log hi)) tets, ragged, two to six times as long as wide."""
+    tets = math.exp(rng.uniform(math.log(lo), math.log(hi)))
+    long = rng.uniform(2.0, 6.0)
+    w = (tets / (6.0 * long)) ** (1.0 / 3.0)
+    nx = max(2, round(w * rng.uniform(0.8, 1.25)))
+    ny = max(2, round(w * rng.uniform(0.8, 1.25)))
+    nz = max(4, round(tets / (6.0 * nx * ny)))
+    return nx, ny, nz
+
+
+def draw(rng):
+    kind = rng.choice(["descent", "descent", "descent", "relgrad", "batch", "implicit", "pd", "material", "train",
+                       "lossgrad", "forward"])
+    if kind == "descent":
+        nx, ny, nz = _dims(rng, 1.0e3, 3.0e6)
+        return dict(kind=kind, nx=nx, ny=ny, nz=nz, precision=rng.choice([32, 32, 64]), material=rng.choice([0, 0, 1]),
+                    iterations=rng.choice([32, 64, 96]), ext=rng.random() < 0.5)
+    if kind == "relgrad":
+        nx, ny, nz = _dims(rng, 3.0e3, 2.0e5)
+        return dict(kind=kind, nx=nx, ny=ny, nz=nz, material=0, mixed=rng.choice([0.0, 0.0, 2e-4]))
+    if kind == "batch":
+        lo = rng.randint(4, 9)
+        zlo = rng.randint(12, 30)
+        return dict(kind=kind, instances=rng.randint(3, 64), lo=lo, hi=lo + rng.randint(2, 7), zlo=zlo,
+                    zhi=zlo + rng.randint(4, 34), precision=rng.choice([32, 32, 64]), iterations=rng.choice([32, 64]))
+    if kind == "implicit":
+        nx, ny, nz = _dims(rng, 1.0e4, 1.2e6)
+        return dict(kind=kind, nx=nx, ny=ny, nz=nz, precision=rng.choice([32, 64]), material=rng.choice([0, 0, 1]))
+    if kind == "pd":
+        nx, ny, nz = _dims(rng, 1.0e4, 7.0e5)
+        return dict(kind=kind, nx=nx, ny=ny, nz=nz, precision=rng.choice([32, 64]))
+    if kind == "material":
+        nx, ny, nz = _dims(rng, 1.0e3, 5.0e5)
+        return dict(kind=kind, nx=nx, ny=ny, nz=nz, precision=rng.choice([32, 64]), material=rng.choice([0, 1]))
+    if kind == "train":
+        batch = round(math.exp(rng.uniform(math.log(512), math.log(16384))))
+        steps = rng.randint(2, 8)
+        return dict(kind=kind, samples=max(batch * steps - rng.randint(0, batch - 1), 33), batch=batch, steps=steps)
+    if kind == "lossgrad":
+        return dict(kind=kind, samples=round(math.exp(rng.uniform(math.log(65), math.log(60000)))))
+    return dict(kind="forward", samples=round(math.exp(rng.uniform(math.log(300), math.log(500000)))))
+
+
+# ---- inputs, from the seed alone ----
+def _bar(nx, ny, nz, rng):
+    """Rest positions (N, 3) float32, tets (T, 4) int32, mask (N,) int32 of a bar."""
+    k, j, i = np.meshgrid(np.arange(nz + 1), np.arange(ny + 1), np.arange(nx + 1), indexing="ij")
+    idx = np.stack([i, j, k], -1).reshape(-1, 3)
+    top = np.array([nx, ny, nz])
+    inner = ((idx > 0) & (idx < top)).astype(np.float32)
+    rest = (idx * EDGE + inner * rng.uniform(-0.08 * EDGE, 0.08 * EDGE, idx.shape)).astype(np.float32)
+    ck, cj, ci = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
+    base = (ci + (nx + 1) * (cj + (ny + 1) * ck)).reshape(-1).astype(np.int32)
+    step = np.array([1, nx + 1, (nx + 1) * (ny + 1)])
+    tets = []
+    for p in itertools.permutations(range(3)):
+        odd = ((p[0] > p[1]) + (p[0] > p[2]) + (p[1] > p[2])) % 2
+        o = [0, step[p[0]], step[p[0]] + step[p[1]], step.sum()]
+        if odd:
+            o[2], o[3] = o[3], o[2]
+        tets.append(np.stack([base + np.int32(v) for v in o], -1))
+    return rest, np.ascontiguousarray(np.stack(tets, 1).reshape(-1, 4)), (idx[:, 0] == 0).astype(np.int32)
+
+
+def _field(rest, rng, size):
+    """A smooth vector field of two random waves per component, about `size` large, zero at x = 0."""
+    r = rest.astype(np.float64)
+    span = np.maximum(r.max(0), EDGE)
+    ramp = r[:, 0] / span[0]
+    out = np.empty_like(r)
+    for d in range(3):
+        a, b = rng.uniform(-1.0, 1.0, 2)
+        w = rng.uniform(0.5, 2.0, 2)
+        ph = rng.uniform(0.0, 2.0 * math.pi, 2)
+        out[:, d] = a * np.sin(math.pi * w[0] * r[:, 2] / span[2] + ph[0]) + b * np.sin(math.pi * w[1] * r[:, 1] / span[1] + ph[1])
+    return size * ramp[:, None] * out
+
+
+def _motion(rest, rng):
+    """(x, v, v_last) float32 of a bar in motion."""
+    x = rest + _field(rest, rng, 0.2 * EDGE)
+    v = _field(rest, rng, 0.2)
+    return x.astype(np.float32), v.astype(np.float32), (0.97 * v).astype(np.float32)
+
+
+def _pull(rest, rng):
+    """External forces (N, 3) float32: a patch of free nodes is pulled."""
+    f = np.zeros_like(rest)
+    far = np.flatnonzero(rest[:, 0] > 0)
+    at = rng.choice(far, max(1, len(far) // 50), replace=False)
+    f[at] = rng.uniform(-2.0, 2.0, 3)
+    return f
+
+
+def _mesh_inputs(case, seed):
+    rng = np.random.default_rng([int(seed), 11])
+    rest, tets, mask = _bar(case["nx"], case["ny"], case["nz"], rng)
+    x, v, vl = _motion(rest, rng)
+    ext = _pull(rest, rng) if case.get("ext") else None
+    return rest, tets, mask, x, v, vl, ext
+
+
+def _batch_inputs(case, seed):
+    rng = np.random.default_rng([int(seed), 13])
+    # the sizes are the case's own; the shapes, states and materials the seed's
+    size = np.random.default_rng([case["instances"], case["lo"], case["hi"], case["zlo"], case["zhi"]])
+    meshes, x, v, vl = [], [], [], []
+    for _ in range(case["instances"]):
+        nx, ny = size.integers(case["lo"], case["hi"] + 1, 2)
+        nz = size.integers(case["zlo"], case["zhi"] + 1)
+        m = _bar(int(nx), int(ny), int(nz), rng)
+        meshes.append(m)
+        for to, a in zip((x, v, vl), _motion(m[0], rng)):
+            to.append(a)
+    youngs = np.exp(rng.uniform(math.log(5e4), math.log(5e5), len(meshes))).astype(np.float32)
+    nu = rng.uniform(0.3, 0.46, len(meshes)).astype(np.float32)
+    return meshes, youngs, nu, np.concatenate(x), np.concatenate(v), np.concatenate(vl)
+
+
+def _samples(case, seed):
+    """Features in the six groups' usual magnitudes (displacement, h v, step, and their differences
+    from the neighbours' mean), a smooth target of them, network parameters and scales."""
+    rng = np.random.default_rng([int(seed), 17])
+    n = case["samples"]
+    group = np.array([0.02, 0.01, 0.012, 0.002, 0.001, 0.001], np.float32)
+    f = (rng.standard_normal((n, 18), np.float32) * np.repeat(group, 3)).astype(np.float32)
+    mix = rng.standard_normal((18, 3)).astype(np.float32)
+    z = f / np.repeat(group, 3)
+    t = (0.004 * np.tanh(0.3 * z @ mix + 0.1 * z[:, :3] * z[:, 3:6])).astype(np.float32)
+    params = []
+    for a, b in ((18, 64), (64, 64), (64, 64), (64, 3)):
+        params.append(rng.uniform(-1, 1, a * b) * math.sqrt(6.0 / (a + b)))
+        params.append(rng.uniform(-0.1, 0.1, b))
+    scales = np.append(group, np.float32(0.003)).astype(np.float32)
+    return f, t, np.concatenate(params).astype(np.float32), scales
+
+
+def _solver_params(case):
+    kw = dict(dt=DT, grav=GRAV, precision=case.get("precision", 64), material=case.get("material", 0))
+    if case["kind"] in ("descent", "batch"):
+        kw["iterations"] = case["iterations"]
+    if case["kind"] == "relgrad":
+        kw.update(relgrad_tol=1e-4, max_iterations=20000, mixed_switch=case["mixed"])
+    return P.default_params(**kw)
+
+
+# ---- what a program holds before the call ----
+def prepare(case, seed):
+    kind = case["kind"]
+    if kind == "batch":
+        meshes, youngs, nu, x, v, vl = _batch_inputs(case, seed)
+        s = P.Solver.batch(meshes, youngs, nu, _solver_params(case))
+        s.set_positions(x)
+        s.set_velocities(v, vl)
+        return dict(kind=kind, s=s)
+    if kind in ("train", "lossgrad", "forward"):
+        f, t, params, scales = _samples(case, seed)
+        rest, tets, mask = _bar(2, 2, 4, np.random.default_rng(1))
+        s = P.Solver(rest, tets, mask, P.default_params())
+        s.learn_set_model(params, scales)
+        if kind == "train":
+            s.learn_collect(len(f))
+            s.learn_add_samples(f, t)
+        return dict(kind=kind, s=s, f=f, t=t, params=params, scales=scales, batch=case.get("batch"))
+    rest, tets, mask, x, v, vl, ext = _mesh_inputs(case, seed)
+    s = P.Solver(rest, tets, mask, _solver_params(case))
+    s.set_positions(x)
+    s.set_velocities(v, vl)
+    return dict(kind=kind, s=s, x=x, v=v, vl=vl, ext=ext, iterations=case.get("iterations"))
+
+
+# ---- one call ----
+def run(state):
+    s, kind = state["s"], state["kind"]
+    if kind == "descent":  # the next step of a simulation
+        if state["ext"] is not None:
+            return s.do_descent_opt(DT, state["iterations"], state["ext"])
+        return s.step(want_positions=True)[1]
+    if kind == "batch":
+        return s.step(want_positions=True)[1]
+    if kind == "relgrad":  # a step solved from a given state
+        s.set_positions(state["x"])
+        s.set_velocities(state["v"], state["vl"])
+        s.step()
+        return s.positions(f64=True), s.velocities()[0]
+    if kind in ("implicit", "pd"):
+        s.set_positions(state["x"])
+        s.set_velocities(state["v"], state["vl"])
+        x = (s.implicit_step if kind == "implicit" else s.pd_step)(want_positions=True)[1]
+        return x, s.velocities()[0]
+    if kind == "material":
+        tf, nf, te = s.compute_forces(state["x"])
+        nh, th = s.compute_hessian_diag(state["x"])
+        return tf, nf, te, nh, th
+    if kind == "train":  # from the same initial network every time
+        s.learn_set_model(state["params"], state["scales"])
+        loss = s.learn_train(1, batch=state["batch"], lr=1e-3, seed=5)
+        return loss, s.learn_get_model()[0]
+    if kind == "lossgrad":
+        return s.learn_loss_grad(state["f"], state["t"])
+    return s.learn_forward(state["f"])
+
+
+# ---- what it cannot do without ----
+MLP_FLOPS = 2 * (18 * 64 + 64 * 64 + 64 * 64 + 64 * 3)
+
+
+def work(case):
+    kind = case["kind"]
+    if kind in ("train", "lossgrad", "forward"):
+        n = case["samples"]
+        if kind == "forward":
+            return dict(bytes=84 * n, flops=MLP_FLOPS * n)
+        return dict(bytes=84 * n, flops=3 * MLP_FLOPS * n)
+    if kind == "batch":
+        w, z = 0.5 * (case["lo"] + case["hi"]), 0.5 * (case["zlo"] + case["zhi"])
+        nt, nn = case["instances"] * 6 * w * w * z, case["instances"] * (w + 1) ** 2 * (z + 1)
+    else:
+        nx, ny, nz = case["nx"], case["ny"], case["nz"]
+        nt, nn = 6 * nx * ny * nz, (nx + 1) * (ny + 1) * (nz + 1)
+    r = 8 if kind == "relgrad" or case.get("precision") == 64 else 4
+    if kind == "material":
+        # connectivity and positions in, the per-tet and per-node results out, for each of the two calls
+        return dict(bytes=nt * (2 * 16 + 13 * 4 + 12 * 4) + nn * 4 * 12, flops=nt * 500)
+    if kind in ("implicit", "pd"):
+        # about 15 blocks a row; one pass over matrix and vectors per iteration, about as many
+        # iterations as the bar is nodes long (backward Euler), or 5 rounds of fewer
+        its = 2.0 * max(nx, ny, nz) if kind == "implicit" else 500
+        block = 9 * r + 4 if kind == "implicit" else r + 4
+        return dict(bytes=its * (15 * nn * block + 8 * 24 * nn), flops=its * 15 * nn * (18 if kind == "implicit" else 6))
+    passes = case.get("iterations") or 1500
+    # a pass reads the connectivity and, per node, position, previous position, target, rest
+    # position, diagonal and mass, and writes the next position
+    return dict(bytes=passes * (16 * nt + nn * (12 * r + 28)), flops=passes * nt * (600 if case.get("material") else 220))
+
+
+# ---- the same in 64 bits, from plain torch ----
+DEV = "cuda" if torch.cuda.is_available() else "cpu"
+
+
+def _t(a, dtype=torch.float64):
+    return torch.as_tensor(np.ascontiguousarray(a), device=DEV).to(dtype)
+
+
+class _Body:
+    """Elastic body in float64; matrices are (9, T) rows of row-major 3x3 entries, vectors (3, T)."""
+
+    def __init__(self, rest, tets, mask, material=0, youngs=1e5, nu=0.45):
+        self.q = _t(tets, torch.int64).t().contiguous()
+        self.rest = _t(rest).t().contiguous()
+        self.free = (_t(mask) == 0).to(torch.float64)
+        self.n = self.rest.shape[1]
+        self.material = material
+        E, v = float(np.float32(youngs)), float(np.float32(nu))
+        self.mu = 0.5 * E / (1.0 + v)
+        self.lam = 2.0 * self.mu / (1.0 - 2.0 * v)
+        D = self.edges(self.rest)
+        self.Di, det = self.inverse(D)
+        self.vol = det.abs() / 6.0
+        m = torch.zeros(self.n, dtype=torch.float64, device=DEV)
+        for c in range(4):
+            m.index_add_(0, self.q[c], self.vol * (1000.0 / 4.0))
+        self.mfree = m  # before the override of fixed nodes
+        self.mass = torch.where(self.free > 0, m, torch.full_like(m, 1e8))
+        self.g = torch.tensor([float(np.float32(a)) for a in GRAV], dtype=torch.float64, device=DEV)[:, None]
+        self.c = [-(self.Di[0:3] + self.Di[3:6] + self.Di[6:9]), self.Di[0:3], self.Di[3:6], self.Di[6:9]]
+
+    def edges(self, x):
+        X = [x[:, self.q[c]] for c in range(4)]
+        return torch.stack([X[1 + j][k] - X[0][k] for k in range(3) for j in range(3)])
+
+    @staticmethod
+    def adj(A):
+        return torch.stack([A[4] * A[8] - A[7] * A[5], A[7] * A[2] - A[1] * A[8], A[1] * A[5] - A[4] * A[2],
+                            A[5] * A[6] - A[3] * A[8], A[0] * A[8] - A[2] * A[6], A[2] * A[3] - A[0] * A[5],
+                            A[3] * A[7] - A[4] * A[6], A[1] * A[6] - A[0] * A[7], A[0] * A[4] - A[1] * A[3]])
+
+    @classmethod
+    def inverse(cls, A):
+        C = cls.adj(A)
+        det = A[0] * C[0] + A[3] * C[1] + A[6] * C[2]
+        return C / det, det
+
+    @staticmethod
+    def mul(A, B):
+        return torch.stack([sum(A[3 * i + k] * B[3 * k + j] for k in range(3)) for i in range(3) for j in range(3)])
+
+    @staticmethod
+    def tr(A):
+        return A[[0, 3, 6, 1, 4, 7, 2, 5, 8]]
+
+    def rotation(self, F):
+        X = F
+        for _ in range(9):
+            Y, det = self.inverse(X)
+            Yt = self.tr(Y)
+            z = ((Yt * Yt).sum(0) / (X * X).sum(0)) ** 0.25
+            X = 0.5 * (z * X + Yt / z)
+        return X
+
+    def deform(self, x):
+        F = self.mul(self.edges(x), self.Di)
+        Fi, J = self.inverse(F)
+        return F, Fi, J
+
+    def stress(self, F, Fi, J):
+        """(P, psi, R): first Piola-Kirchhoff stress, energy density, rotation (stretch material)."""
+        if self.material == 0:
+            lj = J.log()
+            return (self.mu * F + (self.lam * lj - self.mu) * self.tr(Fi),
+                    0.5 * self.mu * ((F * F).sum(0) - 3.0) - self.mu * lj + 0.5 * self.lam * lj * lj, None)
+        R = self.rotation(F)
+        return (2.0 * self.mu * (F - R) + self.lam * (J - 1.0) * J * self.tr(Fi),
+                self.mu * ((F - R) ** 2).sum(0) + 0.5 * self.lam * (J - 1.0) ** 2, R)
+
+    def corner_forces(self, Pm):
+        """Per corner (3, T): -vol P c."""
+        return [torch.stack([-self.vol * (Pm[3 * a] * c[0] + Pm[3 * a + 1] * c[1] + Pm[3 * a + 2] * c[2]) for a in range(3)])
+                for c in self.c]
+
+    def gather(self, corners):
+        out = torch.zeros(3, self.n, dtype=torch.float64, device=DEV)
+        for c in range(4):
+            out.index_add_(1, self.q[c], corners[c])
+        return out
+
+    def diagonal(self, F, Fi, J, R):
+        """Per corner (3, T): the diagonal of -df/dx."""
+        out = []
+        if self.material != 0:
+            S = self.mul(self.tr(R), F)
+            t = S[0] + S[4] + S[8]
+            Gi, _ = self.inverse(torch.stack([t - S[0], -S[1], -S[2], -S[3], t - S[4], -S[5], -S[6], -S[7], t - S[8]]))
+        for c in self.c:
+            cc = (c * c).sum(0)
+            h = []
+            for d in range(3):
+                s = c[0] * Fi[d] + c[1] * Fi[3 + d] + c[2] * Fi[6 + d]
+                if self.material == 0:
+                    h.append(self.vol * (self.mu * cc + (self.mu + self.lam - self.lam * J.log()) * s * s))
+                else:
+                    w = torch.cross(c, R[3 * d:3 * d + 3], dim=0)
+                    rot = sum(w[i] * Gi[3 * i + j] * w[j] for i in range(3) for j in range(3))
+                    h.append(self.vol * (2.0 * self.mu * (cc - rot) + self.lam * J * J * s * s))
+            out.append(torch.stack(h))
+        return out
+
+
+def _cheb(k, rho, om):
+    if k == 0:
+        rho, om = 0.0, 1.0
+    om = 4.0 / (4.0 - rho * rho * om)
+    for kk, rr in ((1, 0.96), (7, 0.991), (10, 0.999)):
+        if k == kk - 1:
+            rho, om = 0.0, 1.0
+        if k == kk:
+            rho = rr
+            om = 2.0 / (2.0 - rho * rho)
+            break
+    return rho, om
+
+
+def _descend(b, x, v, vl, ext, iterations, tol=0.0):
+    """One step: (positions, velocities) (3, N)."""
+    h = float(np.float32(DT))
+    free = b.free > 0
+    xt = x + h * v
+    cur = xt + float(np.float32(0.2)) * (v - vl) * h
+    mh2 = b.mfree / (h * h)
+    fe = b.g * b.mfree + (ext if ext is not None else 0.0)
+    alpha, k, kc, budget = float(np.float32(0.1)), 0, 0, 20000 if tol else iterations
+    rho = om = 0.0
+    last = old = cur
+    e_old = g0 = None
+    hd = torch.zeros_like(cur)
+    rho, om = _cheb(0, 0.0, 1.0)
+    while True:
+        F, Fi, J = b.deform(cur)
+        Pm, psi, R = b.stress(F, Fi, J)
+        f = b.gather(b.corner_forces(Pm))
+        if k % 32 == 0:
+            hd = b.gather(b.diagonal(F, Fi, J, R))
+        dd = cur - xt
+        g = (dd * mh2 - f - fe) * b.free
+        if tol:
+            gn = float(g.norm())
+            g0 = gn if g0 is None else g0
+            if gn <= tol * g0:
+                break
+        rolled = False
+        if k % 8 == 0:
+            e = float((psi * b.vol).clamp(min=0.0).sum() + ((0.5 * dd * dd * mh2 - fe * cur) * b.free).sum())
+            if k and e_old is not None and not e <= e_old:
+                alpha *= float(np.float32(0.7))
+                if tol:
+                    kc = k
+                else:
+                    budget -= k - 8
+                cur, rolled = old, True
+            else:
+                e_old, old = e, cur
+        if not rolled:
+            nx = cur - alpha * g / (hd + mh2)
+            if om != 1.0:
+                nx = om * (nx - last) + last
+            nx = torch.where(free, nx, cur)
+            last, cur = cur, nx
+            k += 1
+            done = (rho, om)
+        if alpha < 0.01 or not k < budget:
+            break
+        # the schedule of the next iteration, from the state of the last accepted one
+        rho, om = _cheb(k - kc, *(done if k else (0.0, 1.0)))
+    vn = (v + (cur - xt) / h) * float(np.float32(0.99))
+    return cur, torch.where(free, vn, v)
+
+
+def _cg(apply, rhs, x, diag, tol, most):
+    """Jacobi-preconditioned conjugate gradients."""
+    r = rhs - apply(x)
+    z = r / diag
+    p = z.clone()
+    rz = float((r * z).sum())
+    stop = tol * tol * float((rhs * rhs / diag).sum())
+    for k in range(most):
+        if rz <= stop:
+            break
+        ap = apply(p)
+        a = rz / float((p * ap).sum())
+        x = x + a * p
+        r = r - a * ap
+        z = r / diag
+        rz, was = float((r * z).sum()), rz
+        p = z + (rz / was) * p
+    return x
+
+
+def _implicit(b, x, v):
+    h = float(np.float32(DT))
+    al, be = float(np.float32(0.02)), float(np.float32(0.02))
+    F, Fi, J = b.deform(x)
+    Pm, _, R = b.stress(F, Fi, J)
+    f = b.gather(b.corner_forces(Pm)) + b.g * b.mfree
+    f = torch.where(b.free > 0, f, 1e8 * (b.rest - x))
+    ms = b.mass * (1.0 + al * h)
+    s = (h + be) * h
+    if b.material != 0:
+        S = b.mul(b.tr(R), F)
+        t = S[0] + S[4] + S[8]
+        Gi, _ = b.inverse(torch.stack([t - S[0], -S[1], -S[2], -S[3], t - S[4], -S[5], -S[6], -S[7], t - S[8]]))
+        Rt = b.tr(R)
+    lj = J.log()
+    FiT = b.tr(Fi)
+
+    def apply(u):
+        dF = b.mul(b.edges(u), b.Di)
+        W = b.mul(Fi, dF)  # F^-1 dF
+        tW = W[0] + W[4] + W[8]
+        FWT = b.mul(FiT, b.tr(b.mul(dF, Fi)))  # F^-T dF^T F^-T
+        if b.material == 0:
+            dP = b.mu * dF + (b.mu - b.lam * lj) * FWT + b.lam * tW * FiT
+        else:
+            K = b.mul(Rt, dF)
+            w = torch.stack([K[7] - K[5], K[2] - K[6], K[3] - K[1]])
+            o = torch.stack([sum(Gi[3 * i + j] * w[j] for j in range(3)) for i in range(3)])
+            z = torch.zeros_like(o[0])
+            dR = b.mul(R, torch.stack([z, -o[2], o[1], o[2], z, -o[0], -o[1], o[0], z]))
+            dP = 2.0 * b.mu * (dF - dR) + b.lam * ((2.0 * J - 1.0) * J * tW * FiT - (J - 1.0) * J * FWT)
+        return ms * u - s * b.gather(b.corner_forces(dP))
+
+    diag = ms + s * b.gather(b.diagonal(F, Fi, J, R))
+    u = _cg(apply, h * f + b.mass * v, v, diag, 1e-9, 4000)
+    return x + h * u, u
+
+
+def _pd(b, x, v):
+    h = float(np.float32(DT))
+    w = 1e6 * b.vol
+    im = b.free / b.mass
+    rhs0 = (x + h * v + h * h * im * (b.g * b.mfree)) * b.mass / (h * h)
+    m = b.mass / (h * h)
+    diag = m + b.gather([(w * (c * c).sum(0)).expand(3, -1) for c in b.c])
+
+    def apply(u):
+        A = b.mul(b.edges(u), b.Di)
+        return m * u + b.gather([torch.stack([w * (A[3 * a] * c[0] + A[3 * a + 1] * c[1] + A[3 * a + 2] * c[2])
+                                              for a in range(3)]) for c in b.c])
+
+    cur = x
+    for _ in range(5):
+        R = b.rotation(b.mul(b.edges(cur), b.Di))
+        rhs = rhs0 + b.gather([torch.stack([w * (R[3 * a] * c[0] + R[3 * a + 1] * c[1] + R[3 * a + 2] * c[2])
+                                            for a in range(3)]) for c in b.c])
+        cur = _cg(apply, rhs, cur, diag, 1e-12, 4000)
+    return cur, (cur - x) / h * float(np.float32(0.99))
+
+
+def _bf(a):
+    return a.to(torch.bfloat16).to(torch.float64)
+
+
+class _Round(torch.autograd.Function):
+    """The network's BF16 rounding of inputs, weights and activations, straight through."""
+
+    @staticmethod
+    def forward(ctx, a):
+        return _bf(a.float())
+
+    @staticmethod
+    def backward(ctx, g):
+        return g
+
+
+def _network(p, f, inv):
+    hcur = _bf((f * inv).float())
+    at = 0
+    for a, c in ((18, 64), (64, 64), (64, 64), (64, 3)):
+        w = p[at:at + a * c].reshape(a, c)
+        z = hcur @ _Round.apply(w) + p[at + a * c:at + a * c + c]
+        at += a * c + c
+        hcur = _Round.apply(torch.nn.functional.silu(z)) if c == 64 else z
+    return hcur
+
+
+def _learn(case, seed):
+    f, t, params, scales = _samples(case, seed)
+    inv = _t(np.repeat(np.float32(1.0) / scales[:6], 3))
+    f, t = _t(f), _t(t) * float(np.float32(1.0) / scales[6])
+    p = _t(params)
+    if case["kind"] == "forward":
+        return _network(p, f, inv).float().cpu().numpy()
+    if case["kind"] == "train":
+        return None  # the library's own order of the samples, epoch by epoch
+    p.requires_grad_(True)
+    loss = ((_network(p, f, inv) - t) ** 2).mean()
+    loss.backward()
+    return float(loss.detach()), p.grad.cpu().numpy()
+
+
+def exact(case, seed):
+    kind = case["kind"]
+    if kind in ("train", "lossgrad", "forward"):
+        return _learn(case, seed)
+    if kind == "batch":
+        meshes, youngs, nu, x, v, vl = _batch_inputs(case, seed)
+        out, at = [], 0
+        for (rest, tets, mask), e, u in zip(meshes, youngs, nu):
+            b = _Body(rest, tets, mask, 0, e, u)
+            part = [_t(a[at:at + len(rest)]).t().contiguous() for a in (x, v, vl)]
+            out.append(_descend(b, *part, None, case["iterations"])[0].t().cpu().numpy())
+            at += len(rest)
+        return np.concatenate(out)
+    if kind == "relgrad" and case["nx"] * case["ny"] * case["nz"] > 200000:
+        return None  # thousands of passes over millions of tets
+    rest, tets, mask, x, v, vl, ext = _mesh_inputs(case, seed)
+    b = _Body(rest, tets, mask, case.get("material", 0))
+    X, V, VL = (_t(a).t().contiguous() for a in (x, v, vl))
+    if kind == "descent":
+        return _descend(b, X, V, VL, None if ext is None else _t(ext).t(), case["iterations"])[0].t().cpu().numpy()
+    if kind == "relgrad":
+        return tuple(a.t().cpu().numpy() for a in _descend(b, X, V, VL, None, 0, 1e-4))
+    if kind == "implicit":
+        return tuple(a.t().cpu().numpy() for a in _implicit(b, X, V))
+    if kind == "pd":
+        return tuple(a.t().cpu().numpy() for a in _pd(b, X, V))
+    F, Fi, J = b.deform(X)
+    Pm, psi, R = b.stress(F, Fi, J)
+    cf, ch = b.corner_forces(Pm), b.diagonal(F, Fi, J, R)
+    rows = lambda c: torch.cat(c).t().cpu().numpy()
+    return (rows(cf), b.gather(cf).t().cpu().numpy(), (psi * b.vol).cpu().numpy(), b.gather(ch).t().cpu().numpy(), rows(ch))
