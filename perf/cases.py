@@ -134,9 +134,11 @@ def _field(rest, rng, size):
 
 
 def _motion(rest, rng):
-    """(x, v, v_last) float32 of a bar in motion."""
-    x = rest + _field(rest, rng, 0.2 * EDGE)
-    v = _field(rest, rng, 0.2)
+    """(x, v, v_last) float32 of a bar in motion: strains and strains per step of a few per cent at
+    most, whatever the bar's size, so that its stiffness matrix stays positive definite."""
+    width = float(rest.max(0).min())
+    x = rest + _field(rest, rng, 0.004 * width)
+    v = _field(rest, rng, 0.06 * width)
     return x.astype(np.float32), v.astype(np.float32), (0.97 * v).astype(np.float32)
 
 
