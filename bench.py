@@ -347,7 +347,7 @@ def implicit_report(P, rest, tets, mask, material, grav, steps=3):
     nblocks = P.lib().pbs_csr_pattern(len(rest), len(t32), t32.ctypes.data, None, None, None, None) // 9
     nn = len(rest)
     spmv_bytes = nblocks * (9 * 4 + 4) + 2 * 24 * nn
-    upd_bytes = 8 * 24 * nn
+    upd_bytes = 9 * 24 * nn  # the two vector passes: x, p, z (twice), Ap, D^-1 read; x, p, z written
     spmv_ms, upd_ms = kt["k_ie_spmv"][0], kt["k_ie_update"][0]
     ach = spmv_bytes / (spmv_ms * 1e-3) / 1e9 if spmv_ms > 0 else 0.0
     return {

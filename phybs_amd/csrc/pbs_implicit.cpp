@@ -99,10 +99,12 @@ int implicit_get(pbs_solver *s, ImplicitState **out) {
   }
   const size_t rsz = s->p.precision == PBS_FP64 ? 8 : 4;
   const size_t n3 = 3 * (size_t)N;
-  const int nb = (3 * N + 255) / 256;  // partial sums: up to one per 256 vector entries
+  // partial sums: the SpMV has at most one block per slice, the start kernel one per 4 slices, the
+  // vector passes one per 1024 entries of 3N
   IeDev &d = S->dev;
   d.n = N;
   d.nslice = S->nslice;
+  ie_vec_split(d);
   int *so = nullptr, *rl = nullptr, *bc = nullptr, *dsl = nullptr;
   char *A = nullptr;
   int rc = ialloc(S, &so, S->nslice + 1);
@@ -110,10 +112,11 @@ int implicit_get(pbs_solver *s, ImplicitState **out) {
   if (!rc) rc = ialloc(S, &bc, S->slots);
   if (!rc) rc = ialloc(S, &dsl, N);
   if (!rc) rc = ialloc(S, &A, 9 * rsz * S->slots);
-  double **vec[7] = {&d.b, &d.x, &d.r, &d.z, &d.p, &d.Ap, &d.dinv};
-  for (int i = 0; i < 7 && !rc; ++i) rc = ialloc(S, vec[i], n3);
-  if (!rc) rc = ialloc(S, &d.part, 4 * (size_t)nb);
-  if (!rc) rc = ialloc(S, &d.ctrl, 1);
+  double **vec[6] = {&d.b, &d.x, &d.z, &d.p, &d.Ap, &d.dinv};
+  for (int i = 0; i < 6 && !rc; ++i) rc = ialloc(S, vec[i], n3);
+  if (!rc) rc = ialloc(S, &d.part_rz, (size_t)S->nslice);
+  if (!rc) rc = ialloc(S, &d.part_pap, (size_t)S->nslice);
+  if (!rc) rc = ialloc(S, &d.ctrl, 2);
   if (rc) {
     implicit_release(S);
     return rc;
@@ -136,10 +139,11 @@ int implicit_get(pbs_solver *s, ImplicitState **out) {
   return PBS_OK;
 }
 
-// Timing events: 4 per CG iteration of a replay (SpMV and update dispatches), 2 around the
-// assembly or the local step.
+// Timing events: 6 per CG iteration of a replay (its three dispatches), 2 around the assembly or
+// the local step.
+constexpr int kIterEvents = 6;
 static int cg_events(ImplicitState *S) {
-  while (S->ev.size() < 4 * (size_t)kGraphIters + 2) {
+  while (S->ev.size() < kIterEvents * (size_t)kGraphIters + 2) {
     hipEvent_t ev;
     HIPCHK(hipEventCreate(&ev));
     S->ev.push_back(ev);
@@ -157,10 +161,9 @@ template <typename R> int cg_graph(pbs_solver *s, const IeDev &dev, CgGraphs &G)
   HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
   hipError_t err = hipSuccess;
   for (int i = 0; i < kGraphIters && err == hipSuccess; ++i) {
+    IeLaunch<R>::dir(dev, s->st);
     IeLaunch<R>::spmv(dev, s->st);
-    IeLaunch<R>::alpha(dev, s->st);
-    IeLaunch<R>::update(dev, s->st);
-    IeLaunch<R>::beta(dev, s->st);
+    IeLaunch<R>::res(dev, s->st);
     err = hipGetLastError();
   }
   hipGraph_t gr = nullptr;
@@ -176,7 +179,7 @@ template <typename R> int cg_graph(pbs_solver *s, const IeDev &dev, CgGraphs &G)
 
 // Solves dev's system from the start vector in dev.x (b, dinv already set): the start kernels,
 // then graph replays until the device-side test stops; with profiling on, the same iterations are
-// launched eagerly instead, the SpMV and update dispatches carrying their own start and end
+// launched eagerly instead, each dispatch carrying its own start and end
 // events.  c receives the final control block.
 template <typename R>
 int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double tol, int maxit, IeCtrl &c) {
@@ -196,10 +199,10 @@ int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double to
     const int k_before = c.k;
     if (timed) {
       for (int i = 0; i < kGraphIters; ++i) {
-        IeLaunch<R>::spmv(dev, s->st, S->ev[4 * i], S->ev[4 * i + 1]);
-        IeLaunch<R>::alpha(dev, s->st);
-        IeLaunch<R>::update(dev, s->st, S->ev[4 * i + 2], S->ev[4 * i + 3]);
-        IeLaunch<R>::beta(dev, s->st);
+        hipEvent_t *e = &S->ev[kIterEvents * i];
+        IeLaunch<R>::dir(dev, s->st, e[0], e[1]);
+        IeLaunch<R>::spmv(dev, s->st, e[2], e[3]);
+        IeLaunch<R>::res(dev, s->st, e[4], e[5]);
       }
       HIPCHK(hipGetLastError());
     } else {
@@ -207,17 +210,17 @@ int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double to
     }
     HIPCHK(hipMemcpyAsync(&c, dev.ctrl, sizeof(IeCtrl), hipMemcpyDeviceToHost, s->st));
     HIPCHK(hipStreamSynchronize(s->st));
-    if (timed) {  // iterations that ran: k advanced by one per completed iteration (+1 if stopped in alpha)
-      const int ran = std::min(kGraphIters, c.k - k_before + (c.indefinite ? 1 : 0));
+    if (timed) {  // iterations that ran: k advances by one per iteration
+      const int ran = std::min(kGraphIters, c.k - k_before);
       for (int i = 0; i < ran; ++i) {
-        float ms = 0.f;
-        if (hipEventElapsedTime(&ms, S->ev[4 * i], S->ev[4 * i + 1]) == hipSuccess) {
+        hipEvent_t *e = &S->ev[kIterEvents * i];
+        float ms = 0.f, ms2 = 0.f;
+        if (hipEventElapsedTime(&ms, e[2], e[3]) == hipSuccess) {
           s->kt_ms[K_IE_SPMV] += ms;
           s->kt_n[K_IE_SPMV] += 1;
         }
-        if (c.indefinite && i == ran - 1) break;
-        if (hipEventElapsedTime(&ms, S->ev[4 * i + 2], S->ev[4 * i + 3]) == hipSuccess) {
-          s->kt_ms[K_IE_UPDATE] += ms;
+        if (hipEventElapsedTime(&ms, e[0], e[1]) == hipSuccess && hipEventElapsedTime(&ms2, e[4], e[5]) == hipSuccess) {
+          s->kt_ms[K_IE_UPDATE] += ms + ms2;  // the two vector passes of an iteration together
           s->kt_n[K_IE_UPDATE] += 1;
         }
       }
@@ -276,7 +279,7 @@ int implicit_step_impl(pbs_solver *s, const pbs_implicit_params *ip, const float
     if (rc) return rc;
   }
   HIPCHK(hipEventRecord(s->ev0, s->st));
-  hipEvent_t *ea = timed ? &S->ev[4 * kGraphIters] : nullptr;  // events around the assembly
+  hipEvent_t *ea = timed ? &S->ev[kIterEvents * kGraphIters] : nullptr;  // events around the assembly
   if (ea) HIPCHK(hipEventRecord(ea[0], s->st));
   IeLaunch<R>::assemble(m, s->td, s->dp, d, a, S->max_width, s->st);
   HIPCHK(hipGetLastError());
@@ -369,7 +372,7 @@ int pd_step_impl(pbs_solver *s, const pbs_pd_params *pp, const float *ext, float
     rc = cg_events(S);
     if (rc) return rc;
   }
-  hipEvent_t *ea = timed ? &S->ev[4 * kGraphIters] : nullptr;  // events around the local step
+  hipEvent_t *ea = timed ? &S->ev[kIterEvents * kGraphIters] : nullptr;  // events around the local step
   for (int it = 0; it < pp->iterations; ++it) {
     // local step at the current iterate (dev.x), global solve warm-started from it
     if (ea) HIPCHK(hipEventRecord(ea[0], s->st));

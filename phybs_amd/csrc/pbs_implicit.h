@@ -16,21 +16,22 @@ namespace pbs {
 // consecutive slot groups so that each of the 9 loads of a wavefront is one contiguous 256-byte
 // (FP32) access.  Padding slots have column = the row itself and zero values.
 struct IeCtrl {
-  double rz, pAp, alpha, beta, rr, bb, rr0, rz0;  // bb = b.D^-1.b
+  double rz, pAp, alpha, beta, bb, rz0;  // bb = b.D^-1.b
   int k, done, converged, indefinite;
 };
 
 struct IeDev {
   int n, nslice, maxit, scalar;    // scalar: one value per slot (block = value x identity)
+  int vec_per, vec_rem;            // vector passes: groups of 64 entries per block, blocks with one more
   double tol2;                     // (relative residual tolerance)^2
   const int *slice_off;            // nslice + 1, in slot groups of 64
   const int *row_len;              // N
   const int *bcol;                 // slots
   const int *diag_slot;            // N: slot index of each row's diagonal block
   void *A;                         // 9 x slots values of the solver's real type
-  double *b, *x, *r, *z, *p, *Ap, *dinv;  // 3N, node-major (x, y, z of a node together)
-  double *part;                    // 4 partial sums per 256-row block (per 256 entries in updates)
-  IeCtrl *ctrl;
+  double *b, *x, *z, *p, *Ap, *dinv;  // 3N, node-major (x, y, z of a node together)
+  double *part_rz, *part_pap;      // partial sums per block: r.z; p.Ap (at the start b.D^-1.b)
+  IeCtrl *ctrl;                    // 2: written in turn within an iteration, [0] at its end
 };
 
 // Constants of one assembly (scales of the system matrix, fixed-node spring, damping).
@@ -41,6 +42,8 @@ struct IeAsm {
   int has_ext;
 };
 
+void ie_vec_split(IeDev &d);  // sets vec_per, vec_rem from n
+
 template <typename R> struct IeLaunch {
   // max_width: the widest slice (slots per row)
   static void assemble(const DevMesh<R> &m, const TileDev &td, const DevParams &p, const IeDev &d, const IeAsm &a,
@@ -49,12 +52,11 @@ template <typename R> struct IeLaunch {
   // per-tet 12 x 12 stiffness of the solver tets ids[0 .. num) at positions x (planes), FP32 out
   static void tet_stiffness(const DevMesh<R> &m, const DevParams &p, const float *inst_mu, const float *inst_lam,
                             const R *x, int num, const int *ids, float *out, hipStream_t st);
-  // one CG iteration = spmv, alpha, update, beta (+ the search-direction update), each a kernel;
-  // e0, e1 (optional): events recording the start and end of the kernel's own dispatch
+  // one CG iteration = dir, spmv, res, each a kernel; e0, e1 (optional): events recording the start
+  // and end of the kernel's own dispatch
+  static void dir(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
   static void spmv(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-  static void alpha(const IeDev &d, hipStream_t st);
-  static void update(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-  static void beta(const IeDev &d, hipStream_t st);
+  static void res(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
   static void finish(const DevMesh<R> &m, const DevParams &p, float h, const IeDev &d, hipStream_t st);
   // projective dynamics: global matrix, momentum term + iterate start, local step, velocity update
   static void pd_matrix(const DevMesh<R> &m, const DevParams &p, float stiffness, const IeDev &d, hipStream_t st);

@@ -8,6 +8,8 @@
 // 3x12 stiffness strip of its corner in closed form and accumulates it into its own SELL-64
 // slots, so the assembly is deterministic and atomic-free; the solve is a Jacobi-preconditioned
 // conjugate gradient in FP64 whose scalars stay on the device.
+#include <algorithm>
+
 #include <hip/hip_ext.h>
 
 #include "pbs_device.h"
@@ -46,58 +48,50 @@ __device__ __forceinline__ double block_sum256(double v, double *lds) {
   return t;
 }
 
-// Sum of component c of the per-block partials, by one block of 1024 threads in a fixed order.
-template <int K>
-__device__ __forceinline__ void partial_sums(const double *part, int nb, const int (&c)[K], double *lds, double (&out)[K]) {
-  // per thread: part[4 i + c] for i = tid, tid + 1024, ... in that order, the loads of 8 terms
-  // issued before their additions (indices past the end clamped to the first, not added)
-  double v[K];
-#pragma unroll
-  for (int k = 0; k < K; ++k) v[k] = 0.0;
-  const int first = threadIdx.x;
-  for (int base = first; base < nb; base += 8 * 1024) {
-    double t[8][K];
+// Sum of nb per-block partials by one block of NT threads in a fixed order, in two halves so that
+// other loads can be issued in between: the first takes the thread's first 8 terms v[tid], v[tid +
+// NT], ... (indices past the end clamped, not added later), the second adds them, any further ones
+// and the block's threads; every thread of the block gets the sum.
+template <int NT> struct PartialSum {
+  double t[8];
+  __device__ __forceinline__ void load(const double *__restrict__ v, int nb, int base = 0) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int i = base + u * 1024 < nb ? base + u * 1024 : first;
+      const int i = base + u * NT + (int)threadIdx.x;
+      t[u] = v[i < nb ? i : nb - 1];
+    }
+  }
+  __device__ __forceinline__ double sum(const double *__restrict__ v, int nb, double *lds) {
+    double a = 0.0;
+    for (int base = 0;;) {
 #pragma unroll
-      for (int k = 0; k < K; ++k) t[u][k] = part[4 * (size_t)i + c[k]];
+      for (int u = 0; u < 8; ++u) a += base + u * NT + (int)threadIdx.x < nb ? t[u] : 0.0;
+      base += 8 * NT;
+      if (base >= nb) break;
+      load(v, nb, base);
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (base + u * 1024 < nb)
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = a;
+    __syncthreads();
+    double r = 0.0;
 #pragma unroll
-        for (int k = 0; k < K; ++k) v[k] += t[u][k];
+    for (int i = 0; i < NT / 64; ++i) r += lds[i];
+    return r;
   }
-#pragma unroll
-  for (int k = 0; k < K; ++k)
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_down(v[k], o, 64);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0)
-#pragma unroll
-    for (int k = 0; k < K; ++k) lds[16 * k + w] = v[k];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    double t = 0.0;
-    if (threadIdx.x == 0)
-      for (int i = 0; i < 16; ++i) t += lds[16 * k + i];
-    out[k] = t;
-  }
-  __syncthreads();
-}
+};
 
-// y += (row n of A) v.  BLK = 3: 3x3 blocks (9 values per slot); BLK = 1: one value per slot,
-// the block being that value times the 3x3 identity.  get(col, v0, v1, v2) supplies v at a column.
+// y += (row `lane` of the slice's A) v over the slots first, first + step, ... below the slice's
+// width.  BLK = 3: 3x3 blocks (9 values per slot); BLK = 1: one value per slot, the block being
+// that value times the 3x3 identity.  get(col, v0, v1, v2) supplies v at a column.
 template <typename R, int BLK, typename Get>
-__device__ __forceinline__ void row_apply(const IeDev &d, int n, Get get, double *y) {
+__device__ __forceinline__ void row_apply(const IeDev &d, int n, int first, int step, Get get, double *y) {
   const R *__restrict__ A = (const R *)d.A;
   // all lanes run to the slice width (padding slots hold zeros and the row's own column), so the
   // loop is uniform across the wavefront and can be unrolled to overlap its loads
   const int lane = n & 63, g0 = d.slice_off[n >> 6], width = d.slice_off[(n >> 6) + 1] - g0;
 #pragma unroll 2
-  for (int j = 0; j < width; ++j) {
+  for (int j = first; j < width; j += step) {
     const int col = d.bcol[(size_t)(g0 + j) * 64 + lane];
     double x0, x1, x2;
     get(col, x0, x1, x2);
@@ -413,18 +407,51 @@ __global__ void k_tet_stiffness(DevParams p, int num, const int *__restrict__ id
     }
 }
 
-// r = b - A x0, z = D^-1 r, p = z; partials r.z, r.r, b.D^-1.b.  The stopping test uses the
-// Jacobi-scaled norms |D^-1/2 r| = sqrt(r.z) and |D^-1/2 b|: fixed nodes carry a 1e8 mass and
-// spring, and in the plain 2-norm their rows would swamp the free nodes' residual.
+// ---------------------------------------------------------------------------------------------
+// Conjugate gradients.  An iteration is three launches, and the two inner products are finished by
+// the launch that needs them: every block of k_ie_dir sums the partials of r.z that k_ie_res left,
+// every block of k_ie_res those of p.Ap that k_ie_spmv left, each in the same fixed order, so no
+// launch of its own stands between two vector passes.  The partials, the control block and the
+// block's first vector entries are all requested before any of them is waited for.  The control
+// block is double-buffered: a launch reads the one and its block 0 writes the other, so no block
+// reads what another one of the same launch has written.
+//
+// z = D^-1 r is the only residual kept (r.z = z.z / D^-1), and x += alpha p is done by the pass that
+// reads p anyway, so the vectors cost 9 passes over 3N doubles per iteration.  Per iteration, 5
+// launches and 11 passes before: 20 K tets 20.3 -> 11.9 us (backward Euler), 729 K 29.5 -> 18.9 us
+// (projective dynamics), 1.5 M 55.6 -> 44.8 us, 6.3 M 229 -> 210 us; launches and their start-up
+// bound the first, the matrix's bytes the last.
+// ---------------------------------------------------------------------------------------------
+// Vector passes: at most kVecBlocks blocks, each one contiguous range of 3N / blocks entries
+// (multiples of 64), so that few blocks have the SpMV's partials to sum and every block the same
+// work (both passes at 6.3 M tets with 512, 1024, 2048 blocks: 52.4, 53.4, 59.7 us);
+// XCD-contiguous as the SpMV's rows.
+constexpr int kVecBlocks = 512;
+constexpr int kVec = 4;  // entries a thread has in flight
+inline int vec_blocks(int n) { return (int)std::min<long>((3 * (long)n + kVec * kBlock - 1) / (kVec * kBlock), kVecBlocks); }
+__device__ __forceinline__ void vec_range(const IeDev &d, int &i0, int &i1) {
+  const int b = xcd_block(blockIdx.x, gridDim.x);
+  i0 = 64 * (b * d.vec_per + min(b, d.vec_rem));
+  i1 = min(i0 + 64 * (d.vec_per + (b < d.vec_rem ? 1 : 0)), 3 * d.n);
+}
+// The thread's kVec entries of v from i on, kBlock apart (past the end: the range's last).
+__device__ __forceinline__ void vec_load(const double *__restrict__ v, int i, int i1, double (&t)[kVec]) {
+#pragma unroll
+  for (int u = 0; u < kVec; ++u) t[u] = v[i + u * kBlock < i1 ? i + u * kBlock : i1 - 1];
+}
+
+// z = D^-1 (b - A x0); partials r.z, b.D^-1.b.  The stopping test uses the Jacobi-scaled norms
+// |D^-1/2 r| = sqrt(r.z) and |D^-1/2 b|: fixed nodes carry a 1e8 mass and spring, and in the plain
+// 2-norm their rows would swamp the free nodes' residual.
 template <typename R, int BLK> __global__ void __launch_bounds__(kBlock) k_ie_start(IeDev d) {
   __shared__ double lds[4];
   const int blk = xcd_block(blockIdx.x, gridDim.x);
   const int n = blk * kBlock + threadIdx.x;
-  double rz = 0.0, rr = 0.0, bb = 0.0;
+  double rz = 0.0, bb = 0.0;
   if (n < d.n) {
     double y[3] = {0.0, 0.0, 0.0};
     const double *__restrict__ xv = d.x;
-    row_apply<R, BLK>(d, n, [&](int col, double &x0, double &x1, double &x2) {
+    row_apply<R, BLK>(d, n, 0, 1, [&](int col, double &x0, double &x1, double &x2) {
       x0 = xv[3 * (size_t)col];
       x1 = xv[3 * (size_t)col + 1];
       x2 = xv[3 * (size_t)col + 2];
@@ -435,145 +462,155 @@ template <typename R, int BLK> __global__ void __launch_bounds__(kBlock) k_ie_st
       const double b = d.b[i];
       const double r = b - y[k];
       const double z = d.dinv[i] * r;
-      d.r[i] = r;
       d.z[i] = z;
-      d.p[i] = z;
       rz += r * z;
-      rr += r * r;
       bb += b * b * d.dinv[i];
     }
   }
   rz = block_sum256(rz, lds);
-  rr = block_sum256(rr, lds);
   bb = block_sum256(bb, lds);
   if (threadIdx.x == 0) {
-    d.part[4 * (size_t)blk + 0] = rz;
-    d.part[4 * (size_t)blk + 1] = rr;
-    d.part[4 * (size_t)blk + 2] = bb;
+    d.part_rz[blk] = rz;
+    d.part_pap[blk] = bb;
   }
 }
 
 __global__ void __launch_bounds__(1024) k_ie_start_ctrl(IeDev d, int nb) {
-  __shared__ double lds[48];
-  double sums[3];
-  partial_sums<3>(d.part, nb, {0, 1, 2}, lds, sums);
-  const double rz = sums[0], rr = sums[1], bb = sums[2];
+  __shared__ double lds[2][16];
+  PartialSum<1024> a, b;
+  a.load(d.part_rz, nb);
+  b.load(d.part_pap, nb);
+  const double rz = a.sum(d.part_rz, nb, lds[0]), bb = b.sum(d.part_pap, nb, lds[1]);
   if (threadIdx.x == 0) {
     IeCtrl c = {};
     c.rz = rz;
-    c.rr = rr;
-    c.rr0 = rr;
     c.rz0 = rz;
     c.bb = bb;
     c.converged = (rz <= d.tol2 * bb) ? 1 : 0;
     c.done = c.converged || d.maxit <= 0;
-    *d.ctrl = c;
+    d.ctrl[0] = c;
   }
 }
 
-// Ap = A p, partial p . Ap.
+// x += alpha p (the step of the iteration before), p = z + beta p.
+__global__ void __launch_bounds__(kBlock) k_ie_dir(IeDev d) {
+  __shared__ double lds[4];
+  int i0, i1;
+  vec_range(d, i0, i1);
+  int i = i0 + threadIdx.x;
+  double *__restrict__ p = d.p, *__restrict__ x = d.x;
+  PartialSum<kBlock> part;
+  part.load(d.part_rz, gridDim.x);
+  const IeCtrl in = d.ctrl[0];
+  double zv[kVec], pv[kVec], xv[kVec];
+  vec_load(d.z, i, i1, zv);
+  vec_load(p, i, i1, pv);
+  vec_load(x, i, i1, xv);
+  __builtin_amdgcn_sched_barrier(0);  // all of them requested before the first is used
+  const bool first = in.k == 0;
+  const double sum = part.sum(d.part_rz, gridDim.x, lds);
+  const double rz = first || in.done ? in.rz : sum, beta = first || in.done ? in.beta : sum / in.rz;
+  const int converged = first || in.done ? in.converged : rz <= d.tol2 * in.bb;
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    d.ctrl[1] = {rz, in.pAp, in.alpha, beta, in.bb, in.rz0, in.k, in.done || converged || in.k >= d.maxit, converged,
+                 in.indefinite};
+  if (in.done) return;
+  const double alpha = in.alpha;
+  while (true) {
+#pragma unroll
+    for (int u = 0; u < kVec; ++u)
+      if (i + u * kBlock < i1) {
+        if (!first) x[i + u * kBlock] = xv[u] + alpha * pv[u];
+        p[i + u * kBlock] = first ? zv[u] : zv[u] + beta * pv[u];
+      }
+    i += kVec * kBlock;
+    if (i - (int)threadIdx.x >= i1) break;
+    vec_load(d.z, i, i1, zv);
+    vec_load(p, i, i1, pv);
+    vec_load(x, i, i1, xv);
+  }
+}
+
+// Ap = A p, partial p . Ap.  One 64-row slice per block, its 4 waves sharing the slots (wave w takes
+// w, w + 4, ...; the shares are added in wave order): 4 times the loads in flight of one wave per
+// slice.  At 6.3 M tets 147 us instead of 161 (3x3) and 49 instead of 64 (scalar), 5.1 TB/s with
+// the padding; at 20 K tets 4.2 instead of 9 us.  Unrolled 4 instead of 2 slots: no faster.
 template <typename R, int BLK> __global__ void __launch_bounds__(kBlock) k_ie_spmv(IeDev d) {
   __shared__ double lds[4];
-  const IeCtrl *c = d.ctrl;
-  if (c->done) return;
-  const int blk = xcd_block(blockIdx.x, gridDim.x);
-  const int n = blk * kBlock + threadIdx.x;
-  double pap = 0.0;
-  if (n < d.n) {
-    double y[3] = {0.0, 0.0, 0.0};
-    const double *__restrict__ p = d.p;
-    row_apply<R, BLK>(d, n, [&](int col, double &x0, double &x1, double &x2) {
+  __shared__ double share[4][3][64];
+  if (d.ctrl[1].done) return;
+  const int sl = xcd_block(blockIdx.x, gridDim.x);
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const double *__restrict__ p = d.p;
+  const int n = sl * 64 + lane;
+  double y[3] = {0.0, 0.0, 0.0};
+  if (n < d.n)
+    row_apply<R, BLK>(d, n, w, 4, [&](int col, double &x0, double &x1, double &x2) {
       x0 = p[3 * (size_t)col];
       x1 = p[3 * (size_t)col + 1];
       x2 = p[3 * (size_t)col + 2];
     }, y);
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const size_t i = 3 * (size_t)n + q;
-      d.Ap[i] = y[q];
-      pap += p[i] * y[q];
+  for (int q = 0; q < 3; ++q) share[w][q][lane] = y[q];
+  __syncthreads();
+  double pap = 0.0;
+  if (w < 3) {  // 192 row components, one per thread of the first three waves
+    const int e = 64 * w + lane, row = e / 3, q = e % 3;
+    const double a = ((share[0][q][row] + share[1][q][row]) + share[2][q][row]) + share[3][q][row];
+    const int i = 192 * sl + e;
+    if (i < 3 * d.n) {
+      d.Ap[i] = a;
+      pap = p[i] * a;
     }
   }
   pap = block_sum256(pap, lds);
-  if (threadIdx.x == 0) d.part[4 * (size_t)blk + 3] = pap;
+  if (threadIdx.x == 0) d.part_pap[sl] = pap;
 }
 
-__global__ void __launch_bounds__(1024) k_ie_alpha(IeDev d, int nb) {
-  __shared__ double lds[16];
-  if (d.ctrl->done) return;
-  double sums[1];
-  partial_sums<1>(d.part, nb, {3}, lds, sums);
-  const double pap = sums[0];
-  if (threadIdx.x == 0) {
-    IeCtrl *c = d.ctrl;
-    if (!(pap > 0.0)) {  // not positive definite (or a non-finite value): stop without a step
-      c->indefinite = 1;
-      c->done = 1;
-      c->alpha = 0.0;
-    } else {
-      c->pAp = pap;
-      c->alpha = c->rz / pap;
-    }
-  }
-}
-
-// x += alpha p_k, r -= alpha Ap, z = D^-1 r; partials r.z, r.r.  A block covers kUpd = 1024
-// consecutive vector entries, 4 per thread 256 apart, so that every load and store of a wavefront
-// is one contiguous 512-byte access and there are 4x fewer partial sums to reduce.
-constexpr int kUpd = 4 * kBlock;
-__global__ void __launch_bounds__(kBlock) k_ie_update(IeDev d) {
+// alpha = r.z / p.Ap, z -= alpha D^-1 Ap; partial r.z.
+__global__ void __launch_bounds__(kBlock) k_ie_res(IeDev d, int nb) {
   __shared__ double lds[4];
-  const IeCtrl *c = d.ctrl;
-  if (c->done) return;
-  const double alpha = c->alpha;
-  const double *__restrict__ pk = d.p;
-  const size_t n3 = 3 * (size_t)d.n;
-  double rz = 0.0, rr = 0.0;
+  int i0, i1;
+  vec_range(d, i0, i1);
+  int i = i0 + threadIdx.x;
+  double *__restrict__ z = d.z;
+  PartialSum<kBlock> part;
+  part.load(d.part_pap, nb);
+  const IeCtrl in = d.ctrl[1];
+  double zv[kVec], av[kVec], dv[kVec];
+  vec_load(z, i, i1, zv);
+  vec_load(d.Ap, i, i1, av);
+  vec_load(d.dinv, i, i1, dv);
+  __builtin_amdgcn_sched_barrier(0);  // all of them requested before the first is used
+  const double pap = part.sum(d.part_pap, nb, lds);
+  // not positive definite (or a non-finite value): stop without a step
+  const bool indefinite = !in.done && !(pap > 0.0), go = !in.done && !indefinite;
+  const double alpha = go ? in.rz / pap : indefinite ? 0.0 : in.alpha;
+  // (the control block is written field by field: a copy modified under conditions would become a
+  // private array, which the compiler moves to LDS at an index it computes from the dispatch packet
+  // in host memory, and those reads cost a launch of 383 blocks 12 us)
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    d.ctrl[0] = {in.rz, go ? pap : in.pAp, alpha, in.beta, in.bb, in.rz0, in.k + (go ? 1 : 0), in.done || indefinite,
+                 in.converged, in.indefinite || indefinite};
+  if (!go) return;
+  double rz = 0.0;
+  while (true) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const size_t i = (size_t)blockIdx.x * kUpd + j * kBlock + threadIdx.x;
-    if (i < n3) {
-      d.x[i] += alpha * pk[i];
-      const double r = d.r[i] - alpha * d.Ap[i];
-      const double z = d.dinv[i] * r;
-      d.r[i] = r;
-      d.z[i] = z;
-      rz += r * z;
-      rr += r * r;
-    }
+    for (int u = 0; u < kVec; ++u)
+      if (i + u * kBlock < i1) {
+        const double zi = zv[u] - dv[u] * (alpha * av[u]);
+        z[i + u * kBlock] = zi;
+        rz += zi * zi / dv[u];
+      }
+    i += kVec * kBlock;
+    if (i - (int)threadIdx.x >= i1) break;
+    vec_load(z, i, i1, zv);
+    vec_load(d.Ap, i, i1, av);
+    vec_load(d.dinv, i, i1, dv);
   }
+  __syncthreads();  // part.sum's slots are read
   rz = block_sum256(rz, lds);
-  rr = block_sum256(rr, lds);
-  if (threadIdx.x == 0) {
-    d.part[4 * (size_t)blockIdx.x + 0] = rz;
-    d.part[4 * (size_t)blockIdx.x + 1] = rr;
-  }
-}
-
-__global__ void __launch_bounds__(1024) k_ie_beta(IeDev d, int nb) {
-  __shared__ double lds[32];
-  if (d.ctrl->done) return;
-  double sums[2];
-  partial_sums<2>(d.part, nb, {0, 1}, lds, sums);
-  const double rz = sums[0], rr = sums[1];
-  if (threadIdx.x == 0) {
-    IeCtrl *c = d.ctrl;
-    c->k += 1;
-    c->rr = rr;
-    c->beta = rz / c->rz;
-    c->rz = rz;
-    c->converged = (rz <= d.tol2 * c->bb) ? 1 : 0;
-    c->done = c->converged || c->k >= d.maxit;
-  }
-}
-
-// p = z + beta p for the next iteration (after k_ie_beta), one thread per vector entry.
-__global__ void __launch_bounds__(kBlock) k_ie_pupdate(IeDev d) {
-  const IeCtrl *c = d.ctrl;
-  if (c->done) return;
-  const double beta = c->beta;
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < 3 * (size_t)d.n) d.p[i] = d.z[i] + beta * d.p[i];
+  if (threadIdx.x == 0) d.part_rz[xcd_block(blockIdx.x, gridDim.x)] = rz;
 }
 
 // v = solution, x += h v for every node (cublasSaxpy in doBackEuler, CUDAInterface.cu:873).
@@ -581,7 +618,7 @@ template <typename R>
 __global__ void k_ie_finish(DevParams p, float h, IeDev d, R *__restrict__ xpos, R *__restrict__ vel) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= d.n) return;
-  const bool zero = d.ctrl->bb == 0.0;  // b = 0: the solution is 0 whatever the start
+  const bool zero = d.ctrl[0].bb == 0.0;  // b = 0: the solution is 0 whatever the start
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const size_t i = (size_t)k * p.nn + n;
@@ -801,25 +838,27 @@ template <typename R> void IeLaunch<R>::start(const IeDev &d, hipStream_t st) {
   hipLaunchKernelGGL(k_ie_start_ctrl, dim3(1), dim3(1024), 0, st, d, nb_of(d.n));
 }
 
+void ie_vec_split(IeDev &d) {
+  const int groups = (3 * d.n + 63) / 64, nblk = vec_blocks(d.n);
+  d.vec_per = groups / nblk;
+  d.vec_rem = groups % nblk;
+}
+
 // e0 set: the launch records the dispatch's start and end in e0, e1 (as a kernel trace times it)
-template <typename F>
-static void ie_launch(F kernel, dim3 grid, dim3 block, hipStream_t st, hipEvent_t e0, hipEvent_t e1, const IeDev &d) {
-  if (e0) hipExtLaunchKernelGGL(kernel, grid, block, 0u, st, e0, e1, 0u, d);
-  else hipLaunchKernelGGL(kernel, grid, block, 0, st, d);
+template <typename F, typename... Args>
+static void ie_launch(F kernel, dim3 grid, dim3 block, hipStream_t st, hipEvent_t e0, hipEvent_t e1, Args... args) {
+  if (e0) hipExtLaunchKernelGGL(kernel, grid, block, 0u, st, e0, e1, 0u, args...);
+  else hipLaunchKernelGGL(kernel, grid, block, 0, st, args...);
+}
+template <typename R> void IeLaunch<R>::dir(const IeDev &d, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  ie_launch(k_ie_dir, dim3(vec_blocks(d.n)), dim3(kBlock), st, e0, e1, d);
 }
 template <typename R> void IeLaunch<R>::spmv(const IeDev &d, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  if (d.scalar) ie_launch(k_ie_spmv<R, 1>, dim3(nb_of(d.n)), dim3(kBlock), st, e0, e1, d);
-  else ie_launch(k_ie_spmv<R, 3>, dim3(nb_of(d.n)), dim3(kBlock), st, e0, e1, d);
+  if (d.scalar) ie_launch(k_ie_spmv<R, 1>, dim3(d.nslice), dim3(kBlock), st, e0, e1, d);
+  else ie_launch(k_ie_spmv<R, 3>, dim3(d.nslice), dim3(kBlock), st, e0, e1, d);
 }
-template <typename R> void IeLaunch<R>::alpha(const IeDev &d, hipStream_t st) {
-  hipLaunchKernelGGL(k_ie_alpha, dim3(1), dim3(1024), 0, st, d, nb_of(d.n));
-}
-template <typename R> void IeLaunch<R>::update(const IeDev &d, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  ie_launch(k_ie_update, dim3((3 * d.n + kUpd - 1) / kUpd), dim3(kBlock), st, e0, e1, d);
-}
-template <typename R> void IeLaunch<R>::beta(const IeDev &d, hipStream_t st) {
-  hipLaunchKernelGGL(k_ie_beta, dim3(1), dim3(1024), 0, st, d, (3 * d.n + kUpd - 1) / kUpd);
-  hipLaunchKernelGGL(k_ie_pupdate, dim3(nb_of(3 * d.n)), dim3(kBlock), 0, st, d);
+template <typename R> void IeLaunch<R>::res(const IeDev &d, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  ie_launch(k_ie_res, dim3(vec_blocks(d.n)), dim3(kBlock), st, e0, e1, d, d.nslice);
 }
 
 template <typename R>

@@ -204,3 +204,28 @@ def test_full_size_stiffness_matrix_matches_oracle():
     err = np.abs(val - kval).max() / np.abs(kval).max()
     say("nnz", len(col), "max |K_gpu - K_oracle| / max |K|", err, "gpu %.1f s, oracle %.1f s" % (t1 - t0, t2 - t1))
     assert err <= 1e-6
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (3, 3, 3), (2, 4, 12), (1, 8, 18), (54, 54, 57)])
+def test_cg_at_the_edges_of_its_blocks(dims):
+    """8 nodes (part of one 64-row slice), 64 (one slice), 195 (a last slice of 3 rows), 342 (1026
+    vector entries: a second vector block of 2), 175,450 (more entries than 512 blocks take at
+    once): the velocities of a step solve the oracle's system.  Tolerance: the CG's own 1e-4 plus
+    as much again for the oracle's matrix, whose entries differ by up to 1e-6 relative (the
+    reference's perturbed singular values) in a product whose terms cancel to about a hundredth."""
+    rest, tets, mask, x0, v0 = case(*dims, twist=2.0)
+    say("CG block edges", dims, len(rest))
+    s = P.Solver(rest, tets, mask, P.default_params(precision=P.FP64))
+    s.set_positions(x0)
+    s.set_velocities(v0, v0)
+    st = s.implicit_step(params=P.implicit_params(cg_tolerance=1e-4))
+    v = ((s.positions(f64=True) - x0.astype(np.float64)) / H).reshape(-1)
+    mu, lam = O.lame(1e5, 0.45)
+    rowptr, col, _, aval, b = O.implicit_system(rest, tets, mask, O.precompute(rest, tets, mask), mu, lam,
+                                                x0.astype(np.float64), v0.astype(np.float64), H)
+    A = sp.csr_matrix((aval, col, rowptr), shape=(len(v), len(v)))
+    d = 1.0 / np.sqrt(A.diagonal())
+    res = np.linalg.norm(d * (b - A @ v)) / np.linalg.norm(d * b)
+    say("its", st.cg_iterations, "residual", res)
+    assert st.converged and res <= 2e-4
+    s.close()
