@@ -165,11 +165,13 @@ template <typename R> struct LearnLaunch {
 };
 void mlp_arrange(const float *params, unsigned short *wA, hipStream_t st);
 void mlp_forward(const MlpDev &net, const float *feat, int n, float *out, hipStream_t st);
-// training: per 32-sample workgroup partial gradients (MLP_NPARAM each) and loss sums
+// training: gradient partials (MLP_NPARAM each) and loss sums of mlp_train_wgs(n) workgroups, then
+// their sums and, with update, the Adam step of params (m1, m2 moments) and wA
+int mlp_train_wgs(int n);
 void mlp_train_partials(const MlpDev &net, const float *ds_x, const float *ds_y, const int *idx, int n, int batch,
                         float *grad_part, float *loss_part, hipStream_t st);
-void mlp_reduce(const float *grad_part, const float *loss_part, int nwg, float *grad, double *loss_acc, hipStream_t st);
-void mlp_adam(float *params, float *m1, float *m2, const float *grad, float lr, float b1t, float b2t, hipStream_t st);
+void mlp_step(const float *grad_part, const float *loss_part, int nwg, float *grad, double *loss_acc, bool update,
+              float *params, float *m1, float *m2, unsigned short *wA, float lr, float b1t, float b2t, hipStream_t st);
 
 void aos_to_planes_f(const float *aos, float *planes, const int *perm, int n, hipStream_t st);
 void planes_to_aos_f(const float *planes, float *aos, const int *perm, int n, hipStream_t st);

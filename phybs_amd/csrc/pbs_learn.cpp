@@ -341,7 +341,7 @@ extern "C" int pbs_learn_fit_scales(pbs_solver *s) {
 
 static int train_batch(pbs_solver *s, LearnState *L, const float *ds_x, const float *ds_y, const int *idx, int n,
                        float lr, bool update) {
-  const int nwg = (n + 31) / 32;
+  const int nwg = mlp_train_wgs(n);
   if (nwg > L->part_cap) {
     lfree(L, L->grad_part);
     lfree(L, L->loss_part);
@@ -354,13 +354,14 @@ static int train_batch(pbs_solver *s, LearnState *L, const float *ds_x, const fl
   }
   const MlpDev net = mlp_dev(*L);
   mlp_train_partials(net, ds_x, ds_y, idx, n, n, L->grad_part, L->loss_part, s->st);
-  mlp_reduce(L->grad_part, L->loss_part, nwg, L->grad, L->loss_acc, s->st);
+  float b1t = 0.0f, b2t = 0.0f;
   if (update) {
     L->adam_t++;
-    const float b1t = (float)std::pow(0.9, (double)L->adam_t), b2t = (float)std::pow(0.999, (double)L->adam_t);
-    mlp_adam(L->params, L->m1, L->m2, L->grad, lr, b1t, b2t, s->st);
-    mlp_arrange(L->params, L->wA, s->st);
+    b1t = (float)std::pow(0.9, (double)L->adam_t);
+    b2t = (float)std::pow(0.999, (double)L->adam_t);
   }
+  mlp_step(L->grad_part, L->loss_part, nwg, L->grad, L->loss_acc, update, L->params, L->m1, L->m2, L->wA, lr, b1t, b2t,
+           s->st);
   HIPCHK(hipGetLastError());
   return PBS_OK;
 }

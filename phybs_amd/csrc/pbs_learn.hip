@@ -6,9 +6,8 @@
 // cores: BF16 weights and activations, FP32 accumulation, v_mfma_f32_16x16x16_bf16 with the
 // layers written transposed (H_{l+1}^T = act(W_l^T H_l^T + b)), so that the accumulator tile of one
 // layer is already the B-operand tile of the next and nothing is shuffled through LDS.  Training
-// (forward and backward in FP32 on the vector units, with the same BF16 roundings) produces
-// per-workgroup gradient partials that are reduced in a fixed order; Adam updates FP32 master
-// weights.
+// (on the matrix cores too: forward in BF16 as inference, backward in FP32) produces per-workgroup
+// gradient partials that are reduced in a fixed order; Adam updates FP32 master weights.
 //
 // The warm start is a guess, never a replacement: both the plain guess and the learned one are
 // evaluated with one gradient pass each, and the descent starts from the learned guess only if its
@@ -30,10 +29,6 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
 __device__ __forceinline__ float bf2f(unsigned short b) { return __uint_as_float((unsigned)b << 16); }
 __device__ __forceinline__ float bfround(float f) { return bf2f(f2bf(f)); }
 __device__ __forceinline__ float silu(float z) { return z / (1.0f + expf(-z)); }
-__device__ __forceinline__ float dsilu(float z) {
-  const float s = 1.0f / (1.0f + expf(-z));
-  return s * (1.0f + z * (1.0f - s));
-}
 
 // Layer table: inputs, outputs, 16-row output tiles, 16-wide input blocks, offsets of the
 // A-operand arrangement, of the packed weights and of the packed biases.
@@ -356,21 +351,55 @@ __global__ void k_collect(DevParams p, const R *__restrict__ xnew, const float *
 }
 
 // ---------------------------------------------------------------------------------------------
-// Training: one 256-thread workgroup per 32 samples, FP32 on the vector units with the BF16
-// roundings of the inference path (inputs, weights and hidden activations), straight-through
-// gradients for the roundings.  Loss = mean over (sample, component) of (out - t / scale)^2 with
-// the mean taken over the whole batch.  Each workgroup writes its gradient partial (packed like
-// the parameters) and its sum of squared errors.
+// Training.  Loss = mean over (sample, component) of (out - t / scale)^2 with the mean taken over
+// the whole batch; the inference path's BF16 roundings (inputs, weights, hidden activations) with
+// straight-through gradients.  Every product is on the matrix cores: the forward ones in BF16 with
+// FP32 accumulation (their factors are BF16 values), the backward ones, whose deltas are FP32, in
+// FP32 (v_mfma_f32_16x16x4_f32), so nothing is rounded further than by the loss itself.
+//
+// A workgroup takes tiles of 64 samples, 16 per wave.  Forward and delta propagation stay in the
+// wave's registers in the transposed form of mlp_tile: an accumulator tile (rows 4 q + i, column r)
+// is the next product's B operand, an FP32 product taking rows 4 q + j, j = 0..3, in its 4 steps.
+// The weight gradients contract over samples, which are the lanes: activations and deltas go
+// through LDS (rows of 64 samples, padded to 68 so that 16 rows start in different banks), and
+// each wave accumulates 11 of the 44 gradient tiles in registers over all tiles of the workgroup.
+// At most 256 workgroups (one per CU: the arrays take 126 KB of LDS) write one gradient partial each.
+//
+// A batch of 8192 samples: 166 -> 20 us (on the vector units, both factors of each multiply-add
+// came from LDS), and its reduction, Adam step and arrangement 77 -> 4.7 us in one launch
+// (k_mlp_step).  128 workgroups of 4 waves: what is left is the chain of one tile (weights 38 KB
+// and samples in, 192 exponentials per sample, 308 FP32 products per wave).  With the weights
+// converted one load at a time and the biases read where they are used it took 31 us.
 // ---------------------------------------------------------------------------------------------
-constexpr int TS = 32;  // samples per training workgroup
+constexpr int TS = 64;         // samples per tile
+constexpr int SP = TS + 4;     // padded row of samples
+constexpr int kTrainWGs = 256;
 struct TrainLds {
-  float W[9536];  // BF16-rounded weights, layers packed without biases
-  float h0[TS][18];
-  float z[3][TS][64], h[3][TS][64];
-  float dA[TS][64], dB[TS][64];
-  float d4[TS][3], t[TS][3];
+  unsigned short wA[MLP_WA];                // forward A operands
+  unsigned short wB[2][64][SP];             // layers 2 and 3, BF16 [in][out], padded likewise
+  float w4[64][4];                          // layer 4 [in][out], column 3 zero
+  float bias[4][64];
+  unsigned short h0[32][SP], h[3][64][SP];  // BF16 inputs (18 rows used) and activations [unit][sample]
+  float dz[3][64][SP], dz4[16][SP];         // deltas [unit][sample] (3 rows of dz4 used)
   double red[4];
 };
+
+__device__ __forceinline__ f32x4 bf4(bf16x4 v) {
+  f32x4 f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f[i] = bf2f((unsigned short)v[i]);
+  return f;
+}
+// SiLU and its derivative from one exponential: s = 1 / (1 + e^-z), refined to the last bit or two
+// (e^-z capped where s is no longer a normal number).
+__device__ __forceinline__ void silu_both(float z, float &v, float &dv) {
+  const float d = 1.0f + fminf(expf(-z), 1e37f);
+  float s = __builtin_amdgcn_rcpf(d);
+  s = fmaf(fmaf(-d, s, 1.0f), s, s);
+  v = z * s;
+  v = fmaf(fmaf(-v, d, z), s, v);  // the quotient z / d to the last bit: it is rounded to BF16 next
+  dv = s * fmaf(z, 1.0f - s, 1.0f);
+}
 
 __global__ void __launch_bounds__(256) k_mlp_train(MlpDev net, const float *__restrict__ ds_x,
                                                    const float *__restrict__ ds_y, const int *__restrict__ idx, int n,
@@ -378,138 +407,259 @@ __global__ void __launch_bounds__(256) k_mlp_train(MlpDev net, const float *__re
                                                    float *__restrict__ loss_part) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   TrainLds &S = *(TrainLds *)smem_raw;
-  const int tid = threadIdx.x, w = blockIdx.x;
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, q = lane >> 4, r = lane & 15;
   const float *P = net.params;
-  const int wofs[4] = {0, 1152, 5248, 9344};  // layer weight offsets in S.W
-  for (int e = tid; e < 9536; e += 256) {
-    int l = 3;
-    while (l > 0 && e < wofs[l]) --l;
-    S.W[e] = bfround(P[kLayers[l].pw + (e - wofs[l])]);
+  // the lane's sample of a tile: 8 scaled features (inputs 4 q + i and 16 + 4 q + i) and, q = 0, the
+  // targets; zeros past the end
+  auto load_sample = [&](int tile, f32x4 (&x)[2], float (&t)[3]) {
+    const int j = tile * TS + 16 * w + r;
+    const bool valid = j < n;
+    const size_t row = valid ? idx[j] : 0;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int k = 16 * kb + 4 * q + i;
+        x[kb][i] = (valid && k < 18) ? ds_x[row * 18 + k] * net.inv_s[k / 3] : 0.0f;
+      }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) t[i] = valid && q == 0 ? ds_y[row * 3 + i] * net.inv_s[6] : 0.0f;
+  };
+  // weights: every load is issued before the first is waited for
+  f32x4 x[2];
+  float t[3];
+  load_sample(blockIdx.x, x, t);
+  {
+    uint4 u[6];
+    f32x4 f[8];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) u[i] = ((const uint4 *)net.wA)[min(tid + 256 * i, MLP_WA / 8 - 1)];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {  // rows of 64 outputs, 4 per load
+      const int e = 4 * (tid + 256 * i), l = e >> 12;
+      const float *v = P + kLayers[1 + l].pw + (e & 4095);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) f[i][c] = v[c];
+    }
+    const float w4 = (tid & 3) < 3 ? bfround(P[9536 + (tid >> 2) * 3 + (tid & 3)]) : 0.0f;
+    const float bias = w < 3 ? P[kLayers[w].pb + lane] : lane < 3 ? P[9728 + lane] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+      if (tid + 256 * i < MLP_WA / 8) ((uint4 *)S.wA)[tid + 256 * i] = u[i];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int e = 4 * (tid + 256 * i);
+      bf16x4 v;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[c] = (short)f2bf(f[i][c]);
+      *(bf16x4 *)&S.wB[e >> 12][(e >> 6) & 63][e & 63] = v;
+    }
+    S.w4[tid >> 2][tid & 3] = w4;
+    S.bias[w][lane] = bias;
   }
-  for (int e = tid; e < TS * 18; e += 256) {
-    const int s = e / 18, k = e % 18, j = w * TS + s;
-    const float f = j < n ? ds_x[(size_t)idx[j] * 18 + k] * net.inv_s[k / 3] : 0.0f;
-    S.h0[s][k] = bfround(f);
-  }
-  for (int e = tid; e < TS * 3; e += 256) {
-    const int s = e / 3, i = e % 3, j = w * TS + s;
-    S.t[s][i] = j < n ? ds_y[(size_t)idx[j] * 3 + i] * net.inv_s[6] : 0.0f;
-  }
+  // gradient tiles of this wave: rows (inputs) of tile mt, columns (outputs) of tile ot; layers 2
+  // and 3: mt = w, ot = 0..3; layer 1: mt = w & 1, ot = 2 (w >> 1) + 0..1; layer 4: mt = w
+  f32x4 g1[2] = {}, g2[4] = {}, g3[4] = {}, g4 = {};
+  float gb[3] = {0.0f, 0.0f, 0.0f}, gb4 = 0.0f;  // bias gradients: unit lane, samples 16 w .. 16 w + 15
+  double se = 0.0;
   __syncthreads();
-  // forward, hidden layers
-  const int o = tid & 63, sg = tid >> 6;
-  for (int l = 0; l < 3; ++l) {
-    const int K = l == 0 ? 18 : 64;
-    const float *Wl = S.W + wofs[l];
-    const float bias = P[kLayers[l].pb + o];
-    for (int jj = 0; jj < TS / 4; ++jj) {
-      const int s = sg + 4 * jj;
-      const float *hin = l == 0 ? S.h0[s] : S.h[l - 1][s];
-      float acc = bias;
-      for (int k = 0; k < K; ++k) acc = fmaf(Wl[k * 64 + o], hin[k], acc);
-      S.z[l][s][o] = acc;
-      S.h[l][s][o] = bfround(silu(acc));
+  for (int tile = blockIdx.x; tile * TS < n; tile += gridDim.x) {
+    const int j = tile * TS + 16 * w + r;  // the lane's sample
+    const bool valid = j < n;
+    bf16x4 h[4], hn[4];
+    f32x4 ds[3][4];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        h[kb][i] = (short)f2bf(x[kb][i]);
+        S.h0[16 * kb + 4 * q + i][16 * w + r] = (unsigned short)h[kb][i];
+      }
+    // forward, hidden layers
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const int nkb = l == 0 ? 2 : 4, wa = l == 0 ? 0 : l == 1 ? 2048 : 6144;
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        f32x4 c = *(const f32x4 *)&S.bias[l][16 * mt + 4 * q];
+#pragma unroll
+        for (int kb = 0; kb < nkb; ++kb) {
+          const bf16x4 a = *(const bf16x4 *)(S.wA + wa + (mt * nkb + kb) * 256 + lane * 4);
+          c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, h[kb], c, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float v, dv;
+          silu_both(c[i], v, dv);
+          ds[l][mt][i] = dv;
+          hn[mt][i] = (short)f2bf(v);
+          S.h[l][16 * mt + 4 * q + i][16 * w + r] = (unsigned short)hn[mt][i];
+        }
+      }
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) h[mt] = hn[mt];
+    }
+    // output layer, loss and output delta: rows 0..2 of the tile, i.e. lanes with q = 0
+    f32x4 c = *(const f32x4 *)&S.bias[3][4 * q];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+      const bf16x4 a = *(const bf16x4 *)(S.wA + 10240 + kb * 256 + lane * 4);
+      c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, h[kb], c, 0, 0, 0);
+    }
+    float d4[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const float diff = c[i] - t[i];
+      d4[i] = valid && q == 0 ? (2.0f / (3.0f * (float)batch)) * diff : 0.0f;
+      if (valid && q == 0) {
+        se += (double)diff * (double)diff;
+      }
+      if (q == 0) S.dz4[i][16 * w + r] = d4[i];
+    }
+    const float e1 = __shfl(d4[1], r, 64), e2 = __shfl(d4[2], r, 64);
+    const float b4 = q == 0 ? d4[0] : q == 1 ? e1 : q == 2 ? e2 : 0.0f;
+    f32x4 d[4];
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+      d[mt] = __builtin_amdgcn_mfma_f32_16x16x4f32(S.w4[16 * mt + r][q], b4, z, 0, 0, 0) * ds[2][mt];
+    }
+#pragma unroll
+    for (int l = 2; l >= 0; --l) {
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S.dz[l][16 * mt + 4 * q + i][16 * w + r] = d[mt][i];
+      if (l == 0) break;
+      f32x4 dn[4];
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) {
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob) {
+          const f32x4 a = bf4(*(const bf16x4 *)&S.wB[l - 1][16 * mt + r][16 * ob + 4 * q]);
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[jj], d[ob][jj], acc, 0, 0, 0);
+        }
+        dn[mt] = acc * ds[l - 1][mt];
+      }
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) d[mt] = dn[mt];
+    }
+    __syncthreads();
+    if ((tile + (int)gridDim.x) * TS < n) load_sample(tile + gridDim.x, x, t);
+    // weight gradients: sum over the 64 samples of h_in[k] dz[o]
+#pragma unroll
+    for (int sb = 0; sb < 4; ++sb) {
+      const int s0 = 16 * sb + 4 * q;
+      const f32x4 a1 = bf4(*(const bf16x4 *)&S.h0[16 * (w & 1) + r][s0]), a2 = bf4(*(const bf16x4 *)&S.h[0][16 * w + r][s0]),
+                  a3 = bf4(*(const bf16x4 *)&S.h[1][16 * w + r][s0]), a4 = bf4(*(const bf16x4 *)&S.h[2][16 * w + r][s0]);
+#pragma unroll
+      for (int ot = 0; ot < 2; ++ot) {
+        const f32x4 bz = *(const f32x4 *)&S.dz[0][16 * (2 * (w >> 1) + ot) + r][s0];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) g1[ot] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[jj], bz[jj], g1[ot], 0, 0, 0);
+      }
+#pragma unroll
+      for (int ot = 0; ot < 4; ++ot) {
+        const f32x4 b2 = *(const f32x4 *)&S.dz[1][16 * ot + r][s0], b3 = *(const f32x4 *)&S.dz[2][16 * ot + r][s0];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          g2[ot] = __builtin_amdgcn_mfma_f32_16x16x4f32(a2[jj], b2[jj], g2[ot], 0, 0, 0);
+          g3[ot] = __builtin_amdgcn_mfma_f32_16x16x4f32(a3[jj], b3[jj], g3[ot], 0, 0, 0);
+        }
+      }
+      const f32x4 bo = *(const f32x4 *)&S.dz4[r][s0];
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) g4 = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[jj], bo[jj], g4, 0, 0, 0);
+      // bias gradients: samples 16 w + 4 sb .. + 3 of unit `lane`
+#pragma unroll
+      for (int l = 0; l < 3; ++l) {
+        const f32x4 v = *(const f32x4 *)&S.dz[l][lane][16 * w + 4 * sb];
+        gb[l] += (v[0] + v[1]) + (v[2] + v[3]);
+      }
+      if (lane < 3) {
+        const f32x4 v = *(const f32x4 *)&S.dz4[lane][16 * w + 4 * sb];
+        gb4 += (v[0] + v[1]) + (v[2] + v[3]);
+      }
     }
     __syncthreads();
   }
-  // output layer, loss, output delta
-  double se = 0.0;
-  if (tid < TS * 3) {
-    const int s = tid / 3, i = tid % 3, j = w * TS + s;
-    float acc = P[9728 + i];
-    for (int k = 0; k < 64; ++k) acc = fmaf(S.W[9344 + k * 3 + i], S.h[2][s][k], acc);
-    const float diff = acc - S.t[s][i];
-    const bool valid = j < n;
-    S.d4[s][i] = valid ? (2.0f / (3.0f * (float)batch)) * diff : 0.0f;
-    se = valid ? (double)diff * (double)diff : 0.0;
+  // the workgroup's partial
+  float *gp = grad_part + (size_t)blockIdx.x * MLP_NPARAM;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k1 = 16 * (w & 1) + 4 * q + i, k = 16 * w + 4 * q + i;
+#pragma unroll
+    for (int ot = 0; ot < 2; ++ot)
+      if (k1 < 18) gp[k1 * 64 + 16 * (2 * (w >> 1) + ot) + r] = g1[ot][i];
+#pragma unroll
+    for (int ot = 0; ot < 4; ++ot) {
+      gp[1216 + k * 64 + 16 * ot + r] = g2[ot][i];
+      gp[5376 + k * 64 + 16 * ot + r] = g3[ot][i];
+    }
+    if (r < 3) gp[9536 + k * 3 + r] = g4[i];
   }
-  // block sum of squared errors (waves 0 and 1 hold the 96 values)
+  float(*sb)[4][64] = (float(*)[4][64])S.dz;  // bias shares of the 4 waves
+#pragma unroll
+  for (int l = 0; l < 3; ++l) sb[l][w][lane] = gb[l];
+  sb[3][w][lane] = gb4;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) se += __shfl_down(se, off, 64);
-  if ((tid & 63) == 0) S.red[tid >> 6] = se;
+  if (lane == 0) S.red[w] = se;
   __syncthreads();
-  float *gp = grad_part + (size_t)w * MLP_NPARAM;
-  if (tid == 0) loss_part[w] = (float)(S.red[0] + S.red[1] + S.red[2] + S.red[3]);
-  // layer 4 gradients and delta into layer 3
-  if (tid < 192) {
-    const int k = tid / 3, i = tid % 3;
-    float a = 0.0f;
-    for (int s = 0; s < TS; ++s) a = fmaf(S.h[2][s][k], S.d4[s][i], a);
-    gp[9536 + k * 3 + i] = a;
-  } else if (tid < 195) {
-    const int i = tid - 192;
-    float a = 0.0f;
-    for (int s = 0; s < TS; ++s) a += S.d4[s][i];
-    gp[9728 + i] = a;
-  }
-  for (int jj = 0; jj < TS / 4; ++jj) {
-    const int s = sg + 4 * jj, k = o;
-    float a = 0.0f;
-    for (int i = 0; i < 3; ++i) a = fmaf(S.W[9344 + k * 3 + i], S.d4[s][i], a);
-    S.dA[s][k] = a * dsilu(S.z[2][s][k]);
-  }
-  __syncthreads();
-  // hidden layers 3, 2, 1 (l = 2, 1, 0): dW = h_{l-1}^T dz, db = sum dz, dh_{l-1} = W dz
-  float(*dz)[64] = S.dA;
-  float(*dn)[64] = S.dB;
-  for (int l = 2; l >= 0; --l) {
-    const int K = l == 0 ? 18 : 64;
-    const int pw = kLayers[l].pw, pb = kLayers[l].pb;
-    for (int e = tid; e < K * 64; e += 256) {
-      const int k = e / 64, oo = e % 64;
-      float a = 0.0f;
-      for (int s = 0; s < TS; ++s) a = fmaf(l == 0 ? S.h0[s][k] : S.h[l - 1][s][k], dz[s][oo], a);
-      gp[pw + k * 64 + oo] = a;
-    }
-    if (tid < 64) {
-      float a = 0.0f;
-      for (int s = 0; s < TS; ++s) a += dz[s][tid];
-      gp[pb + tid] = a;
-    }
-    if (l > 0) {
-      const float *Wl = S.W + wofs[l];
-      for (int jj = 0; jj < TS / 4; ++jj) {
-        const int s = sg + 4 * jj, k = o;
-        float a = 0.0f;
-        for (int oo = 0; oo < 64; ++oo) a = fmaf(Wl[k * 64 + oo], dz[s][oo], a);
-        dn[s][k] = a * dsilu(S.z[l - 1][s][k]);
-      }
-      __syncthreads();
-      float(*tmp)[64] = dz;
-      dz = dn;
-      dn = tmp;
-    }
-  }
+  const float bsum = (sb[w][0][lane] + sb[w][1][lane]) + (sb[w][2][lane] + sb[w][3][lane]);
+  if (w < 3) gp[kLayers[w].pb + lane] = bsum;
+  else if (lane < 3) gp[9728 + lane] = bsum;
+  if (tid == 0) loss_part[blockIdx.x] = (float)((S.red[0] + S.red[1]) + (S.red[2] + S.red[3]));
 }
 
-// grad[p] = sum over workgroups (in order) of the partials; loss_acc += sum of squared errors.
-__global__ void k_mlp_reduce(const float *__restrict__ grad_part, const float *__restrict__ loss_part, int nwg,
-                             float *__restrict__ grad, double *__restrict__ loss_acc) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < MLP_NPARAM) {
-    float a = 0.0f;
-    for (int w = 0; w < nwg; ++w) a += grad_part[(size_t)w * MLP_NPARAM + p];
-    grad[p] = a;
+// grad[p] = sum over the workgroups of the partials (4 interleaved shares, each in order, then the
+// shares in order; 8 loads in flight per thread); loss_acc += sum of squared errors.  With `update`
+// also Adam (beta1 = 0.9, beta2 = 0.999, eps = 1e-8; b1t, b2t = beta^t) and the parameter's place in
+// the BF16 A-operand arrangement, which were two launches of their own.
+__global__ void __launch_bounds__(256) k_mlp_step(const float *__restrict__ grad_part, const float *__restrict__ loss_part,
+                                                  int nwg, float *__restrict__ grad, double *__restrict__ loss_acc,
+                                                  int update, float *__restrict__ params, float *__restrict__ m1,
+                                                  float *__restrict__ m2, unsigned short *__restrict__ wA, float lr,
+                                                  float b1t, float b2t) {
+  __shared__ float share[4][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, p = blockIdx.x * 64 + lane;
+  const float *v = grad_part + min(p, MLP_NPARAM - 1);
+  float a = 0.0f;
+  for (int i = w; i < nwg; i += 32) {
+    float t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = v[(size_t)(i + 4 * u < nwg ? i + 4 * u : i) * MLP_NPARAM];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a += i + 4 * u < nwg ? t[u] : 0.0f;
   }
-  if (p == 0) {
+  share[w][lane] = a;
+  __syncthreads();
+  if (blockIdx.x == 0 && w == 1) {
     double l = 0.0;
-    for (int w = 0; w < nwg; ++w) l += (double)loss_part[w];
-    *loss_acc += l;
+    for (int i = lane; i < nwg; i += 64) l += (double)loss_part[i];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
+    if (lane == 0) *loss_acc += l;
   }
-}
-
-// Adam (beta1 = 0.9, beta2 = 0.999, eps = 1e-8); b1t, b2t = beta^t.
-__global__ void k_mlp_adam(float *__restrict__ params, float *__restrict__ m1, float *__restrict__ m2,
-                           const float *__restrict__ grad, float lr, float b1t, float b2t) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= MLP_NPARAM) return;
-  const float g = grad[p];
-  const float a = 0.9f * m1[p] + 0.1f * g;
-  const float b = 0.999f * m2[p] + 0.001f * g * g;
-  m1[p] = a;
-  m2[p] = b;
-  const float mh = a / (1.0f - b1t), vh = b / (1.0f - b2t);
-  params[p] -= lr * mh / (sqrtf(vh) + 1e-8f);
+  if (w != 0 || p >= MLP_NPARAM) return;
+  const float g = (share[0][lane] + share[1][lane]) + (share[2][lane] + share[3][lane]);
+  grad[p] = g;
+  if (!update) return;
+  const float a1 = 0.9f * m1[p] + 0.1f * g;
+  const float a2 = 0.999f * m2[p] + 0.001f * g * g;
+  m1[p] = a1;
+  m2[p] = a2;
+  const float mh = a1 / (1.0f - b1t), vh = a2 / (1.0f - b2t);
+  const float np = params[p] - lr * mh / (sqrtf(vh) + 1e-8f);
+  params[p] = np;
+  int l = 3;
+  while (l > 0 && p < kLayers[l].pw) --l;
+  const Layer L = kLayers[l];
+  if (p >= L.pb) return;  // a bias
+  const int k = (p - L.pw) / L.out, o = (p - L.pw) % L.out;
+  wA[L.wa + (((o >> 4) * L.kb + (k >> 4)) * 64 + ((k >> 2) & 3) * 16 + (o & 15)) * 4 + (k & 3)] = f2bf(np);
 }
 
 // ---- launch wrappers ----
@@ -576,18 +726,17 @@ void mlp_forward(const MlpDev &net, const float *feat, int n, float *out, hipStr
   const unsigned grid = (unsigned)std::min<long>((tiles + 3) / 4, 2048);
   hipLaunchKernelGGL(k_mlp_forward, dim3(grid), dim3(256), 0, st, net, feat, n, out);
 }
+int mlp_train_wgs(int n) { return std::min((n + TS - 1) / TS, kTrainWGs); }
 void mlp_train_partials(const MlpDev &net, const float *ds_x, const float *ds_y, const int *idx, int n, int batch,
                         float *grad_part, float *loss_part, hipStream_t st) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_mlp_train, dim3(nb(n, TS)), dim3(256), sizeof(TrainLds), st, net, ds_x, ds_y, idx, n, batch,
+  hipLaunchKernelGGL(k_mlp_train, dim3(mlp_train_wgs(n)), dim3(256), sizeof(TrainLds), st, net, ds_x, ds_y, idx, n, batch,
                      grad_part, loss_part);
 }
-void mlp_reduce(const float *grad_part, const float *loss_part, int nwg, float *grad, double *loss_acc, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_reduce, dim3(nb(MLP_NPARAM, 256)), dim3(256), 0, st, grad_part, loss_part, nwg, grad,
-                     loss_acc);
-}
-void mlp_adam(float *params, float *m1, float *m2, const float *grad, float lr, float b1t, float b2t, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_adam, dim3(nb(MLP_NPARAM, 256)), dim3(256), 0, st, params, m1, m2, grad, lr, b1t, b2t);
+void mlp_step(const float *grad_part, const float *loss_part, int nwg, float *grad, double *loss_acc, bool update,
+              float *params, float *m1, float *m2, unsigned short *wA, float lr, float b1t, float b2t, hipStream_t st) {
+  hipLaunchKernelGGL(k_mlp_step, dim3(nb(MLP_NPARAM, 64)), dim3(256), 0, st, grad_part, loss_part, nwg, grad, loss_acc,
+                     update ? 1 : 0, params, m1, m2, wA, lr, b1t, b2t);
 }
 
 }  // namespace pbs

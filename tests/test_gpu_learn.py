@@ -69,6 +69,35 @@ def test_mlp_loss_and_gradient_match_spec():
     s.close()
 
 
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 16385])
+def test_training_at_the_edges_of_its_tiles(n):
+    """One sample, one wave's 16 and one more, a workgroup's 64 and one more, one more than 256
+    workgroups take in a first tile: loss and gradient against numpy, and after one Adam step the
+    forward pass (which reads the arranged BF16 weights) against numpy on the read-back parameters.
+    Tolerances as in the tests above; where a hidden activation's BF16 rounding flips, a sample's
+    share (1 / n) of loss and gradient moves by up to 1 and 2 per cent."""
+    rest, tets, mask, _ = bar()
+    say("training tiles", n)
+    s = P.Solver(rest, tets, mask, P.default_params())
+    s.learn_set_model(model(), SCALES)
+    rng = np.random.default_rng(n)
+    f = rng.normal(0, 1, (n, 18)).astype(np.float32)
+    t = rng.normal(0, 1, (n, 3)).astype(np.float32)
+    loss, g = s.learn_loss_grad(f, t)
+    lref, gref = MO.loss_grad(model(), SCALES, f, t)
+    say("loss", loss, lref, "grad rel err", np.linalg.norm(g - gref) / np.linalg.norm(gref))
+    assert loss == pytest.approx(lref, rel=1e-5 + 1e-2 / n)
+    assert np.linalg.norm(g - gref) <= (1e-3 + 2e-2 / n) * np.linalg.norm(gref)
+    s.learn_collect(n)
+    s.learn_add_samples(f, t)
+    s.learn_train(1, batch=n, lr=1e-2, seed=3)
+    p, sc = s.learn_get_model()
+    assert not np.array_equal(p, model())
+    out, ref = s.learn_forward(f), MO.forward(p, sc, f)[0]
+    assert np.abs(out - ref).max() <= 1e-2 * np.abs(ref).max()
+    s.close()
+
+
 def adjacency(nn, tets):
     nb = [set() for _ in range(nn)]
     for t in tets:
