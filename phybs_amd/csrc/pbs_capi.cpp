@@ -145,6 +145,13 @@ template <typename R> static int upload_planes(pbs_solver *s, const float *aos, 
   HIPCHK(hipGetLastError());
   return PBS_OK;
 }
+// Caller's AoS positions -> ring buffer 0, where the standalone calls evaluate.
+template <typename R> static int upload_ring(pbs_solver *s, const float *aos) {
+  HIPCHK(hipMemcpyAsync(s->stage, aos, sizeof(float) * 3 * (size_t)s->nn, hipMemcpyHostToDevice, s->st));
+  Launch<R>::aos_to_nodes(s->stage, mesh<R>(s).ring.b[0], mesh<R>(s).perm, s->nn, s->st);
+  HIPCHK(hipGetLastError());
+  return PBS_OK;
+}
 template <typename R> static int download_planes(pbs_solver *s, const R *planes, float *aos) {
   Launch<R>::planes_to_aos(planes, s->stage, mesh<R>(s).perm, s->nn, s->st);
   HIPCHK(hipGetLastError());
@@ -183,6 +190,7 @@ template <typename R> static int alloc_impl(pbs_solver *s) {
   int rc = 0;
   rc |= dalloc(s, &m.tets, T);
   rc |= dalloc(s, &m.rest, 3 * N);
+  rc |= dalloc(s, &m.rest4, N);
   rc |= dalloc(s, &m.dmi, 9 * T);
   rc |= dalloc(s, &m.vol, T);
   rc |= dalloc(s, &m.inc_off, N + 1);
@@ -209,11 +217,12 @@ template <typename R> static int alloc_impl(pbs_solver *s) {
   const TilePlan &P = s->plan;
   const size_t H = std::max<long>(P.halo_total, 1);
   TileInfo *tiles;
-  int *halo, *bnd_off, *hslot;
+  int *halo, *ids, *bnd_off, *hslot;
   uint32_t *tlp;
   unsigned short *toff;
   rc |= dalloc(s, &tiles, (size_t)P.ntiles);
   rc |= dalloc(s, &halo, H);
+  rc |= dalloc(s, &ids, (size_t)P.ntiles * s->td.lstride);
   rc |= dalloc(s, &tlp, 4 * T);
   rc |= dalloc(s, &toff, P.tile_off.size());
   rc |= dalloc(s, &bnd_off, N + 1);
@@ -227,6 +236,7 @@ template <typename R> static int alloc_impl(pbs_solver *s) {
   rc |= dalloc(s, &m.hparth, 3 * H);
   s->td.tiles = tiles;
   s->td.halo = halo;
+  s->td.ids = ids;
   s->td.tet_lp = (const uint4 *)tlp;
   s->td.tile_off = toff;
   s->td.bnd_off = bnd_off;
@@ -263,6 +273,9 @@ template <typename R> static int setup_impl(pbs_solver *s, const int *mask) {
     for (int d = 0; d < 3; ++d) planes[d * N + i] = s->rest_h[3 * (size_t)P.perm[i] + d];
   if (s->nt > 0) HIPCHK(hipMemcpyAsync(m.tets, P.tets_new.data(), sizeof(int) * 4 * (size_t)s->nt, hipMemcpyHostToDevice, s->st));
   HIPCHK(hipMemcpyAsync(m.rest, planes.data(), sizeof(float) * 3 * N, hipMemcpyHostToDevice, s->st));
+  std::vector<float4> rest4(N);
+  for (size_t i = 0; i < N; ++i) rest4[i] = make_float4(planes[i], planes[N + i], planes[2 * N + i], 0.0f);
+  HIPCHK(hipMemcpyAsync(m.rest4, rest4.data(), sizeof(float4) * N, hipMemcpyHostToDevice, s->st));
   std::vector<int> mk(N, 0);
   if (mask)
     for (size_t i = 0; i < N; ++i) mk[i] = mask[P.perm[i]] ? 1 : 0;
@@ -292,6 +305,16 @@ template <typename R> static int setup_impl(pbs_solver *s, const int *mask) {
     int rc = upload_lame(s);
     if (rc) return rc;
   }
+  std::vector<int> ids((size_t)P.ntiles * s->td.lstride);
+  for (int b = 0; b < P.ntiles; ++b) {
+    const TileInfo &ti = P.tiles[b];
+    int *v = &ids[(size_t)b * s->td.lstride];
+    for (int i = 0; i < s->td.lstride; ++i)
+      v[i] = i < ti.own_cnt                  ? ti.own_start + i
+             : i < ti.own_cnt + ti.halo_cnt ? P.halo[ti.halo_off + i - ti.own_cnt]
+                                            : ti.own_start;
+  }
+  HIPCHK(hipMemcpyAsync((void *)s->td.ids, ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice, s->st));
   if (!P.halo.empty())
     HIPCHK(hipMemcpyAsync((void *)s->td.halo, P.halo.data(), sizeof(int) * P.halo.size(), hipMemcpyHostToDevice, s->st));
   if (s->nt > 0)
@@ -408,11 +431,8 @@ static int create_impl(int ninst, const int *node_off, const int *tet_off, const
   }
   // Tile size (tets per tile): 256, halved while the mesh would give fewer than 1024 tiles, and
   // while the tile pass could need more than 40 KiB of LDS (four workgroups per 160 KiB CU); a
-  // plan with tile_tets = t has at most t tets and max(64, t / 2) local nodes per tile.  FP64
-  // neo-Hookean arithmetic (not the mixed mode) takes 224 instead of 256: 27.0 KB of LDS per
-  // workgroup instead of 30.8 KB lets 6 workgroups share a CU, as many as the kernel's 6 waves
-  // per SIMD allow (FP64 tile pass 135.8 -> 131.3 us at 6.3 M tets; 224-tet tiles alone, at 5
-  // workgroups per CU, take 137.7 us).
+  // plan with tile_tets = t has at most t tets and max(64, t / 2) local nodes per tile (FP64
+  // neo-Hookean at 6.3 M tets: 115 us per tile pass, with 224-tet tiles 130).
   const bool f64 = p->precision == PBS_FP64;
   auto lds_need = [&](int lcap, int tcap) {
     TileDev t{};
@@ -424,7 +444,6 @@ static int create_impl(int ninst, const int *node_off, const int *tet_off, const
   if (tt == 0) {
     tt = 256;
     while (tt > 64 && (nt / tt < 1024 || lds_need(std::max(64, tt / 2), tt) > std::min<size_t>(s->lds_budget, 40960))) tt /= 2;
-    if (tt == 256 && f64 && p->material == 0 && !(p->mixed_switch > 0)) tt = 224;
   }
   std::string msg;
   const bool planned = inst_tiles ? build_batch_plan(ninst, node_off, tet_off, rest, tets, inst_tiles, s->plan, msg)
@@ -440,6 +459,7 @@ static int create_impl(int ninst, const int *node_off, const int *tet_off, const
   // one thread per tet of a full tile, in whole wavefronts, at most 256
   s->td.threads = std::min(256, std::max(64, (s->plan.tile_tets + 63) / 64 * 64));
   s->td.halo_total = s->plan.halo_total;
+  s->td.lstride = std::min(s->td.lcap, s->td.threads);
   s->td.ninst = ninst;
   s->td.nblk = 0;
   for (int i = 0; i < ninst; ++i) s->td.nblk += (node_off[i + 1] - node_off[i] + 255) / 256;
@@ -1122,7 +1142,7 @@ template <typename T> static int download_records(pbs_solver *s, const T *dev, f
 
 template <typename R> static int forces_impl(pbs_solver *s, const float *pos, float *tf, float *nf, float *te) {
   DevMesh<R> &m = mesh<R>(s);
-  int rc = upload_planes<R>(s, pos, m.ring.b[0]);
+  int rc = upload_ring<R>(s, pos);
   if (rc) return rc;
   Launch<R>::standalone_ctrl(m, 0, s->st);
   Launch<R>::tet(m, s->td, s->dp, s->bs, 0, 1, s->st);
@@ -1151,7 +1171,7 @@ extern "C" int pbs_compute_forces(pbs_solver *s, const float *pos, float *tf, fl
 
 template <typename R> static int hd_impl(pbs_solver *s, const float *pos, float *nh, float *th) {
   DevMesh<R> &m = mesh<R>(s);
-  int rc = upload_planes<R>(s, pos, m.ring.b[0]);
+  int rc = upload_ring<R>(s, pos);
   if (rc) return rc;
   Launch<R>::standalone_ctrl(m, 0, s->st);
   Launch<R>::tet(m, s->td, s->dp, s->bs, 1, 0, s->st);
@@ -1177,7 +1197,7 @@ extern "C" int pbs_compute_hessian_diag(pbs_solver *s, const float *pos, float *
 
 template <typename R> static int tile_forces_impl(pbs_solver *s, const float *pos, double *nf, double *nh, double *en) {
   DevMesh<R> &m = mesh<R>(s);
-  int rc = upload_planes<R>(s, pos, m.ring.b[0]);
+  int rc = upload_ring<R>(s, pos);
   if (rc) return rc;
   DevParams dp = s->dp;
   dp.f32math = 0;

@@ -25,6 +25,7 @@ namespace pbs {
 // the compiler may not hoist): left to itself, the compiler keeps all nine in 18 VGPRs across the
 // tet loop (FP64 tile pass: 94 instead of 85 VGPRs).  The arithmetic is the same either way.
 __device__ __forceinline__ double log_f64(double x) {
+#pragma clang fp contract(on)  // within a statement only: the same rounding wherever this is inlined
   double m = __builtin_amdgcn_frexp_mant(x);  // [0.5, 1)
   int e = __builtin_amdgcn_frexp_exp(x);
   if (m < 0.70710678118654752440) {

@@ -471,7 +471,7 @@ int tet_stiffness_run(pbs_solver *s, const float *pos, int num, const int *sid, 
   DevMesh<R> &m = mesh<R>(s);
   hipError_t e = hipMemcpyAsync(s->stage, pos, sizeof(float) * 3 * (size_t)s->nn, hipMemcpyHostToDevice, s->st);
   if (e == hipSuccess) {
-    Launch<R>::aos_to_planes(s->stage, m.ring.b[0], m.perm, s->nn, s->st);
+    Launch<R>::aos_to_nodes(s->stage, m.ring.b[0], m.perm, s->nn, s->st);
     e = hipMemcpyAsync(dids, sid, sizeof(int) * num, hipMemcpyHostToDevice, s->st);
   }
   if (e == hipSuccess) {

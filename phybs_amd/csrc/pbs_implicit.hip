@@ -311,7 +311,7 @@ __global__ void __launch_bounds__(kBlock)
 }
 
 // Per-tet stiffness K = -df/dx (12 x 12, rows 3 a + d, columns 3 b + e over the tet's corners a,
-// b and axes d, e) at the positions in planes x: the blocks of the closed form the assembly above
+// b and axes d, e) at the node-major positions x: the blocks of the closed form the assembly above
 // accumulates, one thread per requested tet (IsotropicMaterial::computeStiffnessMatrixFromPos,
 // IsotropicMaterial.cpp:503-552).  ids: solver tet ids; out: 144 FP32 values per requested tet.
 template <typename R, int MAT>
@@ -321,7 +321,7 @@ __global__ void k_tet_stiffness(DevParams p, int num, const int *__restrict__ id
                                 float *__restrict__ out) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= num) return;
-  const int t = ids[k], N = p.nn, T = p.nt;
+  const int t = ids[k], T = p.nt;
   const int4 q4 = tets[t];
   const int qn[4] = {q4.x, q4.y, q4.z, q4.w};
   R Dmi[9];
@@ -333,7 +333,7 @@ __global__ void k_tet_stiffness(DevParams p, int num, const int *__restrict__ id
 #pragma unroll
   for (int c = 0; c < 4; ++c)
 #pragma unroll
-    for (int d = 0; d < 3; ++d) X[c][d] = x[(size_t)d * N + qn[c]];
+    for (int d = 0; d < 3; ++d) X[c][d] = x[3 * (size_t)qn[c] + d];
   R Ds[9], F[9], C[9];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {

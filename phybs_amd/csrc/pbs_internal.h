@@ -55,6 +55,9 @@ struct TileDev {
   long halo_total;
   const TileInfo *tiles;
   const int *halo;
+  int lstride;                  // min(lcap, threads)
+  const int *ids;               // per tile, its first lstride local nodes (node ids; short tiles padded with
+                                // their first node), tile b at b * lstride
   const uint4 *tet_lp;          // per tet: corner local ids, corner contribution positions (16 bits each)
   const unsigned short *tile_off;
   const int *bnd_off;           // per node: its halo partial slots [bnd_off[n], bnd_off[n+1]), tile order
@@ -69,13 +72,14 @@ template <typename R> struct ContribWidth { static constexpr int value = 3; };
 template <> struct ContribWidth<float> { static constexpr int value = 4; };
 
 template <typename R> struct Ring {
-  R *b[4];  // each: 3 planes of nn values (x | y | z)
+  R *b[4];  // each: 3 nn values, node-major (xyz of a node together)
 };
 
 // Device buffers of one solver instance.
 template <typename R> struct DevMesh {
   int4 *tets;       // T (solver order, solver node ids)
   float *rest;      // 3 planes
+  float4 *rest4;    // the same per node (x, y, z, 0), for the tile pass's staging
   float *dmi;       // 9 planes of T (Dm^-1 row-major entry e at dmi[e*T + t])
   float *vol;       // T
   int *inc_off;     // N+1
@@ -87,10 +91,10 @@ template <typename R> struct DevMesh {
                     // this one array instead of mask and mass)
   float *gforce;    // 3 planes: mass (before the fixed override) * grav
   float *ext;       // 3 planes
-  float *hd;        // 3 planes: Hessian diagonal
+  float *hd;        // 3N node-major: Hessian diagonal
   R *frec;          // 12T per-tet force records
   float *hrec;      // 12T per-tet Hessian-diagonal records
-  R *xt;            // 3 planes: inertial target x~
+  R *xt;            // 3N node-major: inertial target x~
   R *xpos;          // 3 planes: positions at step start / after the step
   R *v, *vl;        // 3 planes each
   Ring<R> ring;
@@ -100,7 +104,7 @@ template <typename R> struct DevMesh {
   Ctrl *ctrl;
   int *flag;        // setup error flag
   R *tete;          // T, optional per-tet energy output
-  R *fown, *hpart;  // tile pass outputs: owned-node partial forces (3 planes of N), halo partials (3 x H)
+  R *fown, *hpart;  // tile pass outputs: owned-node partial forces (3N node-major), halo partials (3 x H)
   float *fownh, *hparth;  // the same for the Hessian diagonal
 };
 
@@ -131,6 +135,8 @@ template <typename R> struct Launch {
   static void aos_to_planes(const float *aos, R *planes, const int *perm, int n, hipStream_t st);
   static void planes_to_aos(const R *planes, float *aos, const int *perm, int n, hipStream_t st);
   static void planes_to_aos64(const R *planes, double *aos, const int *perm, int n, hipStream_t st);
+  static void aos_to_nodes(const float *aos, R *nodes, const int *perm, int n, hipStream_t st);
+  static void nodes_to_aos64(const R *nodes, double *aos, const int *perm, int n, hipStream_t st);
   static void aos64_to_planes(const double *aos, R *planes, const int *perm, int n, hipStream_t st);
 };
 // ---- learned warm start (pbs_learn.hip) ----

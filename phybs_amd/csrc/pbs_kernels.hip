@@ -8,8 +8,10 @@
 // CUDAInterface::doDescentOpt (CUDAInterface.cu:482-1007) with no host round trip and no atomics.
 // k_tet + k_gather evaluate forces and the Hessian diagonal for the standalone material calls.
 //
-// Layout: nodes are renumbered in Morton order and tets sorted by their smallest node; node
-// vectors are 3 planes (x | y | z) of nn values (SoA); per-tet rest data are 10 planes (Dm^-1
+// Layout: nodes are renumbered in Morton order and tets sorted by their smallest node.  The vectors
+// of the descent pass (iterates, inertial target, partial forces, Hessian diagonal) are node-major,
+// xyz of a node together, so that a tile's scattered halo nodes cost one access each and not three;
+// the state between steps is 3 planes (x | y | z) of nn values; per-tet rest data are 10 planes (Dm^-1
 // entries, volume) plus 16 bytes per tet of tile-local ids and contribution slots for the tile
 // pass; per-tet force records of the standalone calls are 12 consecutive values.
 #include <algorithm>
@@ -17,8 +19,7 @@
 
 #include <hip/hip_ext.h>
 
-#include "pbs_device.h"
-#include "pbs_internal.h"
+#include "pbs_pass.h"
 
 namespace pbs {
 
@@ -64,63 +65,12 @@ template <int N> __device__ __forceinline__ void block_sums(double (&v)[N], doub
   __syncthreads();
 }
 
-// Chebyshev schedule of the reference (CUDAInterface.cu:967-986; DescentOptimize.cpp:156-175).
-__device__ __forceinline__ void cheb_schedule(const DevParams &p, int k, float &rho, float &omega) {
-  if (k == 0) {
-    rho = 0.0f;
-    omega = 1.0f;
-  }
-  omega = 4.0f / (4.0f - rho * rho * omega);
-  for (int i = 0; i < p.profile_n; ++i) {
-    if (k == p.profile_k[i] - 1) {
-      rho = 0.0f;
-      omega = 1.0f;
-    }
-    if (k == p.profile_k[i]) {
-      rho = p.profile_rho[i];
-      omega = 2.0f / (2.0f - rho * rho);
-      break;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------------------------
 // Setup: rest-shape data (compute_DmInv_ANs_Mass, CUDAInterface.cu:273-325; TetMesh.cpp:189-216).
 // Contraction is off so that Dm^-1, volumes and masses round exactly as the FP32 reference
 // formulas written out without fused multiply-adds.
 // ---------------------------------------------------------------------------------------------
 #pragma clang fp contract(off)
-// Dm^-1 (row-major) and the volume |det Dm| / 6 of a rest tet from its corners' rest positions
-// r[c][k] (compute_DmInv_ANs_Mass, CUDAInterface.cu:273-325; TetMesh.cpp:189-216); returns det Dm.
-// The setup kernel and the tile pass both call this, so the tile pass's values are bitwise the
-// stored ones.
-__device__ __forceinline__ float rest_shape(const float r[4][3], float Dmi[9], float &V) {
-  float Dm[9], C[9];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const float x0 = r[0][k];
-    Dm[3 * k + 0] = r[1][k] - x0;
-    Dm[3 * k + 1] = r[2][k] - x0;
-    Dm[3 * k + 2] = r[3][k] - x0;
-  }
-  // adjugate and determinant written out here so that the no-contraction pragma applies
-  C[0] = Dm[4] * Dm[8] - Dm[7] * Dm[5];
-  C[1] = Dm[7] * Dm[2] - Dm[1] * Dm[8];
-  C[2] = Dm[1] * Dm[5] - Dm[4] * Dm[2];
-  C[3] = Dm[5] * Dm[6] - Dm[3] * Dm[8];
-  C[4] = Dm[0] * Dm[8] - Dm[2] * Dm[6];
-  C[5] = Dm[2] * Dm[3] - Dm[0] * Dm[5];
-  C[6] = Dm[3] * Dm[7] - Dm[4] * Dm[6];
-  C[7] = Dm[1] * Dm[6] - Dm[0] * Dm[7];
-  C[8] = Dm[0] * Dm[4] - Dm[1] * Dm[3];
-  const float det = Dm[0] * C[0] + Dm[3] * C[1] + Dm[6] * C[2];
-  V = fabsf(det) / 6.0f;
-  const float inv = 1.0f / det;
-#pragma unroll
-  for (int i = 0; i < 9; ++i) Dmi[i] = C[i] * inv;
-  return det;
-}
-
 __global__ void k_setup_tets(DevParams p, const float *__restrict__ rest, const int4 *__restrict__ tets,
                              float *__restrict__ dmi, float *__restrict__ vol, int *__restrict__ flag) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -180,7 +130,7 @@ __global__ void __launch_bounds__(256) k_tet(DevParams p, const Ctrl *__restrict
   const int hd = force_hd >= 0 ? force_hd : ctrl->hd_now;
   const R *__restrict__ x = ring.b[ctrl->cur];
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int N = p.nn, T = p.nt;
+  const int T = p.nt;
   double e = 0.0;
   if (t < T) {
     const int4 q = tets[t];
@@ -191,11 +141,10 @@ __global__ void __launch_bounds__(256) k_tet(DevParams p, const Ctrl *__restrict
     R Ds[9];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      const R *xk = x + (size_t)k * N;
-      const R x0 = xk[q.x];
-      Ds[3 * k + 0] = xk[q.y] - x0;
-      Ds[3 * k + 1] = xk[q.z] - x0;
-      Ds[3 * k + 2] = xk[q.w] - x0;
+      const R x0 = x[3 * (size_t)q.x + k];
+      Ds[3 * k + 0] = x[3 * (size_t)q.y + k] - x0;
+      Ds[3 * k + 1] = x[3 * (size_t)q.z + k] - x0;
+      Ds[3 * k + 2] = x[3 * (size_t)q.w + k] - x0;
     }
     R F[9];
     mul3(Ds, Dmi, F);
@@ -229,66 +178,6 @@ __global__ void __launch_bounds__(256) k_tet(DevParams p, const Ctrl *__restrict
   if (threadIdx.x == 0) etet[blockIdx.x] = s;
 }
 
-// ---------------------------------------------------------------------------------------------
-// Loop control of the reference (CUDAInterface.cu:917-1003) applied on the device after the
-// pass over iterate x_k: E = incremental potential at x_k (FP64), g2 = |g(x_k)|^2.
-// ---------------------------------------------------------------------------------------------
-__device__ void control_apply(const DevParams &p, Ctrl &C, double E, double g2) {
-  const double g = sqrt(g2);
-  C.g = g;
-  if (C.first) {
-    if (C.g0 < 0.0) C.g0 = g;
-    C.first = 0;
-  }
-  // (mixed mode: convergence is only declared on a pass with FP64 forces)
-  if (p.relgrad_tol > 0.0 && !p.f32math && g <= p.relgrad_tol * C.g0) {
-    C.converged = 1;
-    C.done = 1;
-    C.passes++;
-    return;
-  }
-  int rb = 0;
-  const bool robust = p.relgrad_tol > 0.0;
-  if (C.check_now) {
-    C.E = E;
-    // Rel-grad mode (no reference counterpart) also rejects a non-finite energy.
-    const bool worse = robust ? !(E <= C.E_old) : (E > C.E_old);
-    if (C.k != 0 && worse) {  // rollback (CUDAInterface.cu:946-958)
-      C.alpha *= p.alpha_decay;
-      if (robust) C.kc = C.k;  // rel-grad mode: keep the budget, restart Chebyshev at k
-      else C.budget -= C.k - p.energy_check;
-      C.cur = C.old;
-      C.rollbacks++;
-      rb = 1;
-    } else {
-      C.E_old = E;
-      C.old = C.cur;
-    }
-  }
-  if (!rb) {
-    C.rho = C.rho_next;
-    C.omega = C.omega_next;
-    C.last = C.cur;
-    C.cur = C.nxt;
-    int f = 0;
-    while (f == C.cur || f == C.last || f == C.old) ++f;
-    C.nxt = f;
-    C.k++;
-  }
-  C.passes++;
-  if (C.alpha < p.alpha_min || !(C.k < C.budget)) {
-    C.done = 1;
-  } else {
-    C.hd_now = (C.k % p.hd_refresh) == 0;
-    C.check_now = (C.k % p.energy_check) == 0;
-    float rho = C.rho, om = C.omega;
-    cheb_schedule(p, C.k - C.kc, rho, om);
-    C.rho_next = rho;
-    C.omega_next = om;
-    C.cheb_now = om != 1.0f;
-  }
-}
-
 // The fields of a control block that a descent pass's tile and node kernels read.
 struct PassCtl {
   int done, cur, nxt, last, hd_now, check_now, cheb_now;
@@ -309,136 +198,32 @@ __device__ __forceinline__ int xcd_tile(int bid, int nblk) {
   return start + k;
 }
 
-// One tet of a tile: F from the tile's LDS positions (stride 4 R per local node), the material
-// response, and its four corner contributions written to their slots of the LDS array rec (W
-// values each): forces on phase 0 (plus the clamped energy on check passes), Hessian-diagonal
-// entries rounded to FP32 on phase 1.  The arithmetic type C is R, or FP32 on FP64 positions (the
-// mixed mode).  Mixed mode: F is formed in R; the energy of check passes is evaluated in R from
-// that F (the same value the FP64 passes compute, so the line search compares like with like);
-// the neo-Hookean force is evaluated in FP32 from the displacement gradient H = F - I, whose FP32
-// rounding is relative to the strain instead of to 1; contributions are stored as FP32.
-template <typename R, typename C, int MAT>
-__device__ __forceinline__ void tile_tet(int phase, const uint4 lp, const float Dmf[9], float Vf,
-                                         const R *__restrict__ sx, C *__restrict__ rec, C mu, C lam, int chk, int clamp,
-                                         double &e_el) {
-  constexpr int W = ContribWidth<C>::value;
-  constexpr bool MIX = sizeof(C) < sizeof(R);
-  const R *p0 = sx + 4 * (lp.x & 0xffff), *p1 = sx + 4 * (lp.x >> 16), *p2 = sx + 4 * (lp.y & 0xffff),
-          *p3 = sx + 4 * (lp.y >> 16);
-  typedef typename std::conditional<MIX, R, C>::type FT;  // type F is formed in
-  FT Ds[9], Dm[9], Fw[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) Dm[k] = (FT)Dmf[k];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const R x0 = p0[k];
-    Ds[3 * k + 0] = (FT)(p1[k] - x0);
-    Ds[3 * k + 1] = (FT)(p2[k] - x0);
-    Ds[3 * k + 2] = (FT)(p3[k] - x0);
-  }
-  mul3(Ds, Dm, Fw);
-  C F[9], Dmi[9];
-#pragma unroll
-  for (int k = 0; k < 9; ++k) {
-    Dmi[k] = (C)Dmf[k];
-    F[k] = (C)Fw[k];
-  }
-  const C V = (C)Vf;
-  C f12[12], h12[12], en = (C)0;
-  const unsigned q[4] = {lp.z & 0xffff, lp.z >> 16, lp.w & 0xffff, lp.w >> 16};
-  if (phase == 0) {
-    if (MIX && MAT == 0) {
-      C H[9];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) H[k] = (C)(Fw[k] - ((k & 3) == 0 ? (FT)1 : (FT)0));
-      neo_tet_disp<C>(H, Dmi, V, mu, lam, f12);
-    } else if (MAT == 0) {
-      neo_tet<C, false>(F, Dmi, V, mu, lam, f12, en, h12);
-    } else {
-      stretch_tet<C, false>(F, Dmi, V, mu, lam, f12, en, h12);
-    }
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      C *r = rec + W * q[c];
-      r[0] = f12[3 * c];
-      r[1] = f12[3 * c + 1];
-      r[2] = f12[3 * c + 2];
-    }
-    if (chk) {
-      R er = MIX ? tet_energy<R, MAT>((const R *)Fw, (R)Vf, (R)mu, (R)lam) : (R)en;
-      if (clamp == 1) er = er > (R)0 ? er : (R)0;          // CUDAInterface.cu:549
-      else if (clamp == 2) er = er > (R)1e-6 ? er : (R)0;  // IsotropicNeohookeanMaterial.cpp:129
-      e_el += (double)er;
-    }
-  } else if (MAT == 0) {
-    // the neo-Hookean stiffness diagonal of neo_tet<C, true>, written corner by corner as it is
-    // formed (the 12 values are never all live: this phase sets the kernel's register count)
-    C Cf[9];
-    const C J = adj3(F, Cf);
-    const C iJ = (C)1 / J;
-    C Fi[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Fi[i] = Cf[i] * iJ;
-    const C k2 = mu + lam - lam * dlog(J);
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-      C c3[3];
-      if (n == 0) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) c3[j] = -((C)Dmf[j] + (C)Dmf[3 + j] + (C)Dmf[6 + j]);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) c3[j] = (C)Dmf[3 * (n - 1) + j];
-      }
-      const C cc = c3[0] * c3[0] + c3[1] * c3[1] + c3[2] * c3[2];
-      C h[3];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const C sd = c3[0] * Fi[d] + c3[1] * Fi[3 + d] + c3[2] * Fi[6 + d];
-        h[d] = V * (mu * cc + k2 * sd * sd);
-      }
-      C *r = rec + W * q[n];
-      r[0] = (C)(float)h[0];
-      r[1] = (C)(float)h[1];
-      r[2] = (C)(float)h[2];
-      // FP64: the store stays here (sunk to the end of the loop it would hold all 12 values)
-      if constexpr (sizeof(C) == 8) __builtin_amdgcn_sched_barrier(0);
-    }
-  } else {
-    stretch_tet<C, true>(F, Dmi, V, mu, lam, f12, en, h12);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      C *r = rec + W * q[c];
-      r[0] = (C)(float)h12[3 * c];
-      r[1] = (C)(float)h12[3 * c + 1];
-      r[2] = (C)(float)h12[3 * c + 2];
-    }
-  }
+// Local node i's run of contributions, and a halo node's partial slot.
+struct NodeRun {
+  unsigned run;  // first contribution, and the next run's in the high half
+  int slot;
+};
+__device__ __forceinline__ NodeRun node_run(const TileInfo &ti, const TileDev &td, int i) {
+  const unsigned short *off = td.tile_off + ti.off_start + i;
+  return {(unsigned)off[0] | (unsigned)off[1] << 16, i < ti.own_cnt ? 0 : td.halo_slot[ti.halo_off + (i - ti.own_cnt)]};
 }
 
 // Gather of one tile: each thread sums the contribution runs of its local nodes in order and
-// writes one partial per owned node (3 planes of N) and per halo node (xyz at its slot); the sums
+// writes one partial (xyz) per owned node and per halo node (at its slot); the sums
 // are formed in R whatever the contributions' type Q.
 template <typename R, typename Q>
 __device__ __forceinline__ void tile_gather(int phase, const TileInfo &ti, const TileDev &td, const Q *__restrict__ rec,
-                                            int N, R *__restrict__ fown, R *__restrict__ hpart,
+                                            NodeRun n0, R *__restrict__ fown, R *__restrict__ hpart,
                                             float *__restrict__ fownh, float *__restrict__ hparth) {
   constexpr int W = ContribWidth<Q>::value;
   const int L = ti.own_cnt + ti.halo_cnt;
-  const unsigned short *off = td.tile_off + ti.off_start;
   for (int i = threadIdx.x; i < L; i += blockDim.x) {
-    const int o0 = off[i], o1 = off[i + 1];
-    size_t d0, stride;
-    if (i < ti.own_cnt) {
-      d0 = (size_t)ti.own_start + i;
-      stride = N;
-    } else {
-      d0 = 3 * (size_t)td.halo_slot[ti.halo_off + (i - ti.own_cnt)];
-      stride = 1;
-    }
+    const NodeRun n = i == (int)threadIdx.x ? n0 : node_run(ti, td, i);
+    const int o0 = n.run & 0xffff, o1 = n.run >> 16;
+    const size_t d0 = 3 * (size_t)(i < ti.own_cnt ? ti.own_start + i : n.slot);
     // the run is summed in order; FP32 contributions are read 4 at a time ahead of their additions
-    // (slots past the run clamped to its first slot and not added: FP32 tile pass 85.6 -> 82.4 us
-    // at 6.3 M tets), FP64 ones one at a time (4 ahead: 148 -> 152 us)
+    // (slots past the run clamped to its first slot and not added: 4 % of the FP32 tile pass), FP64
+    // ones one at a time (4 ahead: 3 % slower)
     constexpr int U = sizeof(Q) == 4 ? 4 : 1;
     if (phase == 0) {
       R a0 = (R)0, a1 = (R)0, a2 = (R)0;
@@ -461,8 +246,8 @@ __device__ __forceinline__ void tile_gather(int phase, const TileInfo &ti, const
       }
       R *o = i < ti.own_cnt ? fown : hpart;
       o[d0] = a0;
-      o[stride + d0] = a1;
-      o[2 * stride + d0] = a2;
+      o[d0 + 1] = a1;
+      o[d0 + 2] = a2;
     } else {
       float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f;
       for (int j = o0; j < o1; j += U) {
@@ -484,8 +269,8 @@ __device__ __forceinline__ void tile_gather(int phase, const TileInfo &ti, const
       }
       float *o = i < ti.own_cnt ? fownh : hparth;
       o[d0] = a0;
-      o[stride + d0] = a1;
-      o[2 * stride + d0] = a2;
+      o[d0 + 1] = a1;
+      o[d0 + 2] = a2;
     }
   }
 }
@@ -514,66 +299,71 @@ template <typename R> __host__ __device__ inline size_t tile_rest_offset(const T
 // (phase 0 forces and energies; phase 1, when hd, the stiffness diagonal), gather each phase.
 template <typename R, int MAT, bool F32M>
 __device__ __forceinline__ void tile_body(const DevParams &p, int chk, const R *__restrict__ x, const TileDev &td,
-                                          int b, const TileInfo &ti, int hdnow, const float *__restrict__ rest,
+                                          int b, const TileInfo &ti, int node0, int hdnow, const float4 *__restrict__ rest,
                                           R *__restrict__ fown, R *__restrict__ hpart, float *__restrict__ fownh,
                                           float *__restrict__ hparth, unsigned char *smem, double *lds_red) {
-  const int L = ti.own_cnt + ti.halo_cnt, N = p.nn, tid = threadIdx.x;
+  const int L = ti.own_cnt + ti.halo_cnt, tid = threadIdx.x;
   typedef typename std::conditional<F32M, float, R>::type C;
   R *sx = (R *)smem;
   C *rec = (C *)(sx + 4 * td.lcap);
   float4 *srest = (float4 *)(smem + tile_rest_offset<R>(td));
   const int nthr = blockDim.x;
   // neo-Hookean: tet tid's local ids and slots, loaded before the staging so that they arrive with
-  // it (FP64 155 -> 148 us per launch at 6.3 M tets).  The stretch material's kernel would lose a
-  // wave per SIMD to the 4 registers it holds across the staging (FP32 137 -> 147 us), so it loads
-  // them after the barrier.
+  // it.  The stretch material's kernel would lose a wave per SIMD to the 4 registers it holds across
+  // the staging (FP32 137 -> 147 us), so it loads them after the barrier.
   constexpr bool PRE = MAT == 0;
   const uint4 lp0 = PRE && tid < ti.tet_cnt ? td.tet_lp[(size_t)ti.tet_start + tid] : make_uint4(0, 0, 0, 0);
   const C mu = (C)td.inst_mu[ti.inst], lam = (C)td.inst_lam[ti.inst];
-  for (int i = tid; i < L; i += nthr) {
-    const int g = i < ti.own_cnt ? ti.own_start + i : td.halo[ti.halo_off + i - ti.own_cnt];
-    sx[4 * i] = x[g];
-    sx[4 * i + 1] = x[N + g];
-    sx[4 * i + 2] = x[2 * (size_t)N + g];
-    srest[i] = make_float4(rest[g], rest[N + g], rest[2 * (size_t)N + g], 0.0f);
-  }
+  // the gather's descriptors of the thread's first local node, read now and not after the tets (FP32
+  // 70.8 -> 69.3 us at 6.3 M tets); the asm below keeps the reads from being moved back there
+  NodeRun n0 = {0, 0};
+  if (tid < L) n0 = node_run(ti, td, tid);
+  auto stage = [&](int i, int g) {
+    const R *xg = x + 3 * (size_t)g;
+    sx[4 * i] = xg[0];
+    sx[4 * i + 1] = xg[1];
+    sx[4 * i + 2] = xg[2];
+    srest[i] = rest[g];
+  };
+  // the first lstride local nodes: ids at a fixed stride, padded with valid ones, so that the staging
+  // waits for no descriptor (node0 was read together with it)
+  if (tid < td.lstride) stage(tid, node0);
+  for (int i = td.lstride + tid; i < L; i += nthr)
+    stage(i, i < ti.own_cnt ? ti.own_start + i : td.halo[ti.halo_off + i - ti.own_cnt]);
+  asm volatile("" ::"v"(n0.run), "v"(n0.slot));
   __syncthreads();
   double e_el = 0.0;
   // the tile's tets and their gather for one phase
-  auto run_phase = [&](int phase) {
+  auto run_phase = [&](auto ph) {
+    constexpr int phase = decltype(ph)::value;
     for (int s = tid; s < ti.tet_cnt; s += nthr) {
       const uint4 lp = PRE && s == tid ? lp0 : td.tet_lp[(size_t)ti.tet_start + s];
-      const int lid[4] = {(int)(lp.x & 0xffff), (int)(lp.x >> 16), (int)(lp.y & 0xffff), (int)(lp.y >> 16)};
-      float r[4][3];
+      auto get_r = [&](float (&r)[4][3]) {
+        const int lid[4] = {(int)(lp.x & 0xffff), (int)(lp.x >> 16), (int)(lp.y & 0xffff), (int)(lp.y >> 16)};
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float4 q = srest[lid[c]];
-        r[c][0] = q.x;
-        r[c][1] = q.y;
-        r[c][2] = q.z;
-      }
-      float Dmf[9], Vf;
-      rest_shape(r, Dmf, Vf);
-      tile_tet<R, C, MAT>(phase, lp, Dmf, Vf, sx, rec, mu, lam, chk, p.clamp, e_el);
+        for (int c = 0; c < 4; ++c) {
+          const float4 q = srest[lid[c]];
+          r[c][0] = q.x;
+          r[c][1] = q.y;
+          r[c][2] = q.z;
+        }
+      };
+      auto get_neo = [&]() {
+        float r[4][3];
+        get_r(r);
+        return NeoRest<C>(r, mu);
+      };
+      tile_tet<R, C, MAT, phase>(lp, get_r, get_neo, sx, rec, mu, lam, chk, p.clamp, e_el);
     }
     __syncthreads();
-    tile_gather<R>(phase, ti, td, rec, N, fown, hpart, fownh, hparth);
+    tile_gather<R>(phase, ti, td, rec, n0, fown, hpart, fownh, hparth);
   };
-  if constexpr (sizeof(C) == 8) {
-    // FP64 arithmetic: the two phases as separate code.  As one loop over the phase the compiler
-    // shares their common arithmetic and keeps its constants in registers, and the neo-Hookean
-    // kernel needs 114 VGPRs (4 waves per SIMD); as separate code, 94 (5 waves; 144 -> 139 us
-    // per launch at 6.3 M tets), and 78 with the logarithm's constants in scalar registers.
-    run_phase(0);
-    if (hdnow) {
-      __syncthreads();  // the Hessian phase reuses the contribution slots
-      run_phase(1);
-    }
-  } else {
-    for (int phase = 0; phase <= hdnow; ++phase) {
-      run_phase(phase);
-      if (phase == 0 && hdnow) __syncthreads();
-    }
+  // The two phases as separate code: as one loop over the phase the compiler would share their common
+  // arithmetic, which the forces of the one do not need.
+  run_phase(std::integral_constant<int, 0>());
+  if (hdnow) {
+    __syncthreads();  // the Hessian phase reuses the contribution slots
+    run_phase(std::integral_constant<int, 1>());
   }
   if (chk) {
     const double se = block_sum(e_el, lds_red);
@@ -582,11 +372,19 @@ __device__ __forceinline__ void tile_body(const DevParams &p, int chk, const R *
 }
 
 // F32M (FP64 state only): the per-tet arithmetic in FP32 after F (the mixed mode's early passes).
-// The FP64 neo-Hookean kernel is held to 6 waves per SIMD (at most 80 VGPRs: it needs 78 without
-// spilling), which pays with tiles small enough for 6 workgroups' LDS (224 tets, see pbs_create).
+//
+// Bound: the staging's scattered halo reads and the LDS traffic of contributions, not the arithmetic
+// (forces with a third fewer FP32 instructions left its time as it was).  So node data is node-major
+// (the three components of a node in one cache line, its rest position one 16-byte read, instead of
+// three lines each), the first lstride ids and the thread's contribution run are read with the
+// descriptor instead of after it, and the neo-Hookean force takes one 3x3 product (neo_force).  Per
+// launch on 6.3 M tets (64x64x256 cells), before -> now: FP32 73 -> 69 us, FP64 139 -> 115, stretch
+// FP32 121 -> 122.  The FP64 neo-Hookean kernel is held to 5 waves per SIMD (at most 102 VGPRs, no
+// spilling), as many as the LDS of 256-tet tiles allows (30.8 KB: 5 workgroups per CU).  6 waves with
+// 224-tet tiles spill (130 us), 4 waves 114 us.
 template <typename R, int MAT, bool F32M>
-__global__ void __launch_bounds__(256, (sizeof(R) == 8 && MAT == 0 && !F32M) ? 6 : 1)
-k_tile(DevParams p, const Ctrl *__restrict__ ctrl, Ring<R> ring, TileDev td, const float *__restrict__ rest,
+__global__ void __launch_bounds__(256, (sizeof(R) == 8 && MAT == 0 && !F32M) ? 5 : 1)
+k_tile(DevParams p, const Ctrl *__restrict__ ctrl, Ring<R> ring, TileDev td, const float4 *__restrict__ rest,
        R *__restrict__ fown, R *__restrict__ hpart, float *__restrict__ fownh, float *__restrict__ hparth) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double lds_red[16];
@@ -595,14 +393,17 @@ k_tile(DevParams p, const Ctrl *__restrict__ ctrl, Ring<R> ring, TileDev td, con
   // after it, so the staging loads wait for one dependent memory access less.  Several: the
   // tile's instance's block, read once the descriptor has arrived.
   PassCtl c = pass_ctl(ctrl);
+  const int node0 = (int)threadIdx.x < td.lstride ? td.ids[(size_t)b * td.lstride + threadIdx.x] : 0;
   const TileInfo ti = td.tiles[b];
   // both reads in flight before either is waited for (otherwise the compiler folds the first into
   // the second, which waits for the descriptor)
   asm volatile("" ::"s"(c.done), "s"(c.cur), "s"(c.hd_now), "s"(c.check_now), "s"(ti.inst));
   if (td.ninst != 1) c = pass_ctl(ctrl + ti.inst);
   if (c.done) return;
-  tile_body<R, MAT, F32M>(p, c.check_now, ring.b[c.cur], td, b, ti, c.hd_now, rest, fown, hpart, fownh, hparth, smem,
-                          lds_red);
+  // (the buffer's pointer is selected, not indexed: that would be one more dependent memory access)
+  const R *x01 = c.cur & 1 ? ring.b[1] : ring.b[0], *x23 = c.cur & 1 ? ring.b[3] : ring.b[2];
+  tile_body<R, MAT, F32M>(p, c.check_now, c.cur & 2 ? x23 : x01, td, b, ti, node0, c.hd_now, rest, fown, hpart, fownh,
+                          hparth, smem, lds_red);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -650,7 +451,7 @@ k_node(DevParams p, const Ctrl *__restrict__ ctrl, Ring<R> ring, TileDev td, con
     float hv[3], ev[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      const size_t i = (size_t)d * N + n;
+      const size_t i = 3 * (size_t)n + d;
       f[d] = fown[i];
       xc[d] = x[i];
       xtv[d] = xt[i];
@@ -660,13 +461,13 @@ k_node(DevParams p, const Ctrl *__restrict__ ctrl, Ring<R> ring, TileDev td, con
     }
     if (!GRAD_ONLY && cheb)
 #pragma unroll
-      for (int d = 0; d < 3; ++d) xlv[d] = xl[(size_t)d * N + n];
+      for (int d = 0; d < 3; ++d) xlv[d] = xl[3 * (size_t)n + d];
     if (p.has_ext)
 #pragma unroll
       for (int d = 0; d < 3; ++d) ev[d] = ext[(size_t)d * N + n];
     if (!GRAD_ONLY)
 #pragma unroll
-      for (int d = 0; d < 3; ++d) hv[d] = hdnow ? fownh[(size_t)d * N + n] : hd[(size_t)d * N + n];
+      for (int d = 0; d < 3; ++d) hv[d] = hdnow ? fownh[3 * (size_t)n + d] : hd[3 * (size_t)n + d];
     for (int e = b0; e < b1; ++e) {
       const R *hp = hpart + 3 * (size_t)e;
 #pragma unroll
@@ -679,12 +480,12 @@ k_node(DevParams p, const Ctrl *__restrict__ ctrl, Ring<R> ring, TileDev td, con
         for (int d = 0; d < 3; ++d) hv[d] += hp[d];
       }
 #pragma unroll
-      for (int d = 0; d < 3; ++d) hd[(size_t)d * N + n] = hv[d];
+      for (int d = 0; d < 3; ++d) hd[3 * (size_t)n + d] = hv[d];
     }
     if (fixed) {
       if (!GRAD_ONLY)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) xn[(size_t)d * N + n] = xc[d];
+        for (int d = 0; d < 3; ++d) xn[3 * (size_t)n + d] = xc[d];
     } else {
       const R hstep = (R)p.h;
       const R mh2 = (R)m / (hstep * hstep);
@@ -701,7 +502,7 @@ k_node(DevParams p, const Ctrl *__restrict__ ctrl, Ring<R> ring, TileDev td, con
         if (!GRAD_ONLY) {
           R nx = xc[d] - alpha * gr / ((R)hv[d] + mh2);
           if (cheb) nx = om * (nx - xlv[d]) + xlv[d];
-          xn[(size_t)d * N + n] = nx;
+          xn[3 * (size_t)n + d] = nx;
         }
       }
       if (!GRAD_ONLY) en += (double)e;
@@ -813,12 +614,12 @@ __global__ void k_step_init(DevParams p, Ctrl *__restrict__ ctrl, int ninst, Rin
     for (int d = 0; d < 3; ++d) {
       const size_t i = (size_t)d * p.nn + n;
       const R t = xpos[i] + v[i] * h;
-      xt[i] = t;
+      xt[3 * (size_t)n + d] = t;
       R x0;
       if (p.semantics == 1) x0 = t + (R)(p.init_momentum * p.h) * (v[i] - vl[i]);
       else if (sizeof(R) == 4) x0 = (R)((double)t + (double)p.init_momentum * (double)(v[i] - vl[i]) * (double)p.h);
       else x0 = t + (R)p.init_momentum * (v[i] - vl[i]) * h;
-      ring.b[0][i] = x0;
+      ring.b[0][3 * (size_t)n + d] = x0;
     }
   }
   if (n < ninst) {  // one control block per instance
@@ -871,13 +672,13 @@ __global__ void k_step_final(DevParams p, const Ctrl *__restrict__ ctrl, TileDev
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     const size_t i = (size_t)d * p.nn + n;
-    const R xf = x[i];
+    const R xf = x[3 * (size_t)n + d];
     if (p.semantics == 1) {
       vl[i] = v[i];
       v[i] = (R)p.damping * (xf - xpos[i]) / h;
     } else if (!mask[n]) {
       vl[i] = v[i];
-      const R vv = v[i] + (xf - xt[i]) * ((R)1 / h);
+      const R vv = v[i] + (xf - xt[3 * (size_t)n + d]) * ((R)1 / h);
       v[i] = (sizeof(R) == 4) ? (R)((double)vv * (double)p.damping) : vv * (R)p.damping;
     }
     xpos[i] = xf;
@@ -912,7 +713,7 @@ __global__ void k_sum_partials(TileDev td, int N, int which, const R *__restrict
   if (which == 0) {
     R f[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) f[d] = fown[(size_t)d * N + n];
+    for (int d = 0; d < 3; ++d) f[d] = fown[3 * (size_t)n + d];
     for (int e = b0; e < b1; ++e)
 #pragma unroll
       for (int d = 0; d < 3; ++d) f[d] += hpart[3 * (size_t)e + d];
@@ -921,7 +722,7 @@ __global__ void k_sum_partials(TileDev td, int N, int which, const R *__restrict
   } else {
     float h[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) h[d] = fownh[(size_t)d * N + n];
+    for (int d = 0; d < 3; ++d) h[d] = fownh[3 * (size_t)n + d];
     for (int e = b0; e < b1; ++e)
 #pragma unroll
       for (int d = 0; d < 3; ++d) h[d] += hparth[3 * (size_t)e + d];
@@ -965,6 +766,24 @@ __global__ void k_planes_to_aos(const A *__restrict__ planes, B *__restrict__ ao
   const size_t o = 3 * (size_t)(perm ? perm[i] : i);
 #pragma unroll
   for (int d = 0; d < 3; ++d) aos[o + d] = (B)planes[(size_t)d * n + i];
+}
+
+// AoS (caller's node order) <-> node-major (solver's node order).
+template <typename A, typename B>
+__global__ void k_aos_to_nodes(const A *__restrict__ aos, B *__restrict__ nodes, const int *__restrict__ perm, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const size_t o = 3 * (size_t)perm[i];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) nodes[3 * (size_t)i + d] = (B)aos[o + d];
+}
+template <typename A, typename B>
+__global__ void k_nodes_to_aos(const A *__restrict__ nodes, B *__restrict__ aos, const int *__restrict__ perm, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const size_t o = 3 * (size_t)perm[i];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) aos[o + d] = (B)nodes[3 * (size_t)i + d];
 }
 
 __global__ void k_fill(float *p, float v, long n) {
@@ -1015,7 +834,7 @@ void Launch<R>::tile_pass(const DevMesh<R> &m, const TileDev &td, const DevParam
   const bool f32m = sizeof(R) == 8 && p.f32math;
 #define PBS_TILE_LAUNCH(MAT, F32M)                                                                               \
   launch_timed(k_tile<R, MAT, F32M>, dim3(td.ntiles), dim3(td.threads), lds, st, e0, e1, p, m.ctrl, m.ring, td, \
-               m.rest, m.fown, m.hpart, m.fownh, m.hparth)
+               m.rest4, m.fown, m.hpart, m.fownh, m.hparth)
   if (p.material == 0 && !f32m) PBS_TILE_LAUNCH(0, false);
   else if (p.material == 0) PBS_TILE_LAUNCH(0, true);
   else if (!f32m) PBS_TILE_LAUNCH(1, false);
@@ -1080,6 +899,14 @@ void Launch<R>::planes_to_aos64(const R *planes, double *aos, const int *perm, i
 template <typename R>
 void Launch<R>::aos64_to_planes(const double *aos, R *planes, const int *perm, int n, hipStream_t st) {
   hipLaunchKernelGGL((k_aos_to_planes<double, R>), dim3(nblk(n, 256)), dim3(256), 0, st, aos, planes, perm, n);
+}
+template <typename R>
+void Launch<R>::aos_to_nodes(const float *aos, R *nodes, const int *perm, int n, hipStream_t st) {
+  hipLaunchKernelGGL((k_aos_to_nodes<float, R>), dim3(nblk(n, 256)), dim3(256), 0, st, aos, nodes, perm, n);
+}
+template <typename R>
+void Launch<R>::nodes_to_aos64(const R *nodes, double *aos, const int *perm, int n, hipStream_t st) {
+  hipLaunchKernelGGL((k_nodes_to_aos<R, double>), dim3(nblk(n, 256)), dim3(256), 0, st, nodes, aos, perm, n);
 }
 void aos_to_planes_f(const float *aos, float *planes, const int *perm, int n, hipStream_t st) {
   hipLaunchKernelGGL((k_aos_to_planes<float, float>), dim3(nblk(n, 256)), dim3(256), 0, st, aos, planes, perm, n);

@@ -471,7 +471,7 @@ template <typename R> static int guess_impl(pbs_solver *s, LearnState *L, double
   for (int which = 0; which < 2; ++which) {
     double *dst = which ? learned : plain;
     if (!dst) continue;
-    Launch<R>::planes_to_aos64(m.ring.b[which], s->stage64, m.perm, s->nn, s->st);
+    Launch<R>::nodes_to_aos64(m.ring.b[which], s->stage64, m.perm, s->nn, s->st);
     HIPCHK(hipMemcpyAsync(dst, s->stage64, sizeof(double) * 3 * (size_t)s->nn, hipMemcpyDeviceToHost, s->st));
   }
   HIPCHK(hipStreamSynchronize(s->st));

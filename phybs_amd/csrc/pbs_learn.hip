@@ -213,8 +213,8 @@ __global__ void __launch_bounds__(256) k_guess(DevParams p, MlpDev net, const fl
       const bool fixed = mask[n] != 0;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const size_t i = (size_t)d * N + n;
-        out[i] = fixed ? plain[i] : y[i] + (R)(o[d] * s_out);
+        const size_t i = 3 * (size_t)n + d;
+        out[i] = fixed ? plain[i] : y[(size_t)d * N + n] + (R)(o[d] * s_out);
       }
     }
   }
@@ -234,7 +234,7 @@ __global__ void k_corr_diff(int N, const int *__restrict__ mask, const R *__rest
   float v[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const size_t i = (size_t)k * N + n;
+    const size_t i = 3 * (size_t)n + k;
     v[k] = mask[n] ? 0.0f : (float)(learned[i] - plain[i]);
   }
   d[n] = make_float4(v[0], v[1], v[2], 0.0f);
@@ -281,7 +281,7 @@ __global__ void k_corr_apply(int N, const Ctrl *__restrict__ ctrl, float beta, c
   const float dv[3] = {v.x, v.y, v.z};
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const size_t i = (size_t)k * N + n;
+    const size_t i = 3 * (size_t)n + k;
     out[i] = plain[i] + b * (R)dv[k];
   }
 }
@@ -325,7 +325,8 @@ __global__ void __launch_bounds__(1024) k_ws_stage(Ctrl *__restrict__ ctrl, cons
       C.cur = use ? 1 : 0;
       C.nxt = use ? 0 : 1;
       C.used_learned = use ? 1 : 0;
-      C.g0 = sqrt(C.g_plain);
+      // (a rejected guess leaves g0 to the first pass, which is then the plain step's own)
+      if (use) C.g0 = sqrt(C.g_plain);
       C.hd_now = 1;
       C.check_now = 1;
     }
