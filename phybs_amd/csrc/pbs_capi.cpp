@@ -241,7 +241,7 @@ template <typename R> static int alloc_impl(pbs_solver *s) {
   s->td.tile_off = toff;
   s->td.bnd_off = bnd_off;
   s->td.halo_slot = hslot;
-  rc |= dalloc(s, &m.ctrl, (size_t)s->ninst);
+  rc |= dalloc(s, &m.ctrl, (size_t)s->ninst + 1);  // the last one: the resident loop's abort flag
   {
     int *a;
     float *f;
@@ -262,6 +262,65 @@ template <typename R> static int alloc_impl(pbs_solver *s) {
   rc |= dalloc(s, &s->stage, 3 * N);
   rc |= dalloc(s, &s->stage64, 3 * N);
   return rc ? PBS_ERR_HIP : PBS_OK;
+}
+
+// The resident descent loop (pbs_persist.hip) of a single mesh with the default tile size and graph
+// length: plan, device arrays and exchange buffers, where the mesh fits it.  Parts of at least 32
+// nodes, at most one per CU, at most 168 nodes each (8 waves of 21), so 43,000 nodes at most.  It is
+// the faster path up to there: us per pass, resident against launches, 45 nodes 4.8 : 10.4, 8.6 K
+// nodes 8.2 : 13.6 (FP64 7.1 : 14.2), 21 K nodes 9.8 : 14.0 (8.4 : 15.5), 40 K nodes 9.9 : 15.4
+// (10.6 : 17.9).
+constexpr int kPersistNodes = 40000;
+template <typename R> static int persist_setup(pbs_solver *s) {
+  s->persist = PersistDev{};
+  if (s->ninst != 1 || s->nt == 0 || s->nn > kPersistNodes) return PBS_OK;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess) return PBS_OK;
+  PersistPlan Q;
+  if (!build_persist_plan(s->plan, std::min(cus, 256), 32, Q)) return PBS_OK;
+  if (Q.own_max > kPersistOwn || Q.ghost_max > kPersistGhosts || Q.tet_max > kPersistTetsPerThread * kPersistThreads)
+    return PBS_OK;
+  PersistDev d{};
+  d.nparts = (int)Q.parts.size();
+  d.tet_max = Q.tet_max;
+  d.local_max = Q.local_max;
+  d.slot_max = Q.slot_max;
+  if (PersistLaunch<R>::lds_bytes(d) + 1024 > s->lds_budget) return PBS_OK;
+  if (std::min(PersistLaunch<R>::max_resident(d, 0, s->device), PersistLaunch<R>::max_resident(d, 1, s->device)) < d.nparts)
+    return PBS_OK;
+  const size_t xb = (4 * 3 * (size_t)s->nn * sizeof(R) + 15) / 16 * 16, pb = 4 * 2 * (size_t)d.nparts * sizeof(double);
+  PersistPart *parts;
+  int *ghost;
+  uint32_t *lp;
+  unsigned short *run;
+  unsigned long long *mask;
+  unsigned char *xch;
+  int rc = dalloc(s, &parts, Q.parts.size());
+  rc |= dalloc(s, &ghost, Q.ghost.size());
+  rc |= dalloc(s, &lp, Q.lp.size());
+  rc |= dalloc(s, &run, Q.run.size());
+  rc |= dalloc(s, &mask, Q.mask.size());
+  rc |= dalloc(s, &xch, xb + pb);
+  if (rc) return PBS_ERR_HIP;
+  auto up = [&](void *to, const void *from, size_t bytes) {
+    return bytes ? hipMemcpy(to, from, bytes, hipMemcpyHostToDevice) : hipSuccess;
+  };
+  HIPCHK(up(parts, Q.parts.data(), sizeof(PersistPart) * Q.parts.size()));
+  HIPCHK(up(ghost, Q.ghost.data(), sizeof(int) * Q.ghost.size()));
+  HIPCHK(up(lp, Q.lp.data(), sizeof(uint32_t) * Q.lp.size()));
+  HIPCHK(up(run, Q.run.data(), sizeof(uint16_t) * Q.run.size()));
+  HIPCHK(up(mask, Q.mask.data(), sizeof(uint64_t) * Q.mask.size()));
+  d.parts = parts;
+  d.ghost = ghost;
+  d.lp = (const uint4 *)lp;
+  d.run = run;
+  d.mask = mask;
+  d.xch = xch;
+  d.part = (double *)(xch + xb);
+  d.xch_bytes = (long)(xb + pb);
+  d.abort = (int *)(mesh<R>(s).ctrl + s->ninst);
+  s->persist = d;
+  return PBS_OK;
 }
 
 template <typename R> static int setup_impl(pbs_solver *s, const int *mask) {
@@ -471,6 +530,10 @@ static int create_impl(int ninst, const int *node_off, const int *tet_off, const
   if (rc) return fail(rc);
   rc = p->precision == PBS_FP64 ? setup_impl<double>(s, mask) : setup_impl<float>(s, mask);
   if (rc) return fail(rc);
+  if (tile_tets == 0 && !inst_tiles) {
+    rc = p->precision == PBS_FP64 ? persist_setup<double>(s) : persist_setup<float>(s);
+    if (rc) return fail(rc);
+  }
   if (nodes) {
     rc = p->precision == PBS_FP64 ? set_positions_impl<double>(s, nodes) : set_positions_impl<float>(s, nodes);
     if (rc) return fail(rc);
@@ -945,15 +1008,23 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
   const int period = s->prof_period;
   s->dp.f32math = 0;  // step start, warm start and eager passes: FP64 arithmetic
   HIPCHK(hipEventRecord(s->ev0, s->st));
-  s->pass_ordinal = -1;
-  int i = timed_begin(s, K_INIT);
-  Launch<R>::step_init(m, s->td, s->dp, s->bs, s->st);
-  timed_end(s, i);
-  HIPCHK(hipGetLastError());
-  if (s->learn) {  // features / learned guess / selection by gradient norm
-    i = timed_begin(s, K_LEARN);
-    int rc = learn_before_descent<R>(s);
+  int i = -1;
+  auto begin_step = [&]() -> int {
+    s->pass_ordinal = -1;
+    i = timed_begin(s, K_INIT);
+    Launch<R>::step_init(m, s->td, s->dp, s->bs, s->st);
     timed_end(s, i);
+    HIPCHK(hipGetLastError());
+    if (s->learn) {  // features / learned guess / selection by gradient norm
+      i = timed_begin(s, K_LEARN);
+      int rc = learn_before_descent<R>(s);
+      timed_end(s, i);
+      if (rc) return rc;
+    }
+    return PBS_OK;
+  };
+  {
+    int rc = begin_step();
     if (rc) return rc;
   }
   const bool relg = s->dp.relgrad_tol > 0;
@@ -998,6 +1069,32 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
     }
   }
   while (true) {
+    // the resident loop: the default graph length, no timing of single kernels, no mixed mode
+    if (s->persist.nparts > 0 && s->p.graph_passes == 0 && !period && !mixed) {
+      // one launch runs the step (at most 4096 passes at a time)
+      const int most = (int)std::min<long>(std::max<long>(cap - launched, 1), 4096);
+      Ctrl two[2];  // the control block and the abort flag behind it
+      hipError_t e = PersistLaunch<R>::run(m, s->td, s->dp, s->persist, most, s->st);
+      if (e == hipSuccess) e = hipMemcpyAsync(two, m.ctrl, sizeof(two), hipMemcpyDeviceToHost, s->st);
+      if (e == hipSuccess) {
+        HIPCHK(hipStreamSynchronize(s->st));
+        int gave_up;
+        std::memcpy(&gave_up, &two[1], sizeof(int));
+        if (!gave_up) {
+          ch[0] = two[0];
+          launched += most;
+          if (all_done()) break;
+          if (launched >= cap) return set_error(PBS_ERR_STATE, "descent loop did not terminate within the pass cap");
+          continue;
+        }
+      }
+      // not launchable, or its workgroups did not all run: the step starts again on the other path
+      (void)hipGetLastError();
+      s->persist.nparts = 0;
+      int rc = begin_step();
+      if (rc) return rc;
+      launched = 0;
+    }
     if (use_graph) {
       if (!fp64_phase) {
         double worst = -1.0;

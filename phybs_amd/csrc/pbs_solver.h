@@ -9,6 +9,7 @@
 
 #include "pbs_host.h"
 #include "pbs_internal.h"
+#include "pbs_persist.h"
 #include "pbs_tiles.h"
 #include "phybs.h"
 
@@ -53,6 +54,7 @@ struct pbs_solver {
   TileDev td{};
   TilePlan plan;
   size_t lds_budget = 65536;
+  PersistDev persist{};       // resident descent loop of a small mesh (nparts 0: not used)
   std::vector<float> rest_h;
   float *stage = nullptr;     // 3N float AoS staging
   double *stage64 = nullptr;  // 3N double AoS staging

@@ -285,4 +285,99 @@ bool build_batch_plan(int ninst, const int *node_off, const int *tet_off, const 
   return true;
 }
 
+bool build_persist_plan(const TilePlan &P, int max_parts, int nodes_per_part, PersistPlan &Q) {
+  Q = PersistPlan();
+  const int N = P.nn;
+  const int G = std::max(1, std::min(max_parts, N / std::max(nodes_per_part, 1)));
+  std::vector<int> tile_of(P.nt), min_node(P.nt);
+  for (int b = 0; b < P.ntiles; ++b)
+    for (int t = P.tiles[b].tet_start; t < P.tiles[b].tet_start + P.tiles[b].tet_cnt; ++t) tile_of[t] = b;
+  for (int t = 0; t < P.nt; ++t)
+    min_node[t] = *std::min_element(&P.tets_new[4 * (size_t)t], &P.tets_new[4 * (size_t)t] + 4);
+  std::vector<int> tile_of_node(N);
+  for (int b = 0; b < P.ntiles; ++b)
+    for (int n = P.tiles[b].own_start; n < P.tiles[b].own_start + P.tiles[b].own_cnt; ++n) tile_of_node[n] = b;
+  // loc: a node's local id in the current part; at_tet: a tet's entry in it (valid where part_of says so)
+  std::vector<int> loc(N), ghost_of(N, -1), at_tet(P.nt), part_of(P.nt, -1), tets, ghosts, inc;
+  std::vector<uint16_t> slot;
+  Q.lp.reserve(5 * (size_t)P.nt);
+  Q.tet.reserve(P.nt + P.nt / 4);
+  for (int g = 0; g < G; ++g) {
+    PersistPart p{};
+    p.own_start = (int)((long)N * g / G);
+    const int n1 = (int)((long)N * (g + 1) / G);
+    p.own_cnt = n1 - p.own_start;
+    tets.clear();
+    for (int e = P.inc_off[p.own_start]; e < P.inc_off[n1]; ++e) {
+      const int t = P.inc[e] >> 2;
+      if (part_of[t] != g) tets.push_back(t);
+      part_of[t] = g;
+    }
+    std::sort(tets.begin(), tets.end());
+    ghosts.clear();
+    for (size_t k = 0; k < tets.size(); ++k) {
+      at_tet[tets[k]] = (int)k;
+      for (int j = 0; j < 4; ++j) {
+        const int n = P.tets_new[4 * (size_t)tets[k] + j];
+        if ((n < p.own_start || n >= n1) && ghost_of[n] != g) {
+          ghost_of[n] = g;
+          ghosts.push_back(n);
+        }
+      }
+    }
+    std::sort(ghosts.begin(), ghosts.end());
+    p.ghost_off = (int)Q.ghost.size();
+    p.ghost_cnt = (int)ghosts.size();
+    p.tet_off = (int)Q.tet.size();
+    p.tet_cnt = (int)tets.size();
+    p.run_off = (int)Q.run.size();
+    p.slots = P.inc_off[n1] - P.inc_off[p.own_start];
+    if (p.own_cnt + p.ghost_cnt > 0xffff || p.slots + 64 > 0x7fff) return false;
+    for (int k = 0; k < p.own_cnt; ++k) loc[p.own_start + k] = k;
+    for (int k = 0; k < p.ghost_cnt; ++k) loc[ghosts[k]] = p.own_cnt + k;
+    slot.resize(4 * tets.size());
+    for (size_t k = 0; k < slot.size(); ++k) slot[k] = (uint16_t)(p.slots + ((k >> 2) & 63));
+    int at = 0;
+    for (int n = p.own_start; n < n1; ++n) {
+      // entries 4 tet + corner: the node's own tile first, then tile order (tets ascend with tiles)
+      inc.assign(P.inc.begin() + P.inc_off[n], P.inc.begin() + P.inc_off[n + 1]);
+      std::sort(inc.begin(), inc.end());
+      const auto own = [&](int e) { return tile_of[e >> 2] == tile_of_node[n]; };
+      const auto o0 = std::find_if(inc.begin(), inc.end(), own);
+      std::rotate(inc.begin(), o0, std::find_if_not(o0, inc.end(), own));
+      if (inc.size() > 64) return false;
+      uint64_t m = 0;
+      Q.run.push_back((uint16_t)at);
+      for (size_t k = 0; k < inc.size(); ++k) {
+        if (k + 1 == inc.size() || tile_of[inc[k + 1] >> 2] != tile_of[inc[k] >> 2]) m |= 1ULL << k;
+        const size_t i = (size_t)at_tet[inc[k] >> 2];
+        slot[4 * i + (inc[k] & 3)] = (uint16_t)at++;
+      }
+      Q.mask.push_back(m);
+    }
+    Q.run.push_back((uint16_t)at);
+    Q.mask.push_back(0);
+    for (size_t k = 0; k < tets.size(); ++k) {
+      const int t = tets[k];
+      uint32_t l[4];
+      for (int j = 0; j < 4; ++j) l[j] = (uint32_t)loc[P.tets_new[4 * (size_t)t + j]];
+      const uint16_t *q = &slot[4 * k];
+      const uint32_t own = min_node[t] >= p.own_start && min_node[t] < n1 ? 0x80000000u : 0u;
+      Q.lp.push_back(l[0] | (l[1] << 16));
+      Q.lp.push_back(l[2] | (l[3] << 16));
+      Q.lp.push_back((uint32_t)q[0] | ((uint32_t)q[1] << 16) | own);
+      Q.lp.push_back((uint32_t)q[2] | ((uint32_t)q[3] << 16));
+      Q.tet.push_back(t);
+    }
+    Q.ghost.insert(Q.ghost.end(), ghosts.begin(), ghosts.end());
+    Q.own_max = std::max(Q.own_max, p.own_cnt);
+    Q.ghost_max = std::max(Q.ghost_max, p.ghost_cnt);
+    Q.local_max = std::max(Q.local_max, p.own_cnt + p.ghost_cnt);
+    Q.tet_max = std::max(Q.tet_max, p.tet_cnt);
+    Q.slot_max = std::max(Q.slot_max, p.slots + 64);
+    Q.parts.push_back(p);
+  }
+  return true;
+}
+
 }  // namespace pbs

@@ -66,4 +66,33 @@ bool build_batch_plan(int ninst, const int *node_off, const int *tet_off, const 
 bool build_batch_plan(int ninst, const int *node_off, const int *tet_off, const float *rest, const int *tets,
                       int tile_tets, TilePlan &plan, std::string &msg);
 
+// Partition for the resident descent kernel (pbs_persist.hip): one workgroup per part, a part owning
+// a contiguous node run and evaluating every tet that touches an owned node (tets across parts are
+// evaluated by each of them, so that no forces have to be exchanged, only positions).  A part's
+// local nodes are its owned nodes, then the other corners of its tets (ghosts, ascending).  An
+// owned node's contributions form one run, ordered as the tile pass adds them: its own tile's
+// tets, then those of the other tiles in tile order, each tile's in (tet, corner) order; bit j of
+// its mask is set where entry j ends one tile's partial sum.
+struct PersistPart {
+  int own_start, own_cnt;
+  int ghost_off, ghost_cnt;  // ghost[ghost_off ..)
+  int tet_off, tet_cnt;      // tet[tet_off ..), lp likewise
+  int run_off;               // run[run_off .. run_off + own_cnt], mask[run_off ..)
+  int slots;                 // contributions of the owned nodes
+};
+struct PersistPlan {
+  std::vector<PersistPart> parts;
+  std::vector<int> ghost;       // solver node ids
+  std::vector<int> tet;         // solver tet ids
+  std::vector<uint32_t> lp;     // 4 words per entry as TilePlan::tet_lp; corners of ghosts get the slots
+                                // `slots` + (entry & 63), which nothing reads; bit 31 of the third word:
+                                // the part owns the tet's smallest node (it counts the tet's energy)
+  std::vector<uint16_t> run;    // per part own_cnt + 1 run offsets
+  std::vector<uint64_t> mask;   // per entry of run
+  int own_max = 0, local_max = 0, ghost_max = 0, tet_max = 0, slot_max = 0;
+};
+// Builds the partition of a single mesh into at most max_parts parts of about nodes_per_part nodes
+// or more.  Returns false where a node has more than 64 incident tets.
+bool build_persist_plan(const TilePlan &P, int max_parts, int nodes_per_part, PersistPlan &Q);
+
 }  // namespace pbs
