@@ -196,6 +196,7 @@ template <typename R> static int alloc_impl(pbs_solver *s) {
   rc |= dalloc(s, &m.inc_off, N + 1);
   rc |= dalloc(s, &m.inc, 4 * T);
   rc |= dalloc(s, &m.perm, N);
+  rc |= dalloc(s, &m.itperm, T);
   rc |= dalloc(s, &m.mask, N);
   rc |= dalloc(s, &m.mass, N);
   rc |= dalloc(s, &m.mnode, N);
@@ -340,6 +341,7 @@ template <typename R> static int setup_impl(pbs_solver *s, const int *mask) {
     for (size_t i = 0; i < N; ++i) mk[i] = mask[P.perm[i]] ? 1 : 0;
   HIPCHK(hipMemcpyAsync(m.mask, mk.data(), sizeof(int) * N, hipMemcpyHostToDevice, s->st));
   HIPCHK(hipMemcpyAsync(m.perm, P.perm.data(), sizeof(int) * N, hipMemcpyHostToDevice, s->st));
+  HIPCHK(hipMemcpyAsync(m.itperm, P.itperm.data(), sizeof(int) * P.itperm.size(), hipMemcpyHostToDevice, s->st));
   HIPCHK(hipMemcpyAsync(m.inc_off, P.inc_off.data(), sizeof(int) * (N + 1), hipMemcpyHostToDevice, s->st));
   if (s->nt > 0) HIPCHK(hipMemcpyAsync(m.inc, P.inc.data(), sizeof(int) * 4 * (size_t)s->nt, hipMemcpyHostToDevice, s->st));
   HIPCHK(hipMemcpyAsync((void *)s->td.tiles, P.tiles.data(), sizeof(TileInfo) * P.tiles.size(), hipMemcpyHostToDevice, s->st));
@@ -1224,16 +1226,13 @@ extern "C" int pbs_do_descent_opt(pbs_solver *s, float h, int iterations, const 
 }
 
 // ---- material calls ----
-// Per-tet records (width values per tet, solver tet order on the device) -> caller tet order.
-template <typename T> static int download_records(pbs_solver *s, const T *dev, float *host, int width) {
-  const size_t n = (size_t)width * s->nt;
-  std::vector<T> tmp(n);
-  HIPCHK(hipMemcpyAsync(tmp.data(), dev, sizeof(T) * n, hipMemcpyDeviceToHost, s->st));
-  HIPCHK(hipStreamSynchronize(s->st));
-  for (int t = 0; t < s->nt; ++t) {
-    const size_t o = (size_t)width * s->plan.tperm[t];
-    for (int k = 0; k < width; ++k) host[o + k] = (float)tmp[(size_t)width * t + k];
-  }
+// Per-tet records (width values per tet, solver tet order on the device) -> caller tet order, through
+// room for them in FP32 on the device.
+template <typename T>
+static int download_records(pbs_solver *s, const T *dev, const int *itperm, float *room, float *host, int width) {
+  tets_to_caller(dev, room, width, itperm, s->nt, s->st);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(host, room, sizeof(float) * width * (size_t)s->nt, hipMemcpyDeviceToHost, s->st));
   return PBS_OK;
 }
 
@@ -1250,11 +1249,11 @@ template <typename R> static int forces_impl(pbs_solver *s, const float *pos, fl
     if (rc) return rc;
   }
   if (tf && s->nt > 0) {
-    rc = download_records<R>(s, m.frec, tf, 12);
+    rc = download_records<R>(s, m.frec, m.itperm, m.hrec, tf, 12);
     if (rc) return rc;
   }
   if (te && s->nt > 0) {
-    rc = download_records<R>(s, m.tete, te, 1);
+    rc = download_records<R>(s, m.tete, m.itperm, m.hrec, te, 1);
     if (rc) return rc;
   }
   HIPCHK(hipStreamSynchronize(s->st));
@@ -1279,11 +1278,11 @@ template <typename R> static int hd_impl(pbs_solver *s, const float *pos, float 
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(nh, s->stage, sizeof(float) * 3 * (size_t)s->nn, hipMemcpyDeviceToHost, s->st));
   }
-  HIPCHK(hipStreamSynchronize(s->st));
   if (th && s->nt > 0) {
-    rc = download_records<float>(s, m.hrec, th, 12);
+    rc = download_records<float>(s, m.hrec, m.itperm, (float *)m.frec, th, 12);
     if (rc) return rc;
   }
+  HIPCHK(hipStreamSynchronize(s->st));
   return PBS_OK;
 }
 

@@ -85,6 +85,7 @@ template <typename R> struct DevMesh {
   int *inc_off;     // N+1
   int *inc;         // 4T, entry = 4*tet + local, per node in ascending caller tet id
   int *perm;        // N: solver node -> caller node
+  int *itperm;      // T: caller tet -> solver tet
   int *mask;        // N
   float *mass;      // N (fixed nodes: fixed_mass)
   float *mnode;     // N: the computed mass of a free node, -1 for a fixed node (the node pass reads
@@ -180,6 +181,8 @@ void mlp_step(const float *grad_part, const float *loss_part, int nwg, float *gr
               float *params, float *m1, float *m2, unsigned short *wA, float lr, float b1t, float b2t, hipStream_t st);
 
 void aos_to_planes_f(const float *aos, float *planes, const int *perm, int n, hipStream_t st);
+// Per-tet records of 12 or 1 values -> FP32 in the caller's tet order.
+template <typename T> void tets_to_caller(const T *rec, float *out, int width, const int *itperm, int nt, hipStream_t st);
 void planes_to_aos_f(const float *planes, float *aos, const int *perm, int n, hipStream_t st);
 void fill_f(float *p, float v, long n, hipStream_t st);
 

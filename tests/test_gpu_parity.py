@@ -525,3 +525,27 @@ def test_full_size_relgrad_step_judged_by_the_oracle():
     assert abs(g0 - st.g0_norm) <= 1e-6 * g0
     assert abs(g - st.g_norm) <= 1e-6 * g0
     assert g <= 1e-4 * g0
+
+
+@pytest.mark.parametrize("precision", [P.FP32, P.FP64])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (3, 5, 7), (7, 7, 9)])
+def test_material_records_come_in_the_callers_tet_order(dims, precision):
+    """Per-tet forces, energies and stiffness diagonals of a mesh whose tets are numbered at random:
+    each caller tet's record is its own, on meshes below and past one block of records.  The records
+    of a mesh do not depend on how it numbers its tets: each tet is evaluated alone, so those of the
+    ordered mesh, permuted, are equal bit for bit (its nodes keep their order within the tet)."""
+    rest, tets = M.bar(*dims, 0.05)
+    mask = M.clamp_x0(rest)
+    x = M.twisted_state(rest, *dims, 0.05, 40.0, 0.01, 5)
+    order = np.random.default_rng(3).permutation(len(tets))
+    got = []
+    for q in (tets, tets[order]):
+        s = P.Solver(rest, q, mask, P.default_params(precision=precision))
+        tf, _, te = s.compute_forces(x)
+        _, th = s.compute_hessian_diag(x)
+        s.close()
+        got.append((tf, te, th))
+    say("records", dims, precision, len(tets), "tets")
+    for a, b in zip(*got):
+        assert np.array_equal(a[order].view(np.uint32), b.view(np.uint32))
+    assert len(np.unique(got[0][0], axis=0)) > len(tets) // 2  # the records differ from tet to tet
