@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -1156,9 +1157,24 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
     }
     if (all_done()) break;
     if (launched >= cap) return set_error(PBS_ERR_STATE, "descent loop did not terminate within the pass cap");
+    // Passes queued before the next look at the control blocks (those after the end do nothing).  Rel-
+    // grad: a look leaves the device idle for 20 to 30 us, so as many as the gradient's decrease so far
+    // predicts: three quarters of it, never more than were run already, and never past the cap (311 K
+    // tets 44.9 -> 43.2 ms, 614 K 65.4 -> 64.5, 1.5 M 122.0 -> 120.4, 6.3 M +0.3 %).
     n = 1;
-    for (const Ctrl &q : ch)
-      if (!q.done) n = std::max<long>(n, relg ? 32 : std::max(1, q.budget - q.k) + 1);
+    for (const Ctrl &q : ch) {
+      if (q.done) continue;
+      if (!relg) {
+        n = std::max<long>(n, std::max(1, q.budget - q.k) + 1);
+        continue;
+      }
+      long ahead = 32;
+      if (fp64_phase && q.g > 0.0 && q.g < q.g0) {
+        const double left = std::log(q.g / (s->dp.relgrad_tol * q.g0)) / std::log(q.g0 / q.g) * q.passes;
+        if (left > 0) ahead = std::max(ahead, (long)std::min(0.75 * left, (double)std::min(launched, cap - launched)) / 32 * 32);
+      }
+      n = std::max(n, ahead);
+    }
   }
   s->dp.f32math = 0;
   s->pass_ordinal = -1;

@@ -180,9 +180,15 @@ template <typename R> int cg_graph(pbs_solver *s, const IeDev &dev, CgGraphs &G)
 // Solves dev's system from the start vector in dev.x (b, dinv already set): the start kernels,
 // then graph replays until the device-side test stops; with profiling on, the same iterations are
 // launched eagerly instead, each dispatch carrying its own start and end
-// events.  c receives the final control block.
+// events.  c receives the final control block; `expect` iterations are queued before the first look at
+// it (those after the stop do nothing).
+//
+// A look (copy to the host, wait, next launch) leaves the device idle for 20 to 30 us, so replays
+// are queued ahead by what the residual's decrease so far predicts: three quarters of it, and never
+// more than were run already.  1.5 M tets, 470 iterations: 23.0 -> 22.4 ms a step; projective
+// dynamics on 0.7 M tets, 525 iterations in 5 solves: 11.1 -> 10.8 ms.
 template <typename R>
-int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double tol, int maxit, IeCtrl &c) {
+int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double tol, int maxit, int expect, IeCtrl &c) {
   dev.tol2 = tol * tol;
   dev.maxit = maxit;
   const bool timed = s->prof_period > 0;
@@ -190,12 +196,17 @@ int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double to
   if (rc) return rc;
   IeLaunch<R>::start(dev, s->st);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(&c, dev.ctrl, sizeof(IeCtrl), hipMemcpyDeviceToHost, s->st));
-  HIPCHK(hipStreamSynchronize(s->st));
-  long replays = 0;
+  c = IeCtrl{};
+  long replays = 0, ahead = std::max(expect / kGraphIters, 1);
   const long max_replays = (maxit + kGraphIters - 1) / kGraphIters + 1;
   while (!c.done) {
-    if (replays++ >= max_replays) return set_error(PBS_ERR_STATE, "CG loop did not stop within its iteration cap");
+    if (replays >= max_replays) return set_error(PBS_ERR_STATE, "CG loop did not stop within its iteration cap");
+    if (replays > 0) {
+      const double left = std::log(c.rz / (dev.tol2 * c.bb)) / std::log(c.rz0 / c.rz) * c.k;
+      ahead = c.rz < c.rz0 && left > 0 ? (long)std::min(0.75 * left / kGraphIters, (double)replays) : 1;
+    }
+    ahead = timed ? 1 : std::min(std::max(ahead, 1L), max_replays - replays);
+    replays += ahead;
     const int k_before = c.k;
     if (timed) {
       for (int i = 0; i < kGraphIters; ++i) {
@@ -206,7 +217,7 @@ int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double to
       }
       HIPCHK(hipGetLastError());
     } else {
-      HIPCHK(hipGraphLaunch(G.graph, s->st));
+      for (long r = 0; r < ahead; ++r) HIPCHK(hipGraphLaunch(G.graph, s->st));
     }
     HIPCHK(hipMemcpyAsync(&c, dev.ctrl, sizeof(IeCtrl), hipMemcpyDeviceToHost, s->st));
     HIPCHK(hipStreamSynchronize(s->st));
@@ -285,7 +296,7 @@ int implicit_step_impl(pbs_solver *s, const pbs_implicit_params *ip, const float
   HIPCHK(hipGetLastError());
   if (ea) HIPCHK(hipEventRecord(ea[1], s->st));
   IeCtrl c{};
-  rc = cg_solve<R>(s, S, d, S->cg_ie, ip->cg_tolerance, ip->cg_max_iterations, c);
+  rc = cg_solve<R>(s, S, d, S->cg_ie, ip->cg_tolerance, ip->cg_max_iterations, 0, c);
   if (rc) return rc;
   if (ea) {
     float ms = 0.f;
@@ -373,6 +384,7 @@ int pd_step_impl(pbs_solver *s, const pbs_pd_params *pp, const float *ext, float
     if (rc) return rc;
   }
   hipEvent_t *ea = timed ? &S->ev[kIterEvents * kGraphIters] : nullptr;  // events around the local step
+  int last_k = 0;  // iterations of the solve before
   for (int it = 0; it < pp->iterations; ++it) {
     // local step at the current iterate (dev.x), global solve warm-started from it
     if (ea) HIPCHK(hipEventRecord(ea[0], s->st));
@@ -380,8 +392,9 @@ int pd_step_impl(pbs_solver *s, const pbs_pd_params *pp, const float *ext, float
     HIPCHK(hipGetLastError());
     if (ea) HIPCHK(hipEventRecord(ea[1], s->st));
     IeCtrl c{};
-    rc = cg_solve<R>(s, S, d, S->cg_pd, pp->cg_tolerance, pp->cg_max_iterations, c);
+    rc = cg_solve<R>(s, S, d, S->cg_pd, pp->cg_tolerance, pp->cg_max_iterations, last_k, c);
     if (rc) return rc;
+    last_k = c.k;
     if (ea) {  // cg_solve synchronised the stream
       float ms = 0.f;
       if (hipEventElapsedTime(&ms, ea[0], ea[1]) == hipSuccess) {
