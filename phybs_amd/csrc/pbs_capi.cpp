@@ -267,11 +267,12 @@ template <typename R> static int alloc_impl(pbs_solver *s) {
 }
 
 // The resident descent loop (pbs_persist.hip) of a single mesh with the default tile size and graph
-// length: plan, device arrays and exchange buffers, where the mesh fits it.  Parts of at least 32
-// nodes, at most one per CU, at most 168 nodes each (8 waves of 21), so 43,000 nodes at most.  It is
-// the faster path up to there: us per pass, resident against launches, 45 nodes 4.8 : 10.4, 8.6 K
-// nodes 8.2 : 13.6 (FP64 7.1 : 14.2), 21 K nodes 9.8 : 14.0 (8.4 : 15.5), 40 K nodes 9.9 : 15.4
-// (10.6 : 17.9).
+// length: plan, device arrays and exchange buffers, where the mesh fits it.  Parts of at least 21
+// nodes (one wave's; 16 or 12 are no faster, 32 take 6 to 14 % more per pass at 1.5 K tets), at most
+// one per CU, at most 168 nodes each (8 waves of 21), so 43,000 nodes at most.  It is the faster path
+// up to there: us per pass of a step, resident against launches, FP32 96 passes (FP64 rel-grad in
+// brackets): 45 nodes 3.3 : 10.1 (3.1 : 11.4), 425 nodes 3.3 : 12.1 (2.9 : 12.9), 8.6 K nodes 4.5 :
+// 13.5 (3.5 : 13.8), 21 K nodes 6.3 : 14.9 (4.6 : 15.1), 39 K nodes 7.1 : 15.4 (7.8 : 17.2).
 constexpr int kPersistNodes = 40000;
 template <typename R> static int persist_setup(pbs_solver *s) {
   s->persist = PersistDev{};
@@ -279,7 +280,7 @@ template <typename R> static int persist_setup(pbs_solver *s) {
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->device) != hipSuccess) return PBS_OK;
   PersistPlan Q;
-  if (!build_persist_plan(s->plan, std::min(cus, 256), 32, Q)) return PBS_OK;
+  if (!build_persist_plan(s->plan, std::min(cus, 256), 21, Q)) return PBS_OK;
   if (Q.own_max > kPersistOwn || Q.ghost_max > kPersistGhosts || Q.tet_max > kPersistTetsPerThread * kPersistThreads)
     return PBS_OK;
   PersistDev d{};
@@ -290,7 +291,8 @@ template <typename R> static int persist_setup(pbs_solver *s) {
   if (PersistLaunch<R>::lds_bytes(d) + 1024 > s->lds_budget) return PBS_OK;
   if (std::min(PersistLaunch<R>::max_resident(d, 0, s->device), PersistLaunch<R>::max_resident(d, 1, s->device)) < d.nparts)
     return PBS_OK;
-  const size_t xb = (4 * 3 * (size_t)s->nn * sizeof(R) + 15) / 16 * 16, pb = 4 * 2 * (size_t)d.nparts * sizeof(double);
+  const size_t xb = (kPersistSlots * 3 * (size_t)s->nn * sizeof(R) + 15) / 16 * 16,
+               pb = kPersistSlots * 2 * (size_t)d.nparts * sizeof(double);
   PersistPart *parts;
   int *ghost;
   uint32_t *lp;

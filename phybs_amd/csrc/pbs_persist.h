@@ -8,6 +8,7 @@
 namespace pbs {
 
 constexpr int kPersistThreads = 512;
+constexpr int kPersistSlots = 8;                          // exchange slots, used in turn
 constexpr int kPersistTetsPerThread = 4;                  // at most
 constexpr int kPersistOwn = kPersistThreads / 64 * 21;    // owned nodes per workgroup: 21 per wave (3 lanes each)
 constexpr int kPersistGhosts = 4 * kPersistThreads / 3;   // ghosts per workgroup: 4 components per thread
@@ -20,8 +21,8 @@ struct PersistDev {
   const uint4 *lp;
   const unsigned short *run;
   const unsigned long long *mask;
-  void *xch;      // 4 slots of 3N values: positions published after a pass (node-major)
-  double *part;   // 4 slots of (energy, |g|^2) per part
+  void *xch;      // kPersistSlots slots of 3N values: positions published after a pass (node-major)
+  double *part;   // kPersistSlots slots of (energy, |g|^2) per part
   long xch_bytes; // of xch and part together (part follows xch)
   int *abort;     // set by a workgroup that gave up waiting
 };
