@@ -8,6 +8,7 @@
 // -(v1 x v2 + v2 x v3 + v3 x v1)/6 area vectors (TetMesh.cpp:279-294), so it is recomputed in
 // registers instead of being stored.
 #pragma once
+#include <type_traits>
 #include <hip/hip_runtime.h>
 
 namespace pbs {
@@ -74,6 +75,27 @@ template <> __device__ __forceinline__ double drsqrt<double>(double v) { return 
 template <typename R> __device__ __forceinline__ R dsqrt(R v);
 template <> __device__ __forceinline__ float dsqrt<float>(float v) { return sqrtf(v); }
 template <> __device__ __forceinline__ double dsqrt<double>(double v) { return sqrt(v); }
+
+// Sum over the wave, the same in every lane: within the rows of 16 lanes, then across them (DPP: no
+// LDS round trips as a shuffle makes).
+__device__ __forceinline__ double wave_sum(double v) {
+  auto step = [&](auto ctrl, auto rows) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
+    v += __builtin_bit_cast(double, (unsigned long long)(unsigned)hi << 32 | (unsigned)lo);
+  };
+  typedef std::integral_constant<int, 0xf> All;
+  step(std::integral_constant<int, 0x111>(), All());  // row_shr:1, 2, 4, 8
+  step(std::integral_constant<int, 0x112>(), All());
+  step(std::integral_constant<int, 0x114>(), All());
+  step(std::integral_constant<int, 0x118>(), All());
+  step(std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());  // row_bcast:15
+  step(std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());  // row_bcast:31
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __builtin_bit_cast(double, (unsigned long long)(unsigned)hi << 32 | (unsigned)lo);
+}
 
 // Adjugate of A (row-major) and det(A) expanded down column 0 (cuMath::Matrix_Inverse_3).
 template <typename R> __device__ __forceinline__ R adj3(const R *A, R *C) {

@@ -47,6 +47,89 @@ template <typename T> int ialloc(ImplicitState *S, T **p, size_t n) {
   return PBS_OK;
 }
 
+// The resident solver's partition: workgroup g owns vector blocks [g per_part, (g + 1) per_part), their
+// slices and rows; the columns it does not own are its ghosts, ascending.  False where the system has
+// more slices than 256 workgroups of 8 waves hold (131,072 rows), wider rows than the registers, or a
+// workgroup more ghosts than its threads read at once.
+bool cg_partition(const ImplicitState &S, const IeDev &d, CgDev &c, std::vector<int> &ghost_off, std::vector<int> &ghost,
+                  std::vector<uint16_t> &lcol) {
+  const int N = d.n;
+  if (S.nslice == 0 || S.nslice > kCgSlices || S.max_width > kCgWidth) return false;
+  c.per_part = d.vec_blocks > 256 ? 2 : 1;
+  c.nparts = (d.vec_blocks + c.per_part - 1) / c.per_part;
+  lcol.assign(S.slots, 0);
+  ghost_off.assign(1, 0);
+  ghost.clear();
+  std::vector<int> local(N, -1), seen;
+  auto first_slice = [&](int b) { return b * d.vec_per + std::min(b, d.vec_rem); };
+  for (int g = 0; g < c.nparts; ++g) {
+    const int s0 = first_slice(g * c.per_part), s1 = first_slice(std::min((g + 1) * c.per_part, d.vec_blocks));
+    const int n0 = 64 * s0, n1 = std::min(N, 64 * s1);
+    c.shares = std::max(c.shares, s1 - s0 <= 2 ? 1 : s1 - s0 <= 4 ? 2 : 4);
+    seen.clear();
+    for (int n = n0; n < n1; ++n) {
+      const long at = S.slice_off_h[n >> 6];
+      for (int j = 0; j < S.row_len_h[n]; ++j) {
+        const int m = S.bcol_h[(at + j) * 64 + (n & 63)];
+        if ((m < n0 || m >= n1) && local[m] < 0) {
+          local[m] = 0;
+          seen.push_back(m);
+        }
+      }
+    }
+    if (seen.size() > (size_t)kCgGhosts) return false;
+    std::sort(seen.begin(), seen.end());
+    for (size_t k = 0; k < seen.size(); ++k) local[seen[k]] = n1 - n0 + (int)k;
+    for (int sl = s0; sl < s1; ++sl)
+      for (long at = 64L * S.slice_off_h[sl]; at < 64L * S.slice_off_h[sl + 1]; ++at) {
+        const int m = S.bcol_h[at];  // (a row's padding: its own column; past the last row: any of its own)
+        lcol[at] = m >= n0 && m < n1 ? (uint16_t)(m - n0) : local[m] >= 0 ? (uint16_t)local[m] : 0;
+      }
+    for (int m : seen) local[m] = -1;
+    ghost.insert(ghost.end(), seen.begin(), seen.end());
+    ghost_off.push_back((int)ghost.size());
+    c.local_max = std::max(c.local_max, n1 - n0 + (int)seen.size());
+  }
+  return true;
+}
+
+// Uploads it with its exchange buffers; without it (or where the device cannot hold it) the vector
+// passes are split for the launches alone.
+template <typename R> int cg_setup(pbs_solver *s, ImplicitState *S) {
+  IeDev &d = S->dev;
+  ie_vec_split(d, true);
+  CgDev c{};
+  std::vector<int> goff, ghost;
+  std::vector<uint16_t> lcol;
+  if (cg_partition(*S, d, c, goff, ghost, lcol))
+    for (int scalar = 0; scalar < 2; ++scalar) S->cg_fits[scalar] = IeLaunch<R>::resident_fits(c, scalar, s->device);
+  if (!S->cg_fits[0] && !S->cg_fits[1]) {
+    ie_vec_split(d, false);
+    return PBS_OK;
+  }
+  int *go, *gh, *abort;
+  unsigned short *lc;
+  const size_t nz = 2 * 3 * (size_t)d.n, nx = (nz + 4 * (size_t)d.vec_blocks + 1) & ~(size_t)1;
+  int rc = ialloc(S, &go, goff.size());
+  if (!rc) rc = ialloc(S, &gh, ghost.size());
+  if (!rc) rc = ialloc(S, &lc, lcol.size());
+  if (!rc) rc = ialloc(S, &abort, 1);
+  if (!rc) rc = ialloc(S, &c.z, nx);
+  if (rc) return rc;
+  HIPCHK(hipMemcpy(go, goff.data(), sizeof(int) * goff.size(), hipMemcpyHostToDevice));
+  if (!ghost.empty()) HIPCHK(hipMemcpy(gh, ghost.data(), sizeof(int) * ghost.size(), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(lc, lcol.data(), sizeof(uint16_t) * lcol.size(), hipMemcpyHostToDevice));
+  c.ghost_off = go;
+  c.ghost = gh;
+  c.lcol = lc;
+  c.abort = abort;
+  c.pap = c.z + nz;
+  c.rz = c.pap + 2 * (size_t)d.vec_blocks;
+  c.xch_bytes = (long)(sizeof(double) * nx);
+  S->cg = c;
+  return PBS_OK;
+}
+
 // Block rows of K in solver order: a node's columns are the nodes sharing a tet with it,
 // ascending, itself included (the block pattern of allocateGlobalStiffnessMatrix,
 // IsotropicMaterial.cpp:554-644), laid out as SELL-64.
@@ -104,7 +187,6 @@ int implicit_get(pbs_solver *s, ImplicitState **out) {
   IeDev &d = S->dev;
   d.n = N;
   d.nslice = S->nslice;
-  ie_vec_split(d);
   int *so = nullptr, *rl = nullptr, *bc = nullptr, *dsl = nullptr;
   char *A = nullptr;
   int rc = ialloc(S, &so, S->nslice + 1);
@@ -133,6 +215,11 @@ int implicit_get(pbs_solver *s, ImplicitState **out) {
   if (e != hipSuccess) {
     implicit_release(S);
     return set_error(PBS_ERR_HIP, std::string("backward-Euler setup: ") + hipGetErrorString(e));
+  }
+  rc = s->p.precision == PBS_FP64 ? cg_setup<double>(s, S) : cg_setup<float>(s, S);
+  if (rc) {
+    implicit_release(S);
+    return rc;
   }
   s->implicit = S;
   *out = S;
@@ -192,11 +279,25 @@ int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double to
   dev.tol2 = tol * tol;
   dev.maxit = maxit;
   const bool timed = s->prof_period > 0;
-  int rc = timed ? cg_events(S) : cg_graph<R>(s, dev, G);
-  if (rc) return rc;
   IeLaunch<R>::start(dev, s->st);
   HIPCHK(hipGetLastError());
   c = IeCtrl{};
+  if (S->cg_fits[dev.scalar] && !timed) {
+    hipError_t e = IeLaunch<R>::resident(dev, S->cg, s->st);
+    int gave_up = 1;
+    if (e == hipSuccess) {
+      HIPCHK(hipMemcpyAsync(&c, dev.ctrl, sizeof(IeCtrl), hipMemcpyDeviceToHost, s->st));
+      HIPCHK(hipMemcpyAsync(&gave_up, S->cg.abort, sizeof(int), hipMemcpyDeviceToHost, s->st));
+      HIPCHK(hipStreamSynchronize(s->st));
+    }
+    if (gave_up) {  // not launchable, or its workgroups did not all run: the launches, from the same start
+      (void)hipGetLastError();
+      S->cg_fits[0] = S->cg_fits[1] = false;
+      c = IeCtrl{};
+    }
+  }
+  int rc = c.done ? PBS_OK : timed ? cg_events(S) : cg_graph<R>(s, dev, G);
+  if (rc) return rc;
   long replays = 0, ahead = std::max(expect / kGraphIters, 1);
   const long max_replays = (maxit + kGraphIters - 1) / kGraphIters + 1;
   while (!c.done) {

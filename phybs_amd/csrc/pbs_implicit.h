@@ -22,7 +22,8 @@ struct IeCtrl {
 
 struct IeDev {
   int n, nslice, maxit, scalar;    // scalar: one value per slot (block = value x identity)
-  int vec_per, vec_rem;            // vector passes: groups of 64 entries per block, blocks with one more
+  // vector passes: entries per group (64, or a slice's 192), groups per block, blocks with one more
+  int vec_unit, vec_per, vec_rem, vec_blocks;
   double tol2;                     // (relative residual tolerance)^2
   const int *slice_off;            // nslice + 1, in slot groups of 64
   const int *row_len;              // N
@@ -42,7 +43,25 @@ struct IeAsm {
   int has_ext;
 };
 
-void ie_vec_split(IeDev &d);  // sets vec_per, vec_rem from n
+// Sets the split of the vector passes: whole slices per block (at most 4), as the resident solver's
+// workgroups own them, or blocks of at least 1024 entries.
+void ie_vec_split(IeDev &d, bool slices);
+
+// The resident CG (k_cg): partition and exchange buffers.  A workgroup owns one or two of the vector
+// passes' blocks and their slices' rows.
+constexpr int kCgThreads = 512;
+// at most: slices, slots of a slice, ghosts of a workgroup
+constexpr int kCgSlices = 2048, kCgWidth = 28, kCgGhosts = 8 * kCgThreads / 3;
+struct CgDev {
+  int nparts, per_part;           // workgroups (0: not used), vector blocks of each
+  int shares;                     // shares of a slice that one wave multiplies (1, 2 or 4)
+  int local_max;                  // rows and ghosts of a workgroup, at most
+  const int *ghost_off, *ghost;   // per workgroup: node ids of the columns it does not own
+  const unsigned short *lcol;     // per slot: local column (own rows, then ghosts)
+  double *z, *pap, *rz;           // 2 slots each: 3N values; partials per vector block
+  long xch_bytes;                 // of the three together (z first)
+  int *abort;                     // set by a workgroup that gave up waiting
+};
 
 template <typename R> struct IeLaunch {
   // max_width: the widest slice (slots per row)
@@ -57,6 +76,9 @@ template <typename R> struct IeLaunch {
   static void dir(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
   static void spmv(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
   static void res(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+  // the whole loop after `start` as one cooperative launch; whether the device can hold it
+  static hipError_t resident(const IeDev &d, const CgDev &c, hipStream_t st);
+  static bool resident_fits(const CgDev &c, int scalar, int device);
   static void finish(const DevMesh<R> &m, const DevParams &p, float h, const IeDev &d, hipStream_t st);
   // projective dynamics: global matrix, momentum term + iterate start, local step, velocity update
   static void pd_matrix(const DevMesh<R> &m, const DevParams &p, float stiffness, const IeDev &d, hipStream_t st);
@@ -89,6 +111,8 @@ struct ImplicitState {
   int *pd_inc_pos = nullptr;                        // projective dynamics: incidence slot of each (tet, corner)
   std::vector<int> slice_off_h, row_len_h, bcol_h;  // host copies (stiffness export)
   CgGraphs cg_ie, cg_pd;
+  CgDev cg{};                                       // resident solver
+  bool cg_fits[2] = {false, false};                 // for 3x3 blocks; for scalar values
   std::vector<hipEvent_t> ev;                       // timing events of the timed replays
   std::vector<void *> allocs;
 };

@@ -13,6 +13,7 @@
 #include <hip/hip_ext.h>
 
 #include "pbs_device.h"
+#include "pbs_exchange.h"
 #include "pbs_implicit.h"
 
 namespace pbs {
@@ -37,8 +38,7 @@ __device__ __forceinline__ int xcd_block(int bid, int nblk) {
 
 // Sum of v over the 256 threads of the block in a fixed order (wave tree, then the 4 waves).
 __device__ __forceinline__ double block_sum256(double v, double *lds) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  v = wave_sum(v);
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) lds[w] = v;
   __syncthreads();
@@ -70,8 +70,7 @@ template <int NT> struct PartialSum {
       if (base >= nb) break;
       load(v, nb, base);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
+    a = wave_sum(a);
     if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = a;
     __syncthreads();
     double r = 0.0;
@@ -80,6 +79,27 @@ template <int NT> struct PartialSum {
     return r;
   }
 };
+
+// The partials of p.Ap (one per slice) as PartialSum takes them: where the vector passes' blocks are
+// whole slices, each block's slices are added first (at most 4 each, 512 blocks).
+__device__ __forceinline__ int first_slice(const IeDev &d, int b) { return b * d.vec_per + min(b, d.vec_rem); }
+__device__ __forceinline__ void load_pap(const IeDev &d, PartialSum<256> &part) {
+  if (d.vec_unit != 192) {
+    part.load(d.part_pap, d.nslice);
+    return;
+  }
+  double v[2][4];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int b = min(u * 256 + (int)threadIdx.x, d.vec_blocks - 1), s = first_slice(d, b), n = first_slice(d, b + 1) - s;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[u][i] = i < n ? d.part_pap[s + i] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < 2; ++u) part.t[u] = ((v[u][0] + v[u][1]) + v[u][2]) + v[u][3];
+#pragma unroll
+  for (int u = 2; u < 8; ++u) part.t[u] = 0.0;
+}
 
 // y += (row `lane` of the slice's A) v over the slots first, first + step, ... below the slice's
 // width.  BLK = 3: 3x3 blocks (9 values per slot); BLK = 1: one value per slot, the block being
@@ -428,11 +448,10 @@ __global__ void k_tet_stiffness(DevParams p, int num, const int *__restrict__ id
 // XCD-contiguous as the SpMV's rows.
 constexpr int kVecBlocks = 512;
 constexpr int kVec = 4;  // entries a thread has in flight
-inline int vec_blocks(int n) { return (int)std::min<long>((3 * (long)n + kVec * kBlock - 1) / (kVec * kBlock), kVecBlocks); }
 __device__ __forceinline__ void vec_range(const IeDev &d, int &i0, int &i1) {
   const int b = xcd_block(blockIdx.x, gridDim.x);
-  i0 = 64 * (b * d.vec_per + min(b, d.vec_rem));
-  i1 = min(i0 + 64 * (d.vec_per + (b < d.vec_rem ? 1 : 0)), 3 * d.n);
+  i0 = d.vec_unit * (b * d.vec_per + min(b, d.vec_rem));
+  i1 = min(i0 + d.vec_unit * (d.vec_per + (b < d.vec_rem ? 1 : 0)), 3 * d.n);
 }
 // The thread's kVec entries of v from i on, kBlock apart (past the end: the range's last).
 __device__ __forceinline__ void vec_load(const double *__restrict__ v, int i, int i1, double (&t)[kVec]) {
@@ -568,21 +587,21 @@ template <typename R, int BLK> __global__ void __launch_bounds__(kBlock) k_ie_sp
 }
 
 // alpha = r.z / p.Ap, z -= alpha D^-1 Ap; partial r.z.
-__global__ void __launch_bounds__(kBlock) k_ie_res(IeDev d, int nb) {
+__global__ void __launch_bounds__(kBlock) k_ie_res(IeDev d) {
   __shared__ double lds[4];
   int i0, i1;
   vec_range(d, i0, i1);
   int i = i0 + threadIdx.x;
   double *__restrict__ z = d.z;
   PartialSum<kBlock> part;
-  part.load(d.part_pap, nb);
+  load_pap(d, part);
   const IeCtrl in = d.ctrl[1];
   double zv[kVec], av[kVec], dv[kVec];
   vec_load(z, i, i1, zv);
   vec_load(d.Ap, i, i1, av);
   vec_load(d.dinv, i, i1, dv);
   __builtin_amdgcn_sched_barrier(0);  // all of them requested before the first is used
-  const double pap = part.sum(d.part_pap, nb, lds);
+  const double pap = part.sum(d.part_pap, d.vec_unit == 192 ? d.vec_blocks : d.nslice, lds);
   // not positive definite (or a non-finite value): stop without a step
   const bool indefinite = !in.done && !(pap > 0.0), go = !in.done && !indefinite;
   const double alpha = go ? in.rz / pap : indefinite ? 0.0 : in.alpha;
@@ -600,7 +619,7 @@ __global__ void __launch_bounds__(kBlock) k_ie_res(IeDev d, int nb) {
       if (i + u * kBlock < i1) {
         const double zi = zv[u] - dv[u] * (alpha * av[u]);
         z[i + u * kBlock] = zi;
-        rz += zi * zi / dv[u];
+        rz += zi * zi * (1.0 / dv[u]);
       }
     i += kVec * kBlock;
     if (i - (int)threadIdx.x >= i1) break;
@@ -611,6 +630,262 @@ __global__ void __launch_bounds__(kBlock) k_ie_res(IeDev d, int nb) {
   __syncthreads();  // part.sum's slots are read
   rz = block_sum256(rz, lds);
   if (threadIdx.x == 0) d.part_rz[xcd_block(blockIdx.x, gridDim.x)] = rz;
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same iterations as one resident kernel, for systems whose launches cost more than their work.
+// A workgroup owns one or two blocks of the vector passes, that is 1 to 8 slices; its entries of x, p,
+// z and D^-1 stay in registers, and so does its part of the matrix; the directions that its rows
+// touch are in LDS.  An iteration waits for the other workgroups twice (pbs_exchange.h): for the
+// partials of p.Ap, and for those of r.z together with the neighbours' z, from which each workgroup
+// forms the neighbours' new directions itself.  All sums are formed as the three launches form them,
+// term by term, so iterates and counts are bitwise theirs.
+//
+// Bound: the two waits, 5,000 to 8,000 cycles each (a store and a read through the memory side, and
+// the slowest workgroup), of 15,000 to 25,000 an iteration; launches took 11 to 18 us an iteration.
+// A step, launches -> resident, backward Euler (projective dynamics in brackets), FP32: 20 K tets 3.3
+// -> 2.0 ms (2.3 -> 1.6), 99 K 5.3 -> 3.8 (4.7 -> 3.5), 338 K 7.6 -> 6.5 (7.1 -> 5.8), 729 K (9.3 ->
+// 7.0).  With the matrix read from memory in every iteration, by 8 waves per CU, backward Euler on
+// 729 K tets took 24 ms instead of 11: hence registers, and the launches where they do not suffice.
+//
+// Slots.  Each exchange has 2, iteration k uses slot k mod 2.  A workgroup that has all partials of
+// r.z of iteration k knows that those of p.Ap of k have been consumed, with all of p.Ap of k + 1 that
+// z and r.z of k have been, and clears its own.  Both clearings are waited for before it publishes
+// the next r.z, and a slot is polled again only by who has that one, or the p.Ap that follows it.
+// ---------------------------------------------------------------------------------------------
+__global__ void k_cg_fill(uint4 *__restrict__ p, long n, int *__restrict__ abort) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  if (i == 0) *abort = 0;
+}
+
+// The first four waves: sum of nb <= 512 published partials, as PartialSum<256> adds them, of which
+// they leave 4 terms in total, to be added in order after a barrier.
+__device__ __forceinline__ void published_sum(const double *v, int nb, double *total, int *abort, int *gave_up) {
+  const int tid = threadIdx.x;
+  if (tid >= 256) return;
+  unsigned long long t[2];
+  int spin = 0;
+  while (true) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) t[u] = u * 256 + tid < nb ? poll(v + u * 256 + tid) : 0;
+    if (t[0] != Bits<double>::none && t[1] != Bits<double>::none) break;
+    if (give_up(spin, abort)) {
+      *gave_up = 1;
+      break;
+    }
+  }
+  double a = 0.0;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) a += u * 256 + tid < nb ? __builtin_bit_cast(double, t[u]) : 0.0;
+  a = wave_sum(a);
+  if ((tid & 63) == 0) total[tid >> 6] = a;
+}
+
+// SH: shares of a slice per wave (a slice has four; 8 / (4 / SH) slices per workgroup at most).
+template <typename R, int BLK, int SH> __global__ void __launch_bounds__(kCgThreads) k_cg(IeDev d, CgDev c) {
+  extern __shared__ double lp[];         // directions of the local rows, x y z of each
+  __shared__ double share[2 * SH][4][3][64];  // Ap of each slice in four shares
+  __shared__ double csum[8][3], zsum[2][4], tot[2][4];
+  __shared__ int gave_up;
+  constexpr int NU = 3, GH = kCgGhosts * 3 / kCgThreads, WS = 4 / SH, NJ = kCgWidth / 4, NV = BLK * BLK;
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const int g = xcd_block(blockIdx.x, c.nparts);
+  IeCtrl in = d.ctrl[0];
+  if (in.done) return;
+  if (tid == 0) gave_up = 0;
+  const int vb0 = g * c.per_part, vb1 = min(vb0 + c.per_part, d.vec_blocks);
+  const int s0 = first_slice(d, vb0), nsl = first_slice(d, vb1) - s0;
+  const int n0 = 64 * s0, own = min(64 * nsl, d.n - n0);
+  // this thread's vector entries: wave w holds chunks w % 4, + 4, + 8 (of 64 entries) of its block
+  const int vb = vb0 + (w >> 2), q = w & 3;
+  const int vs = vb < vb1 ? first_slice(d, vb) : 0, vn = vb < vb1 ? 3 * (first_slice(d, vb + 1) - vs) : 0;
+  int ei[NU];
+  double x[NU], p[NU], z[NU], di[NU], ri[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int ch = q + 4 * u, i = 192 * vs + 64 * ch + lane;
+    ei[u] = ch < vn && i < 3 * d.n ? i : -1;
+    const int k = ei[u] < 0 ? 0 : i;
+    x[u] = d.x[k];
+    z[u] = d.z[k];
+    di[u] = d.dinv[k];
+    ri[u] = 1.0 / di[u];
+    p[u] = 0.0;
+  }
+  // ghost components: entry, z, direction
+  const int goff = c.ghost_off[g], gcnt = c.ghost_off[g + 1] - goff;
+  int gi[GH];
+  double gz[GH], gp[GH];
+#pragma unroll
+  for (int u = 0; u < GH; ++u) {
+    const int e = tid + u * kCgThreads;
+    gi[u] = e < 3 * gcnt ? 3 * c.ghost[goff + e / 3] + e % 3 : -1;
+    gz[u] = gi[u] >= 0 ? d.z[gi[u]] : 0.0;
+    gp[u] = 0.0;
+  }
+  // the product: WS waves per slice; this wave's shares of its slice in registers
+  const int sl = w / WS, sub = w % WS;
+  const bool mul = sl < nsl;
+  const int g0 = mul ? d.slice_off[s0 + sl] : 0, width = mul ? d.slice_off[s0 + sl + 1] - g0 : 0;
+  const R *__restrict__ A = (const R *)d.A;
+  R av[SH][NJ][NV];
+  int ac[SH][NJ];
+#pragma unroll
+  for (int h = 0; h < SH; ++h)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const int jj = sub + WS * h + 4 * j;
+      if (jj < width) {
+        ac[h][j] = 3 * (int)c.lcol[(size_t)(g0 + jj) * 64 + lane];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) av[h][j][v] = BLK == 3 ? A[val_idx(g0 + jj, v, lane)] : A[(size_t)(g0 + jj) * 64 + lane];
+      }
+    }
+  const bool row = mul && 64 * (s0 + sl) + lane < d.n;
+  double rz = in.rz, alpha = in.alpha, beta = in.beta, pap = in.pAp;
+  int k = in.k, converged = in.converged, indefinite = 0;
+  __syncthreads();
+  for (int it = 0;; ++it) {
+    const int slot = it & 1;
+    double *pz = c.z + (size_t)slot * 3 * d.n;
+    // as k_ie_dir
+    if (it > 0) {
+      double sum = 0.0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum += tot[1][i];
+      beta = sum / rz;
+      rz = sum;
+      converged = rz <= d.tol2 * in.bb;
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      if (it > 0) x[u] = x[u] + alpha * p[u];
+      p[u] = it > 0 ? z[u] + beta * p[u] : z[u];
+      if (ei[u] >= 0) lp[ei[u] - 3 * n0] = p[u];
+    }
+    if (converged || k >= d.maxit) break;
+#pragma unroll
+    for (int u = 0; u < GH; ++u) {
+      gp[u] = it > 0 ? gz[u] + beta * gp[u] : gz[u];
+      if (gi[u] >= 0) lp[3 * own + tid + u * kCgThreads] = gp[u];
+    }
+    __syncthreads();
+    // as k_ie_spmv
+#pragma unroll
+    for (int h = 0; h < SH; ++h) {
+      double y[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (sub + WS * h + 4 * j < width) {
+          const double *v = lp + ac[h][j];
+          const double x0 = v[0], x1 = v[1], x2 = v[2];
+          // (FP32 values stay so: converted here, not once before the loop into twice the registers)
+          if constexpr (sizeof(R) == 4) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(av[h][j][i]));
+          }
+          if (BLK == 3) {
+#pragma unroll
+            for (int r = 0; r < 3; ++r)
+              y[r] += (double)av[h][j][3 * r] * x0 + (double)av[h][j][3 * r + 1] * x1 + (double)av[h][j][3 * r + 2] * x2;
+          } else {
+            const double a = (double)av[h][j][0];
+            y[0] += a * x0;
+            y[1] += a * x1;
+            y[2] += a * x2;
+          }
+        }
+      if (mul) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r) share[sl][sub + WS * h][r][lane] = row ? y[r] : 0.0;
+      }
+    }
+    __syncthreads();
+    double ap[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int ch = q + 4 * u;
+      if (ch >= vn) continue;
+      const int s = vs - s0 + ch / 3, e = 64 * (ch % 3) + lane, rw = e / 3, r = e % 3;
+      ap[u] = ((share[s][0][r][rw] + share[s][1][r][rw]) + share[s][2][r][rw]) + share[s][3][r][rw];
+      const double t = wave_sum(ei[u] >= 0 ? p[u] * ap[u] : 0.0);
+      if (lane == 0) csum[s][ch % 3] = t;
+    }
+    __syncthreads();
+    if (tid < vb1 - vb0) {
+      const int a = first_slice(d, vb0 + tid) - s0, n = first_slice(d, vb0 + tid + 1) - s0 - a;
+      double v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = i < n ? (csum[a + i][0] + csum[a + i][1]) + (csum[a + i][2] + 0.0) : 0.0;
+      publish(c.pap + (size_t)slot * d.vec_blocks + vb0 + tid, ((v[0] + v[1]) + v[2]) + v[3]);
+    }
+    published_sum(c.pap + (size_t)slot * d.vec_blocks, d.vec_blocks, tot[0], c.abort, &gave_up);
+    __syncthreads();
+    if (gave_up) break;
+    if (it > 0) {
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+        if (ei[u] >= 0) clear(c.z + (size_t)(slot ^ 1) * 3 * d.n + ei[u]);
+      if (tid < vb1 - vb0) clear(c.rz + (size_t)(slot ^ 1) * d.vec_blocks + vb0 + tid);
+    }
+    // as k_ie_res
+    {
+      double sum = 0.0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum += tot[0][i];
+      indefinite = !(sum > 0.0);
+      alpha = indefinite ? 0.0 : rz / sum;
+      if (indefinite) break;
+      pap = sum;
+      ++k;
+    }
+    double zz = 0.0;
+#pragma unroll
+    for (int u = 0; u < NU; ++u)
+      if (ei[u] >= 0) {
+        const double zi = z[u] - di[u] * (alpha * ap[u]);
+        z[u] = zi;
+        publish(pz + ei[u], zi);
+        zz += zi * zi * ri[u];
+      }
+    zz = wave_sum(zz);
+    if (lane == 0) zsum[w >> 2][q] = zz;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // clearings are complete
+    __syncthreads();
+    if (tid < vb1 - vb0)
+      publish(c.rz + (size_t)slot * d.vec_blocks + vb0 + tid, (zsum[tid][0] + zsum[tid][1]) + (zsum[tid][2] + zsum[tid][3]));
+    published_sum(c.rz + (size_t)slot * d.vec_blocks, d.vec_blocks, tot[1], c.abort, &gave_up);
+    {
+      unsigned long long t[GH];
+      int spin = 0;
+      while (true) {
+        bool wait = false;
+#pragma unroll
+        for (int u = 0; u < GH; ++u) t[u] = gi[u] >= 0 ? poll(pz + gi[u]) : 0;
+#pragma unroll
+        for (int u = 0; u < GH; ++u) wait = wait || t[u] == Bits<double>::none;
+        if (!wait) break;
+        if (give_up(spin, c.abort)) {
+          gave_up = 1;
+          break;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < GH; ++u) gz[u] = __builtin_bit_cast(double, t[u]);
+    }
+    __syncthreads();
+    if (gave_up) break;
+    if (tid < vb1 - vb0) clear(c.pap + (size_t)slot * d.vec_blocks + vb0 + tid);
+  }
+  if (gave_up) {
+    if (tid == 0) __hip_atomic_store(c.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < NU; ++u)
+    if (ei[u] >= 0) d.x[ei[u]] = x[u];
+  if (blockIdx.x == 0 && tid == 0) d.ctrl[0] = {rz, pap, alpha, beta, in.bb, in.rz0, k, 1, converged, indefinite};
 }
 
 // v = solution, x += h v for every node (cublasSaxpy in doBackEuler, CUDAInterface.cu:873).
@@ -838,10 +1113,13 @@ template <typename R> void IeLaunch<R>::start(const IeDev &d, hipStream_t st) {
   hipLaunchKernelGGL(k_ie_start_ctrl, dim3(1), dim3(1024), 0, st, d, nb_of(d.n));
 }
 
-void ie_vec_split(IeDev &d) {
-  const int groups = (3 * d.n + 63) / 64, nblk = vec_blocks(d.n);
-  d.vec_per = groups / nblk;
-  d.vec_rem = groups % nblk;
+void ie_vec_split(IeDev &d, bool slices) {
+  d.vec_unit = slices ? 192 : 64;
+  const int groups = slices ? d.nslice : (3 * d.n + 63) / 64;
+  const long most = slices ? d.nslice : (3 * (long)d.n + kVec * kBlock - 1) / (kVec * kBlock);
+  d.vec_blocks = (int)std::min<long>(most, kVecBlocks);
+  d.vec_per = groups / d.vec_blocks;
+  d.vec_rem = groups % d.vec_blocks;
 }
 
 // e0 set: the launch records the dispatch's start and end in e0, e1 (as a kernel trace times it)
@@ -851,14 +1129,48 @@ static void ie_launch(F kernel, dim3 grid, dim3 block, hipStream_t st, hipEvent_
   else hipLaunchKernelGGL(kernel, grid, block, 0, st, args...);
 }
 template <typename R> void IeLaunch<R>::dir(const IeDev &d, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  ie_launch(k_ie_dir, dim3(vec_blocks(d.n)), dim3(kBlock), st, e0, e1, d);
+  ie_launch(k_ie_dir, dim3(d.vec_blocks), dim3(kBlock), st, e0, e1, d);
 }
 template <typename R> void IeLaunch<R>::spmv(const IeDev &d, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
   if (d.scalar) ie_launch(k_ie_spmv<R, 1>, dim3(d.nslice), dim3(kBlock), st, e0, e1, d);
   else ie_launch(k_ie_spmv<R, 3>, dim3(d.nslice), dim3(kBlock), st, e0, e1, d);
 }
 template <typename R> void IeLaunch<R>::res(const IeDev &d, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  ie_launch(k_ie_res, dim3(vec_blocks(d.n)), dim3(kBlock), st, e0, e1, d, d.nslice);
+  ie_launch(k_ie_res, dim3(d.vec_blocks), dim3(kBlock), st, e0, e1, d);
+}
+
+template <typename R, int BLK> static const void *cg_kernel_of(int shares) {
+  return shares == 1 ? (const void *)k_cg<R, BLK, 1> : shares == 2 ? (const void *)k_cg<R, BLK, 2> : (const void *)k_cg<R, BLK, 4>;
+}
+template <typename R> static const void *cg_kernel(const CgDev &c, int scalar) {
+  // (the 3 x 3 blocks are held for as many shares as the registers take, see resident_fits)
+  if (scalar) return cg_kernel_of<R, 1>(c.shares);
+  return c.shares == 1 ? (const void *)k_cg<R, 3, 1> : (const void *)k_cg<R, 3, 2>;
+}
+static size_t cg_lds(const CgDev &c) { return sizeof(double) * 3 * (size_t)c.local_max; }
+template <typename R> bool IeLaunch<R>::resident_fits(const CgDev &c, int scalar, int device) {
+  // at most 126 registers of matrix values (7 slots of 9 values per share): FP32 up to two shares,
+  // about 65,000 nodes, FP64 one, about 32,000; scalar values always
+  if (!scalar && c.shares * (int)sizeof(R) > 8) return false;
+  int coop = 0, cus = 0;
+  if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess || !coop) return false;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus < c.nparts) return false;
+  int per = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, cg_kernel<R>(c, scalar), kCgThreads, cg_lds(c)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return per > 0;
+}
+template <typename R> hipError_t IeLaunch<R>::resident(const IeDev &d, const CgDev &c, hipStream_t st) {
+  const long n16 = c.xch_bytes / 16;
+  hipLaunchKernelGGL(k_cg_fill, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, (uint4 *)c.z, n16, c.abort);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  IeDev dd = d;
+  CgDev cc = c;
+  void *args[] = {&dd, &cc};
+  return hipLaunchCooperativeKernel(cg_kernel<R>(c, d.scalar), dim3(c.nparts), dim3(kCgThreads), args, (unsigned)cg_lds(c), st);
 }
 
 template <typename R>

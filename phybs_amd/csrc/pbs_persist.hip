@@ -7,10 +7,7 @@
 // nodes, and exchanges only positions and the pass's two sums with the other workgroups.  Every
 // workgroup then takes the loop's decision itself, from the same sums added in the same order.
 //
-// Exchange.  Values cross workgroups as relaxed atomics at agent scope (8 or 4 bytes each, written
-// through to and read from the point where all XCDs see them), and they are their own flags: a slot
-// holds all-ones bits until its owner has written it, a reader polls until it does not (a computed
-// value with that bit pattern, a NaN, is replaced by another NaN).
+// Values cross the workgroups as pbs_exchange.h says.
 //
 // Decisions.  Only a check pass can roll back, and only its sums are waited for at once.  On other
 // passes the control goes on as if not converged; the sums are read during the next pass, while the
@@ -38,6 +35,7 @@
 // groups and order); the energy and |g|^2 are FP64 sums in another fixed order.
 #include <algorithm>
 
+#include "pbs_exchange.h"
 #include "pbs_pass.h"
 #include "pbs_persist.h"
 
@@ -46,56 +44,6 @@ namespace {
 
 constexpr int T = kPersistThreads, NW = T / 64;
 constexpr int CW = NW - 1;  // the wave that runs the loop's control: the last to have tets or nodes
-constexpr int kSpin = 1 << 20;  // polls before giving up (about a second)
-
-template <typename R> struct Bits;
-template <> struct Bits<double> {
-  typedef unsigned long long type;
-  static constexpr type none = ~0ULL, nan = 0x7ff8000000000000ULL;
-};
-template <> struct Bits<float> {
-  typedef unsigned type;
-  static constexpr type none = ~0U, nan = 0x7fc00000U;
-};
-template <typename R> __device__ __forceinline__ void publish(R *p, R v) {
-  typedef typename Bits<R>::type B;
-  B b = __builtin_bit_cast(B, v);
-  if (b == Bits<R>::none) b = Bits<R>::nan;
-  __hip_atomic_store((B *)p, b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename R> __device__ __forceinline__ void clear(R *p) {
-  __hip_atomic_store((typename Bits<R>::type *)p, Bits<R>::none, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename R> __device__ __forceinline__ typename Bits<R>::type poll(const R *p) {
-  return __hip_atomic_load((const typename Bits<R>::type *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// One more poll in vain: whether to give up.
-__device__ __forceinline__ bool give_up(int &spin, int *abort) {
-  return ++spin >= kSpin || (spin % 1024 == 0 && __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-
-// Sum over the wave, the same in every lane: within the rows of 16 lanes, then across them (DPP: no
-// LDS round trips as a shuffle makes).
-__device__ __forceinline__ double wave_sum(double v) {
-  auto step = [&](auto ctrl, auto rows) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
-    v += __builtin_bit_cast(double, (unsigned long long)(unsigned)hi << 32 | (unsigned)lo);
-  };
-  typedef std::integral_constant<int, 0xf> All;
-  step(std::integral_constant<int, 0x111>(), All());  // row_shr:1, 2, 4, 8
-  step(std::integral_constant<int, 0x112>(), All());
-  step(std::integral_constant<int, 0x114>(), All());
-  step(std::integral_constant<int, 0x118>(), All());
-  step(std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());  // row_bcast:15
-  step(std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());  // row_bcast:31
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const int lo = __builtin_amdgcn_readlane((int)b, 63), hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
-  return __builtin_bit_cast(double, (unsigned long long)(unsigned)hi << 32 | (unsigned)lo);
-}
-
 // Sum over each 8 lanes, the same in all of them.
 __device__ __forceinline__ double sum8(double v) {
   auto step = [&](auto ctrl) {

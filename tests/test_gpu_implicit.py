@@ -229,3 +229,28 @@ def test_cg_at_the_edges_of_its_blocks(dims):
     say("its", st.cg_iterations, "residual", res)
     assert st.converged and res <= 2e-4
     s.close()
+
+
+@pytest.mark.parametrize("kind", ["implicit", "pd"])
+@pytest.mark.parametrize("precision", [P.FP32, P.FP64])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (3, 3, 3), (2, 4, 12), (16, 16, 60), (20, 20, 80), (30, 30, 135), (31, 31, 130)])
+def test_resident_cg_equals_its_launches(dims, precision, kind):
+    """One, one full, four slices (the last with 3 rows); 276 slices (two per workgroup); 559 (up to
+    four, two shares per wave); 2043 (eight, all four shares); 2096 (too many for the resident loop).
+    Timed solvers launch every CG kernel by itself: iteration counts, positions and velocities are
+    equal bit for bit, since both paths add the same terms in the same order."""
+    rest, tets, mask, x0, v0 = case(*dims, twist=2.0)
+    say("resident CG", dims, precision, kind, len(rest))
+    out = []
+    for prof in (0, 1):
+        s = P.Solver(rest, tets, mask, P.default_params(precision=precision))
+        s.set_positions(x0)
+        s.set_velocities(v0, v0)
+        s.set_profiling(prof)
+        st = [s.implicit_step() if kind == "implicit" else s.pd_step() for _ in range(2)]
+        out.append(([q.cg_iterations for q in st], s.positions(f64=True), s.velocities()[0]))
+        s.close()
+    say("its", out[0][0])
+    assert out[0][0] == out[1][0]
+    assert np.array_equal(out[0][1].view(np.uint64), out[1][1].view(np.uint64))
+    assert np.array_equal(out[0][2].view(np.uint32), out[1][2].view(np.uint32))
