@@ -329,7 +329,7 @@ __device__ __forceinline__ void tile_tet(const uint4 lp, GetR get_r, GetNeo get_
       for (int k = 0; k < 9; ++k) H[k] = (C)(Fw[k] - ((k & 3) == 0 ? (FT)1 : (FT)0));
       neo_tet_disp<C>(H, Dmi, V, mu, lam, f12);
     } else {
-      stretch_tet<C, false>(F, Dmi, V, mu, lam, f12, en, h12);
+      stretch_tet<C, false, true>(F, Dmi, V, mu, lam, f12, en, h12);
     }
     store(f12);
     if (chk) count(MIX ? tet_energy<R, MAT>((const R *)Fw, (R)Vf, (R)mu, (R)lam) : (R)en);

@@ -549,3 +549,27 @@ def test_material_records_come_in_the_callers_tet_order(dims, precision):
     for a, b in zip(*got):
         assert np.array_equal(a[order].view(np.uint32), b.view(np.uint32))
     assert len(np.unique(got[0][0], axis=0)) > len(tets) // 2  # the records differ from tet to tet
+
+
+@pytest.mark.parametrize("amplitude", [1e-4, 0.05, 0.3, 1.0])
+def test_stretch_forces_of_a_pass_over_its_polar_range(amplitude):
+    """Stretch material, FP64, node forces as a descent pass forms them against the oracle's SVD, from
+    nearly undeformed tets (the polar iteration's fewest steps) over condition numbers up to its limit
+    of 20 to inverted tets (which take the SVD).  Tolerance relative to the sum of the magnitudes of a
+    node's terms: the rotation is good to 1e-15 where its smallest sum of two singular values is of
+    the order of 1, and a thousand nodes' tets come as near as 1e-5 or so to zero there, 1e-10; taken
+    100 times as large.  At amplitude 1e-4 the terms are 1e-4 of the rotation's size: 1e-11."""
+    rest, tets = M.bar(6, 6, 24, 0.05)
+    mask = M.clamp_x0(rest)
+    x = (rest + 0.05 * amplitude * np.random.default_rng(9).uniform(-1, 1, rest.shape)).astype(np.float32)
+    s = P.Solver(rest, tets, mask, P.default_params(precision=P.FP64, material=P.MAT_STRETCH))
+    nf, _, _ = s.tile_forces(x)
+    s.close()
+    mu, lam = O.lame(1e5, 0.45)
+    rf, _ = O.tet_forces(x.astype(np.float64), tets, oracle_pre(rest, tets, mask), mu, lam, O.MAT_STRETCH, O.CLAMP_GPU, 64)
+    ref, scale = np.zeros((len(rest), 3)), np.zeros(len(rest))
+    np.add.at(ref, tets.reshape(-1), rf.reshape(-1, 3))
+    np.add.at(scale, tets.reshape(-1), np.linalg.norm(rf.reshape(-1, 3), axis=1))
+    err = np.linalg.norm(nf - ref, axis=1) / scale
+    say("stretch pass", amplitude, "max err / sum|terms| %.2e" % err.max())
+    assert err.max() <= 1e-8
