@@ -553,12 +553,14 @@ def test_material_records_come_in_the_callers_tet_order(dims, precision):
 
 @pytest.mark.parametrize("amplitude", [1e-4, 0.05, 0.3, 1.0])
 def test_stretch_forces_of_a_pass_over_its_polar_range(amplitude):
-    """Stretch material, FP64, node forces as a descent pass forms them against the oracle's SVD, from
+    """Stretch material, FP64, node forces as a descent pass forms them against numpy's SVD, from
     nearly undeformed tets (the polar iteration's fewest steps) over condition numbers up to its limit
-    of 20 to inverted tets (which take the SVD).  Tolerance relative to the sum of the magnitudes of a
-    node's terms: the rotation is good to 1e-15 where its smallest sum of two singular values is of
-    the order of 1, and a thousand nodes' tets come as near as 1e-5 or so to zero there, 1e-10; taken
-    100 times as large.  At amplitude 1e-4 the terms are 1e-4 of the rotation's size: 1e-11."""
+    of 20 to inverted tets (which take the SVD).  Reference in FP64 from the solver's FP32 Dm^-1 and
+    volumes (the oracle rounds their product to FP32 once more, 6e-8).  Tolerance relative to the sum
+    of the magnitudes of a node's terms: the rotation is good to 1e-15 where its smallest sum of two
+    singular values is of the order of 1, and a thousand nodes' tets come as near as 1e-5 or so to
+    zero there, 1e-10; taken 100 times as large.  At amplitude 1e-4 the terms are 1e-4 of the
+    rotation's size: 1e-11."""
     rest, tets = M.bar(6, 6, 24, 0.05)
     mask = M.clamp_x0(rest)
     x = (rest + 0.05 * amplitude * np.random.default_rng(9).uniform(-1, 1, rest.shape)).astype(np.float32)
@@ -566,7 +568,16 @@ def test_stretch_forces_of_a_pass_over_its_polar_range(amplitude):
     nf, _, _ = s.tile_forces(x)
     s.close()
     mu, lam = O.lame(1e5, 0.45)
-    rf, _ = O.tet_forces(x.astype(np.float64), tets, oracle_pre(rest, tets, mask), mu, lam, O.MAT_STRETCH, O.CLAMP_GPU, 64)
+    pre = oracle_pre(rest, tets, mask)
+    Dmi = pre["dminv"].reshape(-1, 3, 3).astype(np.float64)
+    xt = x.astype(np.float64)[tets]
+    F = (xt[:, 1:] - xt[:, :1]).transpose(0, 2, 1) @ Dmi
+    U, S, Vt = np.linalg.svd(F)
+    U[:, :, 2] *= np.sign(np.linalg.det(F))[:, None]  # rotation: the last singular value carries the sign
+    J = np.linalg.det(F)[:, None, None]
+    Pk = 2 * mu * (F - U @ Vt) + lam * (J - 1) * J * np.linalg.inv(F).transpose(0, 2, 1)
+    G = -pre["vol"].reshape(-1, 1, 1).astype(np.float64) * (Pk @ Dmi.transpose(0, 2, 1))
+    rf = np.concatenate([-G.sum(2)[:, None], G.transpose(0, 2, 1)], axis=1)
     ref, scale = np.zeros((len(rest), 3)), np.zeros(len(rest))
     np.add.at(ref, tets.reshape(-1), rf.reshape(-1, 3))
     np.add.at(scale, tets.reshape(-1), np.linalg.norm(rf.reshape(-1, 3), axis=1))
