@@ -63,3 +63,29 @@ def test_resident_loop_matches_launches(dims, kw):
         assert a.energy == pytest.approx(b.energy, rel=1e-11)
     assert np.array_equal(xa.view(np.uint64), xb.view(np.uint64))
     assert np.array_equal(va[0].view(np.uint32), vb[0].view(np.uint32))
+
+
+def test_two_threads_step_at_once():
+    """Two solvers of one device stepped from two threads, descent and projective dynamics: each gives
+    what it gives alone (launches that hold the whole device take turns, they do not block each other)."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    rest, tets = M.bar(12, 12, 50, 0.05)
+    mask = M.clamp_x0(rest)
+    x0 = M.twisted_state(rest, 12, 12, 50, 0.05, 20.0, 0.005, 1)
+
+    def work(kind):
+        s = P.Solver(rest, tets, mask, P.default_params(precision=P.FP64))
+        s.set_positions(x0)
+        for _ in range(6):
+            s.pd_step() if kind else s.step()
+        out = s.positions(f64=True)
+        s.close()
+        return out
+
+    alone = [work(k) for k in (0, 1)]
+    say("two threads")
+    for kinds in ((0, 0), (0, 1), (1, 1)):
+        with ThreadPoolExecutor(2) as pool:
+            for k, x in zip(kinds, pool.map(work, kinds)):
+                assert np.array_equal(x.view(np.uint64), alone[k].view(np.uint64))
