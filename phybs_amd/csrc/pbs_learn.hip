@@ -366,8 +366,8 @@ __global__ void k_collect(DevParams p, const R *__restrict__ xnew, const float *
 // each wave accumulates 11 of the 44 gradient tiles in registers over all tiles of the workgroup.
 // At most 256 workgroups (one per CU: the arrays take 126 KB of LDS) write one gradient partial each.
 //
-// A batch of 8192 samples: 166 -> 20 us (on the vector units, both factors of each multiply-add
-// came from LDS), and its reduction, Adam step and arrangement 77 -> 4.7 us in one launch
+// A batch of 8192 samples: 166 -> 23 us (on the vector units, both factors of each multiply-add
+// came from LDS; 20 us without the activations formed again in FP64), and its reduction, Adam step and arrangement 77 -> 4.7 us in one launch
 // (k_mlp_step).  128 workgroups of 4 waves: what is left is the chain of one tile (weights 38 KB
 // and samples in, 192 exponentials per sample, 308 FP32 products per wave).  With the weights
 // converted one load at a time and the biases read where they are used it took 31 us.
@@ -400,6 +400,17 @@ __device__ __forceinline__ void silu_both(float z, float &v, float &dv) {
   v = z * s;
   v = fmaf(fmaf(-v, d, z), s, v);  // the quotient z / d to the last bit: it is rounded to BF16 next
   dv = s * fmaf(z, 1.0f - s, 1.0f);
+}
+
+// Whether a hidden activation v = SiLU(z), z = z0 + z1 + z2 + z3, is as near to the middle of two BF16
+// values as its own rounding error (about 1 in 2000).  One rounded to the other neighbour of an exact
+// evaluation's changes the sample's gradient in the third digit, far more than FP32 rounding does, so
+// those are formed again in FP64, by the whole wave (each by its own lane alone: 28 instead of 23 us a
+// batch; without it 20).  Relative error of the gradient against 64 bits, 30 seeds each of 65 to 30,000
+// samples: at most 1.7e-7, without it up to 7e-5; a bound of 1e-7 instead of 1.5e-7 misses a few.
+__device__ __forceinline__ bool near_middle(float v, float z0, float z1, float z2, float z3) {
+  const float mid = __builtin_bit_cast(float, (__builtin_bit_cast(unsigned, v) & 0xffff0000u) | 0x8000u);
+  return fabsf(v - mid) <= 1.5e-7f * (fabsf(z0) + fabsf(z1) + fabsf(z2) + fabsf(z3));
 }
 
 __global__ void __launch_bounds__(256) k_mlp_train(MlpDev net, const float *__restrict__ ds_x,
@@ -480,22 +491,48 @@ __global__ void __launch_bounds__(256) k_mlp_train(MlpDev net, const float *__re
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
       const int nkb = l == 0 ? 2 : 4, wa = l == 0 ? 0 : l == 1 ? 2048 : 6144;
+      unsigned again = 0;  // activations to form again, bit 4 mt + i
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt) {
-        f32x4 c = *(const f32x4 *)&S.bias[l][16 * mt + 4 * q];
+        f32x4 c[4] = {*(const f32x4 *)&S.bias[l][16 * mt + 4 * q], {}, {}, {}};
 #pragma unroll
         for (int kb = 0; kb < nkb; ++kb) {
           const bf16x4 a = *(const bf16x4 *)(S.wA + wa + (mt * nkb + kb) * 256 + lane * 4);
-          c = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, h[kb], c, 0, 0, 0);
+          c[kb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, h[kb], c[kb], 0, 0, 0);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           float v, dv;
-          silu_both(c[i], v, dv);
+          silu_both((c[0][i] + c[1][i]) + (c[2][i] + c[3][i]), v, dv);
           ds[l][mt][i] = dv;
           hn[mt][i] = (short)f2bf(v);
+          again |= (near_middle(v, c[0][i], c[1][i], c[2][i], c[3][i]) ? 1u : 0u) << (4 * mt + i);
           S.h[l][16 * mt + 4 * q + i][16 * w + r] = (unsigned short)hn[mt][i];
         }
+      }
+      // the whole wave forms each of them, lane k the product of input k; inputs and results in LDS
+      const unsigned short(*in)[SP] = l == 0 ? S.h0 : S.h[l > 0 ? l - 1 : 0];
+      const bool redo = again != 0;
+      for (unsigned long long left = __ballot(redo); left; left = __ballot(again != 0)) {
+        const int src = __ffsll(left) - 1, e = __ffs(__builtin_amdgcn_readlane((int)again, src)) - 1;
+        const int mt = e >> 2, row = 4 * (src >> 4) + (e & 3), col = 16 * w + (src & 15);
+        double z = 0.0;
+        if (lane < 16 * nkb) {
+          const int at = wa + (mt * nkb + (lane >> 4)) * 256 + (16 * ((lane >> 2) & 3) + row) * 4 + (lane & 3);
+          z = (double)bf2f(S.wA[at]) * (double)bf2f(in[lane][col]);
+        }
+        z = wave_sum(z) + (double)S.bias[l][16 * mt + row];
+        const unsigned short v = f2bf((float)(z / (1.0 + exp(-z))));
+        if (lane == src) {
+          S.h[l][16 * mt + row][col] = v;
+          again &= again - 1;
+        }
+      }
+      if (redo) {
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) hn[mt][i] = (short)S.h[l][16 * mt + 4 * q + i][16 * w + r];
       }
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt) h[mt] = hn[mt];

@@ -98,6 +98,41 @@ def test_training_at_the_edges_of_its_tiles(n):
     s.close()
 
 
+@pytest.mark.parametrize("n", [65, 700, 5003])
+def test_no_activation_rounds_to_the_other_side(n):
+    """Loss and gradient against 64 bits with the same BF16 roundings (of inputs, weights and hidden
+    activations, these from their exact values).  Every activation rounds as the exact one, so what is
+    left is FP32 rounding of deltas and sums, about 2e-7; taken 5 times as large.  One activation on
+    the other side would cost about 5e-3 / n."""
+    say("training against 64 bits", n)
+    rest, tets, mask, _ = bar()
+    s = P.Solver(rest, tets, mask, P.default_params())
+    s.learn_set_model(model(), SCALES)
+    inv = (np.float32(1) / SCALES).astype(np.float64)
+    p = list(zip(*MO.unpack(model(), np.float64)))
+    for seed in range(3):
+        rng = np.random.default_rng(seed)
+        f = rng.normal(0, 1, (n, 18)).astype(np.float32)
+        t = rng.normal(0, 1, (n, 3)).astype(np.float32)
+        loss, g = s.learn_loss_grad(f, t)
+        bf = lambda a: MO.bf16(a.astype(np.float32)).astype(np.float64)
+        h, z = [bf(f * np.repeat(inv[:6], 3))], []
+        for k, (w, b) in enumerate(p):
+            z.append(h[-1] @ bf(w) + b)
+            h.append(bf(MO.silu(z[-1])) if k < 3 else z[-1])
+        diff = h[-1] - t * inv[6]
+        lref, d, gref = (diff ** 2).mean(), 2 * diff / diff.size, []
+        for k in range(3, -1, -1):
+            gref = [(h[k].T @ d).reshape(-1), d.sum(0)] + gref
+            if k:
+                d = (d @ bf(p[k][0]).T) * MO.dsilu(z[k - 1])
+        gref = np.concatenate(gref)
+        err = np.linalg.norm(g - gref) / np.linalg.norm(gref)
+        say("loss", loss, lref, "grad rel err %.2e" % err)
+        assert loss == pytest.approx(lref, rel=1e-6) and err <= 1e-6
+    s.close()
+
+
 def adjacency(nn, tets):
     nb = [set() for _ in range(nn)]
     for t in tets:
