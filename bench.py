@@ -28,9 +28,9 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, 8 TB/s
 # same counter's reading for a plain elementwise kernel of known size) on the 64x64x256 bar:
 # (kernel, bytes per position component) -> bytes.  These are not measured by this script (a
 # counter run serialises every dispatch); the bench line names the profile they come from.  All
-# four were measured with 256-tet tiles (FP64 neo-Hookean solvers now default to 224).
-TRAFFIC_PROFILE = "profiles/k_tile_k_node_bar64x64x256_relgrad_f64.md"
-MEASURED_TRAFFIC = {("k_tile", 8): 237.6e6, ("k_tile", 4): 188.7e6, ("k_node", 8): 202.4e6, ("k_node", 4): 118.5e6}
+# four were measured with the default 256-tet tiles, the kernels launched one by one.
+TRAFFIC_PROFILE = "profiles/k_tile_k_node_bar64x64x256_counters.md"
+MEASURED_TRAFFIC = {("k_tile", 8): 246.5e6, ("k_tile", 4): 197.9e6, ("k_node", 8): 191.6e6, ("k_node", 4): 107.2e6}
 
 WORKLOADS = {
     # name: (nx, ny, nz, material, twist_deg, jitter, fixed iterations)

@@ -71,8 +71,9 @@ typedef struct pbs_params {
   int block_size;       /* threads per workgroup of the per-tet / per-node utility kernels, 0 = 256 */
   int tile_tets;        /* max tets per workgroup of the tile pass (16..4096); 0 = chosen from mesh size and
                            LDS; -1 = autotuned at creation (64, 128, 256, 512 timed on 32 passes) */
-  int graph_passes;     /* descent passes per captured HIP graph replay: 0 = 32, -1 = no graph
-                           (kernels launched one by one) */
+  int graph_passes;     /* descent passes per captured HIP graph replay: 0 = 32 (a single mesh of at most
+                           40,000 nodes with default tile_tets: the whole loop in one launch instead,
+                           the same iterates), -1 = no graph (kernels launched one by one) */
   double mixed_switch;  /* PBS_FP64 with graphs only (no reference counterpart): while |g|/|g_0| of
                            the last graph replay is above this, the tile pass forms F in FP64 and
                            evaluates the per-tet forces in FP32 (neo-Hookean: from H = F - I) with
@@ -204,15 +205,18 @@ int pbs_tile_forces(pbs_solver *s, const float *pos, double *node_forces, double
 /* ---- measurement ---- */
 /* Average device time per launch (ms) of each kernel of the last pbs_step calls, measured with
  * HIP events on the handle's stream: names[i] / avg_ms[i] / launches[i] for i < *count.  The
- * descent-pass kernels and the CG solves' SpMV and vector update are timed by events attached to
- * their own dispatch (the interval a kernel trace reports); step start, warm start, end, the
- * backward-Euler assembly and the PD local step by events recorded around them. */
+ * descent-pass kernels and the CG solves' SpMV and vector update (an iteration's two passes
+ * together) are timed by events attached to their own dispatch (the interval a kernel trace
+ * reports); step start, warm start, end, the backward-Euler assembly and the PD local step by
+ * events recorded around them. */
 int pbs_kernel_times(pbs_solver *s, int max, const char **names, double *avg_ms, long *launches, int *count);
 int pbs_reset_kernel_times(pbs_solver *s);
 /* period 0: no timing (default); 1: every descent-pass kernel is timed; n > 1: the kernels of
  * every n-th graph replay (every n-th pass without graphs) are timed, the timed replay's passes
  * being launched one by one instead of from the graph.  Launches that run after the loop has
- * stopped within a replay are not counted.  Any period > 0 times every CG replay. */
+ * stopped within a replay are not counted.  Any period > 0 times every CG replay.  A timed solver
+ * launches its kernels one by one where an untimed one of its size runs a resident loop; the iterates
+ * are the same. */
 int pbs_set_profiling(pbs_solver *s, int period);
 
 /* ---- backward Euler (the reference's GPU implicit path, fvm.cpp:179-183) ---- */
