@@ -289,11 +289,16 @@ bool build_persist_plan(const TilePlan &P, int max_parts, int nodes_per_part, Pe
   Q = PersistPlan();
   const int N = P.nn;
   const int G = std::max(1, std::min(max_parts, N / std::max(nodes_per_part, 1)));
-  std::vector<int> tile_of(P.nt), min_node(P.nt);
+  std::vector<int> tile_of(P.nt), first_tet(N + 1, 0);  // tets by smallest node: [first_tet[n], first_tet[n + 1])
   for (int b = 0; b < P.ntiles; ++b)
     for (int t = P.tiles[b].tet_start; t < P.tiles[b].tet_start + P.tiles[b].tet_cnt; ++t) tile_of[t] = b;
-  for (int t = 0; t < P.nt; ++t)
-    min_node[t] = *std::min_element(&P.tets_new[4 * (size_t)t], &P.tets_new[4 * (size_t)t] + 4);
+  std::vector<int> inc_sorted(P.inc.size()), fill(P.inc_off.begin(), P.inc_off.end());  // a node's entries, ascending
+  for (int t = 0; t < P.nt; ++t) {
+    const int *q = &P.tets_new[4 * (size_t)t];
+    first_tet[*std::min_element(q, q + 4) + 1]++;
+    for (int j = 0; j < 4; ++j) inc_sorted[fill[q[j]]++] = 4 * t + j;
+  }
+  for (int n = 0; n < N; ++n) first_tet[n + 1] += first_tet[n];
   std::vector<int> tile_of_node(N);
   for (int b = 0; b < P.ntiles; ++b)
     for (int n = P.tiles[b].own_start; n < P.tiles[b].own_start + P.tiles[b].own_cnt; ++n) tile_of_node[n] = b;
@@ -307,13 +312,18 @@ bool build_persist_plan(const TilePlan &P, int max_parts, int nodes_per_part, Pe
     p.own_start = (int)((long)N * g / G);
     const int n1 = (int)((long)N * (g + 1) / G);
     p.own_cnt = n1 - p.own_start;
+    // its tets, ascending: those of earlier nodes, then the run whose smallest node it owns
     tets.clear();
+    const int t0 = first_tet[p.own_start], t1 = first_tet[n1];
     for (int e = P.inc_off[p.own_start]; e < P.inc_off[n1]; ++e) {
-      const int t = P.inc[e] >> 2;
-      if (part_of[t] != g) tets.push_back(t);
-      part_of[t] = g;
+      const int t = inc_sorted[e] >> 2;
+      if (t < t0 && part_of[t] != g) {
+        part_of[t] = g;
+        tets.push_back(t);
+      }
     }
     std::sort(tets.begin(), tets.end());
+    for (int t = t0; t < t1; ++t) tets.push_back(t);
     ghosts.clear();
     for (size_t k = 0; k < tets.size(); ++k) {
       at_tet[tets[k]] = (int)k;
@@ -340,8 +350,7 @@ bool build_persist_plan(const TilePlan &P, int max_parts, int nodes_per_part, Pe
     int at = 0;
     for (int n = p.own_start; n < n1; ++n) {
       // entries 4 tet + corner: the node's own tile first, then tile order (tets ascend with tiles)
-      inc.assign(P.inc.begin() + P.inc_off[n], P.inc.begin() + P.inc_off[n + 1]);
-      std::sort(inc.begin(), inc.end());
+      inc.assign(inc_sorted.begin() + P.inc_off[n], inc_sorted.begin() + P.inc_off[n + 1]);
       const auto own = [&](int e) { return tile_of[e >> 2] == tile_of_node[n]; };
       const auto o0 = std::find_if(inc.begin(), inc.end(), own);
       std::rotate(inc.begin(), o0, std::find_if_not(o0, inc.end(), own));
@@ -362,11 +371,10 @@ bool build_persist_plan(const TilePlan &P, int max_parts, int nodes_per_part, Pe
       uint32_t l[4];
       for (int j = 0; j < 4; ++j) l[j] = (uint32_t)loc[P.tets_new[4 * (size_t)t + j]];
       const uint16_t *q = &slot[4 * k];
-      const uint32_t own = min_node[t] >= p.own_start && min_node[t] < n1 ? 0x80000000u : 0u;
-      Q.lp.push_back(l[0] | (l[1] << 16));
-      Q.lp.push_back(l[2] | (l[3] << 16));
-      Q.lp.push_back((uint32_t)q[0] | ((uint32_t)q[1] << 16) | own);
-      Q.lp.push_back((uint32_t)q[2] | ((uint32_t)q[3] << 16));
+      const uint32_t own = t >= t0 ? 0x80000000u : 0u;
+      const uint32_t w[4] = {l[0] | (l[1] << 16), l[2] | (l[3] << 16), (uint32_t)q[0] | ((uint32_t)q[1] << 16) | own,
+                             (uint32_t)q[2] | ((uint32_t)q[3] << 16)};
+      Q.lp.insert(Q.lp.end(), w, w + 4);
       Q.tet.push_back(t);
     }
     Q.ghost.insert(Q.ghost.end(), ghosts.begin(), ghosts.end());
