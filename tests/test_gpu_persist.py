@@ -42,6 +42,8 @@ CASES = [
     ((4, 4, 16), dict(iterations=1)),
     ((4, 4, 16), dict(iterations=0)),
     ((12, 12, 50), dict(precision=P.FP64, relgrad_tol=1e-4, max_iterations=20000)),
+    ((4, 4, 16), dict(iterations=5000)),                                     # ends in rollbacks
+    ((6, 6, 40), dict(precision=P.FP64, relgrad_tol=1e-7, max_iterations=9000, profile=[])),  # several launches
     ((17, 18, 60), dict()),                                                  # 110 K tets: two tets per thread
     ((17, 18, 60), dict(precision=P.FP64, material=P.MAT_STRETCH, iterations=40)),
     ((24, 25, 60), dict()),                                                  # 216 K tets
