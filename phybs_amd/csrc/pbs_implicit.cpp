@@ -47,78 +47,39 @@ template <typename T> int ialloc(ImplicitState *S, T **p, size_t n) {
   return PBS_OK;
 }
 
-// The resident solver's partition: workgroup g owns vector blocks [g per_part, (g + 1) per_part), their
-// slices and rows; the columns it does not own are its ghosts, ascending.  False where the system has
-// more slices than 256 workgroups of 8 waves hold (131,072 rows), wider rows than the registers, or a
-// workgroup more ghosts than its threads read at once.
-bool cg_partition(const ImplicitState &S, const IeDev &d, CgDev &c, std::vector<int> &ghost_off, std::vector<int> &ghost,
-                  std::vector<uint16_t> &lcol) {
-  const int N = d.n;
-  if (S.nslice == 0 || S.nslice > kCgSlices || S.max_width > kCgWidth) return false;
-  c.per_part = d.vec_blocks > 256 ? 2 : 1;
-  c.nparts = (d.vec_blocks + c.per_part - 1) / c.per_part;
-  lcol.assign(S.slots, 0);
-  ghost_off.assign(1, 0);
-  ghost.clear();
-  std::vector<int> local(N, -1), seen;
-  auto first_slice = [&](int b) { return b * d.vec_per + std::min(b, d.vec_rem); };
-  for (int g = 0; g < c.nparts; ++g) {
-    const int s0 = first_slice(g * c.per_part), s1 = first_slice(std::min((g + 1) * c.per_part, d.vec_blocks));
-    const int n0 = 64 * s0, n1 = std::min(N, 64 * s1);
-    c.shares = std::max(c.shares, s1 - s0 <= 2 ? 1 : s1 - s0 <= 4 ? 2 : 4);
-    seen.clear();
-    for (int n = n0; n < n1; ++n) {
-      const long at = S.slice_off_h[n >> 6];
-      for (int j = 0; j < S.row_len_h[n]; ++j) {
-        const int m = S.bcol_h[(at + j) * 64 + (n & 63)];
-        if ((m < n0 || m >= n1) && local[m] < 0) {
-          local[m] = 0;
-          seen.push_back(m);
-        }
-      }
-    }
-    if (seen.size() > (size_t)kCgGhosts) return false;
-    std::sort(seen.begin(), seen.end());
-    for (size_t k = 0; k < seen.size(); ++k) local[seen[k]] = n1 - n0 + (int)k;
-    for (int sl = s0; sl < s1; ++sl)
-      for (long at = 64L * S.slice_off_h[sl]; at < 64L * S.slice_off_h[sl + 1]; ++at) {
-        const int m = S.bcol_h[at];  // (a row's padding: its own column; past the last row: any of its own)
-        lcol[at] = m >= n0 && m < n1 ? (uint16_t)(m - n0) : local[m] >= 0 ? (uint16_t)local[m] : 0;
-      }
-    for (int m : seen) local[m] = -1;
-    ghost.insert(ghost.end(), seen.begin(), seen.end());
-    ghost_off.push_back((int)ghost.size());
-    c.local_max = std::max(c.local_max, n1 - n0 + (int)seen.size());
-  }
-  return true;
-}
-
-// Uploads it with its exchange buffers; without it (or where the device cannot hold it) the vector
-// passes are split for the launches alone.
+// Plans the resident solver and uploads it with its exchange buffers; without it (or where the device
+// cannot hold it) the vector passes are split for the launches alone.
 template <typename R> int cg_setup(pbs_solver *s, ImplicitState *S) {
   IeDev &d = S->dev;
-  ie_vec_split(d, true);
   CgDev c{};
-  std::vector<int> goff, ghost;
-  std::vector<uint16_t> lcol;
-  if (cg_partition(*S, d, c, goff, ghost, lcol))
+  CgPlan Q;
+  if (build_cg_plan(S->rows, Q)) {
+    c.nparts = Q.nparts;
+    c.per_part = Q.per_part;
+    c.shares = Q.shares;
+    c.local_max = Q.local_max;
     for (int scalar = 0; scalar < 2; ++scalar) S->cg_fits[scalar] = IeLaunch<R>::resident_fits(c, scalar, s->device);
+  }
   if (!S->cg_fits[0] && !S->cg_fits[1]) {
-    ie_vec_split(d, false);
+    ie_vec_split(d);
     return PBS_OK;
   }
+  d.vec_unit = 192;
+  d.vec_per = Q.vec_per;
+  d.vec_rem = Q.vec_rem;
+  d.vec_blocks = Q.vec_blocks;
   int *go, *gh, *abort;
   unsigned short *lc;
   const size_t nz = 2 * 3 * (size_t)d.n, nx = (nz + 4 * (size_t)d.vec_blocks + 1) & ~(size_t)1;
-  int rc = ialloc(S, &go, goff.size());
-  if (!rc) rc = ialloc(S, &gh, ghost.size());
-  if (!rc) rc = ialloc(S, &lc, lcol.size());
+  int rc = ialloc(S, &go, Q.ghost_off.size());
+  if (!rc) rc = ialloc(S, &gh, Q.ghost.size());
+  if (!rc) rc = ialloc(S, &lc, Q.lcol.size());
   if (!rc) rc = ialloc(S, &abort, 1);
   if (!rc) rc = ialloc(S, &c.z, nx);
   if (rc) return rc;
-  HIPCHK(hipMemcpy(go, goff.data(), sizeof(int) * goff.size(), hipMemcpyHostToDevice));
-  if (!ghost.empty()) HIPCHK(hipMemcpy(gh, ghost.data(), sizeof(int) * ghost.size(), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(lc, lcol.data(), sizeof(uint16_t) * lcol.size(), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(go, Q.ghost_off.data(), sizeof(int) * Q.ghost_off.size(), hipMemcpyHostToDevice));
+  if (!Q.ghost.empty()) HIPCHK(hipMemcpy(gh, Q.ghost.data(), sizeof(int) * Q.ghost.size(), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(lc, Q.lcol.data(), sizeof(uint16_t) * Q.lcol.size(), hipMemcpyHostToDevice));
   c.ghost_off = go;
   c.ghost = gh;
   c.lcol = lc;
@@ -130,9 +91,7 @@ template <typename R> int cg_setup(pbs_solver *s, ImplicitState *S) {
   return PBS_OK;
 }
 
-// Block rows of K in solver order: a node's columns are the nodes sharing a tet with it,
-// ascending, itself included (the block pattern of allocateGlobalStiffnessMatrix,
-// IsotropicMaterial.cpp:554-644), laid out as SELL-64.
+// The block rows of K (pbs_cg_plan.h), the system's buffers and the resident solver's, at the first use.
 int implicit_get(pbs_solver *s, ImplicitState **out) {
   if (s->implicit) {
     *out = s->implicit;
@@ -140,64 +99,27 @@ int implicit_get(pbs_solver *s, ImplicitState **out) {
   }
   if (s->ninst != 1) return set_error(PBS_ERR_STATE, "backward-Euler step: not available on a batched solver");
   const int N = s->nn;
-  const TilePlan &P = s->plan;
-  std::vector<int> row_off(N + 1, 0), cols, tmp;
-  cols.reserve((size_t)N * 16);
-  for (int n = 0; n < N; ++n) {
-    tmp.clear();
-    for (int e = P.inc_off[n]; e < P.inc_off[n + 1]; ++e) {
-      const int t = P.inc[e] >> 2;
-      for (int c = 0; c < 4; ++c) tmp.push_back(P.tets_new[4 * (size_t)t + c]);
-    }
-    tmp.push_back(n);
-    std::sort(tmp.begin(), tmp.end());
-    tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
-    cols.insert(cols.end(), tmp.begin(), tmp.end());
-    row_off[n + 1] = (int)cols.size();
-  }
   ImplicitState *S = new ImplicitState();
-  S->nslice = (N + 63) / 64;
-  S->slice_off_h.assign(S->nslice + 1, 0);
-  S->row_len_h.resize(N);
-  for (int n = 0; n < N; ++n) S->row_len_h[n] = row_off[n + 1] - row_off[n];
-  for (int sl = 0; sl < S->nslice; ++sl) {
-    int w = 0;
-    for (int n = 64 * sl; n < std::min(N, 64 * sl + 64); ++n) w = std::max(w, S->row_len_h[n]);
-    S->slice_off_h[sl + 1] = S->slice_off_h[sl] + w;
-  }
-  S->slots = 64L * S->slice_off_h[S->nslice];
-  for (int sl = 0; sl < S->nslice; ++sl)
-    S->max_width = std::max(S->max_width, S->slice_off_h[sl + 1] - S->slice_off_h[sl]);
-  S->bcol_h.assign(S->slots, 0);
-  std::vector<int> diag(N);
-  for (int n = 0; n < N; ++n) {
-    const long g0 = S->slice_off_h[n >> 6], w = S->slice_off_h[(n >> 6) + 1] - g0;
-    const int lane = n & 63;
-    for (long j = 0; j < w; ++j) {
-      const bool real = j < S->row_len_h[n];
-      const int c = real ? cols[row_off[n] + j] : n;
-      S->bcol_h[(g0 + j) * 64 + lane] = c;
-      if (real && c == n) diag[n] = (int)((g0 + j) * 64 + lane);
-    }
-  }
+  BlockRows &B = S->rows;
+  build_block_rows(s->plan, B);
   const size_t rsz = s->p.precision == PBS_FP64 ? 8 : 4;
   const size_t n3 = 3 * (size_t)N;
   // partial sums: the SpMV has at most one block per slice, the start kernel one per 4 slices, the
   // vector passes one per 1024 entries of 3N
   IeDev &d = S->dev;
   d.n = N;
-  d.nslice = S->nslice;
+  d.nslice = B.nslice;
   int *so = nullptr, *rl = nullptr, *bc = nullptr, *dsl = nullptr;
   char *A = nullptr;
-  int rc = ialloc(S, &so, S->nslice + 1);
+  int rc = ialloc(S, &so, B.nslice + 1);
   if (!rc) rc = ialloc(S, &rl, N);
-  if (!rc) rc = ialloc(S, &bc, S->slots);
+  if (!rc) rc = ialloc(S, &bc, B.slots);
   if (!rc) rc = ialloc(S, &dsl, N);
-  if (!rc) rc = ialloc(S, &A, 9 * rsz * S->slots);
+  if (!rc) rc = ialloc(S, &A, 9 * rsz * B.slots);
   double **vec[6] = {&d.b, &d.x, &d.z, &d.p, &d.Ap, &d.dinv};
   for (int i = 0; i < 6 && !rc; ++i) rc = ialloc(S, vec[i], n3);
-  if (!rc) rc = ialloc(S, &d.part_rz, (size_t)S->nslice);
-  if (!rc) rc = ialloc(S, &d.part_pap, (size_t)S->nslice);
+  if (!rc) rc = ialloc(S, &d.part_rz, (size_t)B.nslice);
+  if (!rc) rc = ialloc(S, &d.part_pap, (size_t)B.nslice);
   if (!rc) rc = ialloc(S, &d.ctrl, 2);
   if (rc) {
     implicit_release(S);
@@ -208,10 +130,10 @@ int implicit_get(pbs_solver *s, ImplicitState **out) {
   d.bcol = bc;
   d.diag_slot = dsl;
   d.A = A;
-  hipError_t e = hipMemcpy(so, S->slice_off_h.data(), sizeof(int) * (S->nslice + 1), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(rl, S->row_len_h.data(), sizeof(int) * N, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(bc, S->bcol_h.data(), sizeof(int) * S->slots, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(dsl, diag.data(), sizeof(int) * N, hipMemcpyHostToDevice);
+  hipError_t e = hipMemcpy(so, B.slice_off.data(), sizeof(int) * (B.nslice + 1), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(rl, B.row_len.data(), sizeof(int) * N, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(bc, B.bcol.data(), sizeof(int) * B.slots, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemcpy(dsl, B.diag.data(), sizeof(int) * N, hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     implicit_release(S);
     return set_error(PBS_ERR_HIP, std::string("backward-Euler setup: ") + hipGetErrorString(e));
@@ -393,7 +315,7 @@ int implicit_step_impl(pbs_solver *s, const pbs_implicit_params *ip, const float
   HIPCHK(hipEventRecord(s->ev0, s->st));
   hipEvent_t *ea = timed ? &S->ev[kIterEvents * kGraphIters] : nullptr;  // events around the assembly
   if (ea) HIPCHK(hipEventRecord(ea[0], s->st));
-  IeLaunch<R>::assemble(m, s->td, s->dp, d, a, S->max_width, s->st);
+  IeLaunch<R>::assemble(m, s->td, s->dp, d, a, S->rows.max_width, s->st);
   HIPCHK(hipGetLastError());
   if (ea) HIPCHK(hipEventRecord(ea[1], s->st));
   IeCtrl c{};
@@ -431,7 +353,7 @@ template <typename R> int pd_get(pbs_solver *s, ImplicitState **out) {
   if (rc) return rc;
   if (!S->pd.A) {
     char *A = nullptr;
-    rc = ialloc(S, &A, sizeof(R) * (size_t)S->slots);
+    rc = ialloc(S, &A, sizeof(R) * (size_t)S->rows.slots);
     if (!rc) rc = ialloc(S, &S->pd_s, 3 * (size_t)s->nn);
     if (!rc) rc = ialloc(S, &S->pd_inc_pos, 4 * (size_t)s->nt);
     if (rc) return rc;
@@ -547,26 +469,26 @@ template <typename R> int stiffness_impl(pbs_solver *s, int64_t nnz, double *csr
   if (rc) return rc;
   const int N = s->nn;
   int64_t total = 0;
-  for (int n = 0; n < N; ++n) total += 9L * S->row_len_h[n];
+  for (int n = 0; n < N; ++n) total += 9L * S->rows.row_len[n];
   if (nnz != total) return set_error(PBS_ERR_ARG, "nnz does not match the stiffness pattern (" + std::to_string(total) + ")");
   IeAsm a{};
   a.raw = 1;
-  IeLaunch<R>::assemble(mesh<R>(s), s->td, s->dp, S->dev, a, S->max_width, s->st);
+  IeLaunch<R>::assemble(mesh<R>(s), s->td, s->dp, S->dev, a, S->rows.max_width, s->st);
   HIPCHK(hipGetLastError());
-  std::vector<R> A(9 * (size_t)S->slots);
+  std::vector<R> A(9 * (size_t)S->rows.slots);
   HIPCHK(hipMemcpyAsync(A.data(), S->dev.A, sizeof(R) * A.size(), hipMemcpyDeviceToHost, s->st));
   HIPCHK(hipStreamSynchronize(s->st));
   // reference CSR order: row 3a+d of caller node a, columns 3b+e with b ascending in caller ids
   const std::vector<int> &perm = s->plan.perm, &iperm = s->plan.iperm;
   std::vector<int64_t> row_start(N + 1, 0);
-  for (int a2 = 0; a2 < N; ++a2) row_start[a2 + 1] = row_start[a2] + 9L * S->row_len_h[iperm[a2]];
+  for (int a2 = 0; a2 < N; ++a2) row_start[a2 + 1] = row_start[a2] + 9L * S->rows.row_len[iperm[a2]];
   std::vector<std::pair<int, long>> nb;
   for (int a2 = 0; a2 < N; ++a2) {
     const int n = iperm[a2];
-    const long g0 = S->slice_off_h[n >> 6];
-    const int lane = n & 63, len = S->row_len_h[n];
+    const long g0 = S->rows.slice_off[n >> 6];
+    const int lane = n & 63, len = S->rows.row_len[n];
     nb.clear();
-    for (int j = 0; j < len; ++j) nb.push_back({perm[S->bcol_h[(g0 + j) * 64 + lane]], g0 + j});
+    for (int j = 0; j < len; ++j) nb.push_back({perm[S->rows.bcol[(g0 + j) * 64 + lane]], g0 + j});
     std::sort(nb.begin(), nb.end());
     const int64_t rs = row_start[a2];
     const int64_t rl = 3L * len;  // values per CSR row

@@ -6,6 +6,7 @@
 
 #include <vector>
 
+#include "pbs_cg_plan.h"
 #include "pbs_internal.h"
 
 namespace pbs {
@@ -43,15 +44,11 @@ struct IeAsm {
   int has_ext;
 };
 
-// Sets the split of the vector passes: whole slices per block (at most 4), as the resident solver's
-// workgroups own them, or blocks of at least 1024 entries.
-void ie_vec_split(IeDev &d, bool slices);
+// Sets the split of the vector passes for the launches alone: blocks of at least 1024 entries (the
+// resident solver's plan has whole slices per block, at most 4).
+void ie_vec_split(IeDev &d);
 
-// The resident CG (k_cg): partition and exchange buffers.  A workgroup owns one or two of the vector
-// passes' blocks and their slices' rows.
-constexpr int kCgThreads = 512;
-// at most: slices, slots of a slice, ghosts of a workgroup
-constexpr int kCgSlices = 2048, kCgWidth = 28, kCgGhosts = 8 * kCgThreads / 3;
+// The resident CG (k_cg): partition (pbs_cg_plan.h) and exchange buffers.
 struct CgDev {
   int nparts, per_part;           // workgroups (0: not used), vector blocks of each
   int shares;                     // shares of a slice that one wave multiplies (1, 2 or 4)
@@ -97,9 +94,7 @@ struct CgGraphs {
 };
 
 struct ImplicitState {
-  int nslice = 0;
-  long slots = 0;
-  int max_width = 0;                                // slots per row of the widest slice
+  BlockRows rows;                                   // (kept for the stiffness export)
   IeDev dev{};                                      // backward Euler: 3x3 blocks
   IeDev pd{};                                       // projective dynamics: same layout and vectors, scalar values
   double *pd_s = nullptr;                           // projective dynamics: momentum term (3N)
@@ -109,7 +104,6 @@ struct ImplicitState {
   float pd_stiffness = 0.0f;
   double pd_h = 0.0;
   int *pd_inc_pos = nullptr;                        // projective dynamics: incidence slot of each (tet, corner)
-  std::vector<int> slice_off_h, row_len_h, bcol_h;  // host copies (stiffness export)
   CgGraphs cg_ie, cg_pd;
   CgDev cg{};                                       // resident solver
   bool cg_fits[2] = {false, false};                 // for 3x3 blocks; for scalar values

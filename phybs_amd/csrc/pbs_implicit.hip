@@ -446,7 +446,6 @@ __global__ void k_tet_stiffness(DevParams p, int num, const int *__restrict__ id
 // (multiples of 64), so that few blocks have the SpMV's partials to sum and every block the same
 // work (both passes at 6.3 M tets with 512, 1024, 2048 blocks: 52.4, 53.4, 59.7 us);
 // XCD-contiguous as the SpMV's rows.
-constexpr int kVecBlocks = 512;
 constexpr int kVec = 4;  // entries a thread has in flight
 __device__ __forceinline__ void vec_range(const IeDev &d, int &i0, int &i1) {
   const int b = xcd_block(blockIdx.x, gridDim.x);
@@ -688,7 +687,7 @@ template <typename R, int BLK, int SH> __global__ void __launch_bounds__(kCgThre
   __shared__ double share[2 * SH][4][3][64];  // Ap of each slice in four shares
   __shared__ double csum[8][3], zsum[2][4], tot[2][4];
   __shared__ int gave_up;
-  constexpr int NU = 3, GH = kCgGhosts * 3 / kCgThreads, WS = 4 / SH, NJ = kCgWidth / 4, NV = BLK * BLK;
+  constexpr int NU = 3, GH = cg_ghost_entries(SH), WS = 4 / SH, NJ = kCgWidth / 4, NV = BLK * BLK;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int g = xcd_block(blockIdx.x, c.nparts);
   IeCtrl in = d.ctrl[0];
@@ -1113,10 +1112,10 @@ template <typename R> void IeLaunch<R>::start(const IeDev &d, hipStream_t st) {
   hipLaunchKernelGGL(k_ie_start_ctrl, dim3(1), dim3(1024), 0, st, d, nb_of(d.n));
 }
 
-void ie_vec_split(IeDev &d, bool slices) {
-  d.vec_unit = slices ? 192 : 64;
-  const int groups = slices ? d.nslice : (3 * d.n + 63) / 64;
-  const long most = slices ? d.nslice : (3 * (long)d.n + kVec * kBlock - 1) / (kVec * kBlock);
+void ie_vec_split(IeDev &d) {
+  d.vec_unit = 64;
+  const int groups = (3 * d.n + 63) / 64;
+  const long most = (3 * (long)d.n + kVec * kBlock - 1) / (kVec * kBlock);
   d.vec_blocks = (int)std::min<long>(most, kVecBlocks);
   d.vec_per = groups / d.vec_blocks;
   d.vec_rem = groups % d.vec_blocks;
