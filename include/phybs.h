@@ -218,6 +218,15 @@ int pbs_reset_kernel_times(pbs_solver *s);
  * launches its kernels one by one where an untimed one of its size runs a resident loop; the iterates
  * are the same. */
 int pbs_set_profiling(pbs_solver *s, int period);
+/* How the last step's descent loop and the last CG solve ran: kernel by kernel, as one resident launch,
+ * or as a resident launch of which some workgroup gave up waiting for another, and then kernel by kernel
+ * from the same start (as does every later one of the handle).  Either pointer may be NULL. */
+enum { PBS_LOOP_NONE = 0, PBS_LOOP_LAUNCHES = 1, PBS_LOOP_RESIDENT = 2, PBS_LOOP_GAVE_UP = 3 };
+int pbs_last_loops(const pbs_solver *s, int *descent, int *cg);
+/* How often a workgroup of a resident launch looks in vain for another's values before it gives up (0: the
+ * default, about a second), from the launch's exchange `from` on (a descent pass has one, a CG iteration
+ * two; those before it keep the default).  The handle's resident loops are tried again. */
+int pbs_set_resident_polls(pbs_solver *s, int polls, int from);
 
 /* ---- backward Euler (the reference's GPU implicit path, fvm.cpp:179-183) ---- */
 typedef struct pbs_implicit_params {

@@ -17,6 +17,7 @@ ERR_ARG, ERR_HIP, ERR_MESH, ERR_IO, ERR_STATE = -1, -2, -3, -4, -5
 SEM_REF_GPU, SEM_REF_CPU = 0, 1
 FP32, FP64 = 32, 64
 MAT_NEOHOOKEAN, MAT_STRETCH = 0, 1
+LOOP_NONE, LOOP_LAUNCHES, LOOP_RESIDENT, LOOP_GAVE_UP = 0, 1, 2, 3
 
 
 class PhybsError(RuntimeError):
@@ -127,6 +128,8 @@ SIGNATURES = {
     "pbs_kernel_times": (C.c_int, [_P, C.c_int, _P, _P, _P, _P]),
     "pbs_reset_kernel_times": (C.c_int, [_P]),
     "pbs_set_profiling": (C.c_int, [_P, C.c_int]),
+    "pbs_last_loops": (C.c_int, [_P, _P, _P]),
+    "pbs_set_resident_polls": (C.c_int, [_P, C.c_int, C.c_int]),
     "pbs_mesh_bar": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_float, _P, _P]),
     "pbs_mesh_twist": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_float, C.c_double, C.c_double, C.c_uint64,
                                  C.c_int, _P]),
@@ -522,6 +525,18 @@ class Solver:
     def set_profiling(self, period=1):
         """period: 0/False off, 1/True every pass, n: every n-th graph replay."""
         _check(lib().pbs_set_profiling(self.h, int(period)))
+
+    def last_loops(self):
+        """How the last step's descent loop and the last CG solve ran: (descent, cg), each LOOP_NONE,
+        LOOP_LAUNCHES, LOOP_RESIDENT or LOOP_GAVE_UP."""
+        d, c = C.c_int(), C.c_int()
+        _check(lib().pbs_last_loops(self.h, C.byref(d), C.byref(c)))
+        return d.value, c.value
+
+    def set_resident_polls(self, polls=0, start=0):
+        """Polls in vain before a workgroup of a resident launch gives up (0: the default), from the
+        launch's exchange `start` on."""
+        _check(lib().pbs_set_resident_polls(self.h, int(polls), int(start)))
 
     def reset_kernel_times(self):
         _check(lib().pbs_reset_kernel_times(self.h))

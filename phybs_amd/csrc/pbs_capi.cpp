@@ -1034,6 +1034,7 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
   }
   const bool relg = s->dp.relgrad_tol > 0;
   const long cap = relg ? (long)s->p.max_iterations + 256 : (long)s->p.iterations + 256;
+  s->descent_loop = PBS_LOOP_LAUNCHES;
   long launched = 0;
   long n = relg ? 32 : std::max(s->p.iterations, 1);
   // control blocks of all instances: the loop runs while any instance is active; a pass counts
@@ -1075,7 +1076,9 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
   }
   while (true) {
     // the resident loop: the default graph length, no timing of single kernels, no mixed mode
-    if (s->persist.nparts > 0 && s->p.graph_passes == 0 && !period && !mixed) {
+    if (s->persist.nparts > 0 && !s->descent_gave_up && s->p.graph_passes == 0 && !period && !mixed) {
+      s->persist.polls = s->resident_polls;
+      s->persist.from = s->resident_from;
       // one launch runs the step (at most 4096 passes at a time)
       const int most = (int)std::min<long>(std::max<long>(cap - launched, 1), 4096);
       Ctrl two[2];  // the control block and the abort flag behind it
@@ -1086,6 +1089,7 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
         int gave_up;
         std::memcpy(&gave_up, &two[1], sizeof(int));
         if (!gave_up) {
+          s->descent_loop = PBS_LOOP_RESIDENT;
           ch[0] = two[0];
           launched += most;
           if (all_done()) break;
@@ -1095,7 +1099,8 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
       }
       // not launchable, or its workgroups did not all run: the step starts again on the other path
       (void)hipGetLastError();
-      s->persist.nparts = 0;
+      s->descent_gave_up = true;
+      s->descent_loop = PBS_LOOP_GAVE_UP;
       int rc = begin_step();
       if (rc) return rc;
       launched = 0;
@@ -1385,6 +1390,21 @@ extern "C" int pbs_get_rest_data(pbs_solver *s, float *dminv, float *vol, float 
 }
 
 // ---- measurement ----
+extern "C" int pbs_last_loops(const pbs_solver *s, int *descent, int *cg) {
+  if (!s) return set_error(PBS_ERR_ARG, "null solver");
+  if (descent) *descent = s->descent_loop;
+  if (cg) *cg = s->cg_loop;
+  return PBS_OK;
+}
+
+extern "C" int pbs_set_resident_polls(pbs_solver *s, int polls, int from) {
+  if (!s || polls < 0 || from < 0) return set_error(PBS_ERR_ARG, "null solver or negative argument");
+  s->resident_polls = polls ? polls : kPolls;
+  s->resident_from = from;
+  s->descent_gave_up = s->cg_gave_up = false;
+  return PBS_OK;
+}
+
 extern "C" int pbs_set_profiling(pbs_solver *s, int period) {
   if (!s) return set_error(PBS_ERR_ARG, "null handle");
   if (period < 0) return set_error(PBS_ERR_ARG, "profiling period must be >= 0");

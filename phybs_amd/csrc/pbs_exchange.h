@@ -9,8 +9,6 @@
 
 namespace pbs {
 
-constexpr int kSpin = 1 << 20;  // polls before giving up (about a second)
-
 template <typename R> struct Bits;
 template <> struct Bits<double> {
   typedef unsigned long long type;
@@ -32,9 +30,9 @@ template <typename R> __device__ __forceinline__ void clear(R *p) {
 template <typename R> __device__ __forceinline__ typename Bits<R>::type poll(const R *p) {
   return __hip_atomic_load((const typename Bits<R>::type *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// One more poll in vain: whether to give up.
-__device__ __forceinline__ bool give_up(int &spin, int *abort) {
-  return ++spin >= kSpin || (spin % 1024 == 0 && __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+// One more poll in vain: whether to give up (after `polls` of them, or when another has).
+__device__ __forceinline__ bool give_up(int &spin, int polls, int *abort) {
+  return ++spin >= polls || (spin % 1024 == 0 && __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
 }  // namespace pbs

@@ -204,7 +204,11 @@ int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double to
   IeLaunch<R>::start(dev, s->st);
   HIPCHK(hipGetLastError());
   c = IeCtrl{};
-  if (S->cg_fits[dev.scalar] && !timed) {
+  s->cg_loop = PBS_LOOP_LAUNCHES;
+  if (S->cg_fits[dev.scalar] && !s->cg_gave_up && !timed) {
+    S->cg.polls = s->resident_polls;
+    S->cg.from = s->resident_from;
+    s->cg_loop = PBS_LOOP_RESIDENT;
     hipError_t e = IeLaunch<R>::resident(dev, S->cg, s->st);
     int gave_up = 1;
     if (e == hipSuccess) {
@@ -214,7 +218,8 @@ int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double to
     }
     if (gave_up) {  // not launchable, or its workgroups did not all run: the launches, from the same start
       (void)hipGetLastError();
-      S->cg_fits[0] = S->cg_fits[1] = false;
+      s->cg_gave_up = true;
+      s->cg_loop = PBS_LOOP_GAVE_UP;
       c = IeCtrl{};
     }
   }

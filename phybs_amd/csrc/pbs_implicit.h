@@ -58,6 +58,7 @@ struct CgDev {
   double *z, *pap, *rz;           // 2 slots each: 3N values; partials per vector block
   long xch_bytes;                 // of the three together (z first)
   int *abort;                     // set by a workgroup that gave up waiting
+  int polls, from;                // polls in vain before it does, from exchange `from` on (before: kPolls)
 };
 
 template <typename R> struct IeLaunch {

@@ -660,7 +660,8 @@ __global__ void k_cg_fill(uint4 *__restrict__ p, long n, int *__restrict__ abort
 
 // The first four waves: sum of nb <= 512 published partials, as PartialSum<256> adds them, of which
 // they leave 4 terms in total, to be added in order after a barrier.
-__device__ __forceinline__ void published_sum(const double *v, int nb, double *total, int *abort, int *gave_up) {
+__device__ __forceinline__ void published_sum(const double *v, int nb, double *total, int polls, int *abort,
+                                              int *gave_up) {
   const int tid = threadIdx.x;
   if (tid >= 256) return;
   unsigned long long t[2];
@@ -669,7 +670,7 @@ __device__ __forceinline__ void published_sum(const double *v, int nb, double *t
 #pragma unroll
     for (int u = 0; u < 2; ++u) t[u] = u * 256 + tid < nb ? poll(v + u * 256 + tid) : 0;
     if (t[0] != Bits<double>::none && t[1] != Bits<double>::none) break;
-    if (give_up(spin, abort)) {
+    if (give_up(spin, polls, abort)) {
       *gave_up = 1;
       break;
     }
@@ -819,7 +820,7 @@ template <typename R, int BLK, int SH> __global__ void __launch_bounds__(kCgThre
       for (int i = 0; i < 4; ++i) v[i] = i < n ? (csum[a + i][0] + csum[a + i][1]) + (csum[a + i][2] + 0.0) : 0.0;
       publish(c.pap + (size_t)slot * d.vec_blocks + vb0 + tid, ((v[0] + v[1]) + v[2]) + v[3]);
     }
-    published_sum(c.pap + (size_t)slot * d.vec_blocks, d.vec_blocks, tot[0], c.abort, &gave_up);
+    published_sum(c.pap + (size_t)slot * d.vec_blocks, d.vec_blocks, tot[0], 2 * it < c.from ? kPolls : c.polls, c.abort, &gave_up);
     __syncthreads();
     if (gave_up) break;
     if (it > 0) {
@@ -848,13 +849,14 @@ template <typename R, int BLK, int SH> __global__ void __launch_bounds__(kCgThre
         publish(pz + ei[u], zi);
         zz += zi * zi * ri[u];
       }
+    const int polls = 2 * it + 1 < c.from ? kPolls : c.polls;
     zz = wave_sum(zz);
     if (lane == 0) zsum[w >> 2][q] = zz;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // clearings are complete
     __syncthreads();
     if (tid < vb1 - vb0)
       publish(c.rz + (size_t)slot * d.vec_blocks + vb0 + tid, (zsum[tid][0] + zsum[tid][1]) + (zsum[tid][2] + zsum[tid][3]));
-    published_sum(c.rz + (size_t)slot * d.vec_blocks, d.vec_blocks, tot[1], c.abort, &gave_up);
+    published_sum(c.rz + (size_t)slot * d.vec_blocks, d.vec_blocks, tot[1], polls, c.abort, &gave_up);
     {
       unsigned long long t[GH];
       int spin = 0;
@@ -865,7 +867,7 @@ template <typename R, int BLK, int SH> __global__ void __launch_bounds__(kCgThre
 #pragma unroll
         for (int u = 0; u < GH; ++u) wait = wait || t[u] == Bits<double>::none;
         if (!wait) break;
-        if (give_up(spin, c.abort)) {
+        if (give_up(spin, polls, c.abort)) {
           gave_up = 1;
           break;
         }

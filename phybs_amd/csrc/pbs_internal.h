@@ -71,6 +71,8 @@ struct TileDev {
 template <typename R> struct ContribWidth { static constexpr int value = 3; };
 template <> struct ContribWidth<float> { static constexpr int value = 4; };
 
+constexpr int kPolls = 1 << 20;  // resident kernels: polls in vain before giving up, by default (about a second)
+
 template <typename R> struct Ring {
   R *b[4];  // each: 3 nn values, node-major (xyz of a node together)
 };

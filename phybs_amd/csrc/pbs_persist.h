@@ -25,6 +25,7 @@ struct PersistDev {
   double *part;   // kPersistSlots slots of (energy, |g|^2) per part
   long xch_bytes; // of xch and part together (part follows xch)
   int *abort;     // set by a workgroup that gave up waiting
+  int polls, from; // polls in vain before it does, from pass `from` of the launch on (before: kPolls)
 };
 
 template <typename R> struct PersistLaunch {

@@ -200,6 +200,7 @@ k_persist(DevParams p, PersistDev d, Ctrl *__restrict__ ctrl, Ring<R> ring, cons
   for (int pass = 0; pass < max_passes; ++pass) {
     const int slot = pass & (kPersistSlots - 1);
     const int before = (pass + kPersistSlots - 1) & (kPersistSlots - 1);
+    const int polls = pass < d.from ? kPolls : d.polls;
     if (w == CW && pending) read_sums(before, false);
     double e_el = 0.0;
     // forces of this workgroup's tets into the contribution slots; phase 1: the stiffness diagonal
@@ -272,7 +273,7 @@ k_persist(DevParams p, PersistDev d, Ctrl *__restrict__ ctrl, Ring<R> ring, cons
 #pragma unroll
           for (int u = 0; u < 4; ++u) wait = wait || be[u] == Bits<double>::none || bg[u] == Bits<double>::none;
           if (!wait) break;
-          if (give_up(spin, d.abort)) {
+          if (give_up(spin, polls, d.abort)) {
             gave_up = 1;
             break;
           }
@@ -347,7 +348,7 @@ k_persist(DevParams p, PersistDev d, Ctrl *__restrict__ ctrl, Ring<R> ring, cons
         for (int u = 0; u < GH; ++u) gv[u] = gnode[u] >= 0 ? poll(xch + (size_t)slot * 3 * N + gnode[u]) : 0;
 #pragma unroll
         for (int u = 0; u < GH; ++u) wait = wait || gv[u] == Bits<R>::none;
-        if (wait && give_up(spin, d.abort)) {
+        if (wait && give_up(spin, polls, d.abort)) {
           gave_up = 1;
           break;
         }

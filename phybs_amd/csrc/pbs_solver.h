@@ -55,6 +55,11 @@ struct pbs_solver {
   TilePlan plan;
   size_t lds_budget = 65536;
   PersistDev persist{};       // resident descent loop of a small mesh (nparts 0: not used)
+  // The resident loops' bounded waits, and how the last descent loop and CG solve ran (PBS_LOOP_*); one
+  // that gave up once leaves its loop to the launches from then on.
+  int resident_polls = kPolls, resident_from = 0;
+  bool descent_gave_up = false, cg_gave_up = false;
+  int descent_loop = 0, cg_loop = 0;
   std::vector<float> rest_h;
   float *stage = nullptr;     // 3N float AoS staging
   double *stage64 = nullptr;  // 3N double AoS staging

@@ -1,0 +1,91 @@
+"""Which loop a step or solve ran in, and what happens when a resident launch's bounded waits end: the
+host sets how often a workgroup looks in vain before it gives up, so every kernel ends by itself, and
+the step or solve goes on through the launches from the same start, with their bits."""
+import sys
+
+import numpy as np
+import pytest
+
+import meshgen as M
+import phybs_amd as P
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print("[gpu-test]", *a, flush=True)
+    sys.stdout.flush()
+
+
+def solver(dims, **kw):
+    rest, tets = M.bar(*dims, 0.05)
+    s = P.Solver(rest, tets, M.clamp_x0(rest), P.default_params(**kw))
+    s.set_positions(M.twisted_state(rest, *dims, 0.05, 2.0, 0.005, 1))
+    return s
+
+
+def bits(s):
+    return s.positions(f64=True).view(np.uint64).copy(), s.velocities()[0].view(np.uint32).copy()
+
+
+@pytest.mark.parametrize("dims,kw,loop", [
+    ((1, 1, 1), dict(), P.LOOP_RESIDENT),
+    ((4, 4, 16), dict(precision=P.FP64, relgrad_tol=1e-4, max_iterations=5000), P.LOOP_RESIDENT),
+    ((17, 18, 60), dict(material=P.MAT_STRETCH), P.LOOP_RESIDENT),
+    ((24, 25, 60), dict(precision=P.FP64), P.LOOP_RESIDENT),                # 39,650 nodes
+    ((24, 25, 61), dict(), P.LOOP_LAUNCHES),                                # 40,300: more than it takes
+    ((4, 4, 16), dict(graph_passes=32), P.LOOP_LAUNCHES),
+    ((4, 4, 16), dict(tile_tets=64), P.LOOP_LAUNCHES),
+    ((4, 4, 16), dict(precision=P.FP64, relgrad_tol=1e-4, max_iterations=5000, mixed_switch=1e-3), P.LOOP_LAUNCHES),
+])
+def test_descent_loop_taken(dims, kw, loop):
+    say("loop of a step", dims, kw)
+    s = solver(dims, **kw)
+    assert s.last_loops() == (P.LOOP_NONE, P.LOOP_NONE)
+    s.step()
+    assert s.last_loops() == (loop, P.LOOP_NONE)
+    s.set_profiling(1)
+    s.step()
+    assert s.last_loops() == (P.LOOP_LAUNCHES, P.LOOP_NONE)
+    s.close()
+
+
+@pytest.mark.parametrize("precision", [P.FP32, P.FP64])
+@pytest.mark.parametrize("dims,blocks,scalar", [((1, 1, 1), True, True), ((16, 16, 60), True, True),
+                                                ((20, 20, 80), None, True),   # two shares: 3x3 blocks in FP32
+                                                ((30, 30, 135), False, True), ((31, 31, 130), False, False)])
+def test_cg_loop_taken(dims, blocks, scalar, precision):
+    """3x3 blocks (backward Euler), scalar values (projective dynamics)."""
+    say("loop of a solve", dims, precision)
+    if blocks is None:
+        blocks = precision == P.FP32
+    s = solver(dims, precision=precision)
+    for call, resident in ((s.implicit_step, blocks), (s.pd_step, scalar)):
+        call()
+        assert s.last_loops()[1] == (P.LOOP_RESIDENT if resident else P.LOOP_LAUNCHES)
+    s.set_profiling(1)
+    s.pd_step()
+    assert s.last_loops()[1] == P.LOOP_LAUNCHES
+    s.close()
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(precision=P.FP64, relgrad_tol=1e-4, max_iterations=20000)])
+def test_descent_goes_on_after_giving_up(kw):
+    dims = (12, 12, 50)
+    a, b = solver(dims, **kw), solver(dims, graph_passes=32, **kw)
+    a.set_resident_polls(1)
+    say("descent gives up", kw)
+    sa, sb = a.step(), b.step()
+    assert a.last_loops()[0] == P.LOOP_GAVE_UP and b.last_loops()[0] == P.LOOP_LAUNCHES
+    assert (sa.passes, sa.rollbacks, sa.converged) == (sb.passes, sb.rollbacks, sb.converged)
+    for loop in (P.LOOP_LAUNCHES, P.LOOP_RESIDENT):
+        for p, q in zip(bits(a), bits(b)):
+            assert np.array_equal(p, q)
+        if loop == P.LOOP_RESIDENT:
+            a.set_resident_polls(0)
+        a.step(), b.step()
+        assert a.last_loops()[0] == loop
+    for p, q in zip(bits(a), bits(b)):
+        assert np.array_equal(p, q)
+    a.close()
+    b.close()
