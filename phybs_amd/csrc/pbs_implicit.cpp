@@ -210,17 +210,22 @@ int cg_solve(pbs_solver *s, ImplicitState *S, IeDev &dev, CgGraphs &G, double to
     S->cg.from = s->resident_from;
     s->cg_loop = PBS_LOOP_RESIDENT;
     hipError_t e = IeLaunch<R>::resident(dev, S->cg, s->st);
-    int gave_up = 1;
+    int gave_up = 0;
     if (e == hipSuccess) {
       HIPCHK(hipMemcpyAsync(&c, dev.ctrl, sizeof(IeCtrl), hipMemcpyDeviceToHost, s->st));
       HIPCHK(hipMemcpyAsync(&gave_up, S->cg.abort, sizeof(int), hipMemcpyDeviceToHost, s->st));
       HIPCHK(hipStreamSynchronize(s->st));
     }
-    if (gave_up) {  // not launchable, or its workgroups did not all run: the launches, from the same start
+    if (e != hipSuccess || gave_up) {  // not launchable, or its workgroups did not all run: the launches
       (void)hipGetLastError();
       s->cg_gave_up = true;
       s->cg_loop = PBS_LOOP_GAVE_UP;
       c = IeCtrl{};
+      if (gave_up) {  // parts of x, the control block, are written: the same start again
+        HIPCHK(hipMemcpyAsync(dev.x, dev.p, sizeof(double) * 3 * (size_t)dev.n, hipMemcpyDeviceToDevice, s->st));
+        IeLaunch<R>::start(dev, s->st);
+        HIPCHK(hipGetLastError());
+      }
     }
   }
   int rc = c.done ? PBS_OK : timed ? cg_events(S) : cg_graph<R>(s, dev, G);

@@ -74,7 +74,8 @@ template <typename R> struct IeLaunch {
   static void dir(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
   static void spmv(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
   static void res(const IeDev &d, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-  // the whole loop after `start` as one cooperative launch; whether the device can hold it
+  // the whole loop after `start` as one cooperative launch, which keeps the start vector in d.p; whether
+  // the device can hold it
   static hipError_t resident(const IeDev &d, const CgDev &c, hipStream_t st);
   static bool resident_fits(const CgDev &c, int scalar, int device);
   static void finish(const DevMesh<R> &m, const DevParams &p, float h, const IeDev &d, hipStream_t st);

@@ -652,9 +652,13 @@ __global__ void __launch_bounds__(kBlock) k_ie_res(IeDev d) {
 // z and r.z of k have been, and clears its own.  Both clearings are waited for before it publishes
 // the next r.z, and a slot is polled again only by who has that one, or the p.Ap that follows it.
 // ---------------------------------------------------------------------------------------------
-__global__ void k_cg_fill(uint4 *__restrict__ p, long n, int *__restrict__ abort) {
+// Clears the exchange buffers (n times 16 bytes, at least one for each of the 3N entries of x) and keeps
+// the start vector in p, which k_cg does not use: where some workgroups give up in the last iteration
+// and others do not, the latter have written their part of x, and the launches begin again from p.
+__global__ void k_cg_fill(IeDev d, uint4 *__restrict__ xch, long n, int *__restrict__ abort) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  if (i < n) xch[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  if (i < 3 * (long)d.n) d.p[i] = d.x[i];
   if (i == 0) *abort = 0;
 }
 
@@ -1165,7 +1169,7 @@ template <typename R> bool IeLaunch<R>::resident_fits(const CgDev &c, int scalar
 }
 template <typename R> hipError_t IeLaunch<R>::resident(const IeDev &d, const CgDev &c, hipStream_t st) {
   const long n16 = c.xch_bytes / 16;
-  hipLaunchKernelGGL(k_cg_fill, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, (uint4 *)c.z, n16, c.abort);
+  hipLaunchKernelGGL(k_cg_fill, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, d, (uint4 *)c.z, n16, c.abort);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   IeDev dd = d;

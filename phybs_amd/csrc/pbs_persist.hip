@@ -22,8 +22,8 @@
 // cleared what pass k - 6 and those before it published: it never meets what pass k - 8 left.
 //
 // Waiting ends: the launch is cooperative, so all workgroups are resident, and every poll is bounded;
-// a workgroup that gives up sets *abort and ends, so do the others, nothing is written back, and the
-// host runs the step through the three launches.
+// a workgroup that gives up sets *abort and ends, so do the others (one that has all values of the last
+// pass writes its nodes back first), and the host starts the step again on the three launches.
 //
 // Bound: the chain of one pass, not bytes or arithmetic.  43 K tets, FP64: about 7,400 cycles, of
 // which tets 2,000, gather 1,500, node step 700, the exchange of positions across the XCDs 2,500, the

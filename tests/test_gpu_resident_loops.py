@@ -89,3 +89,37 @@ def test_descent_goes_on_after_giving_up(kw):
         assert np.array_equal(p, q)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("iterations", [1, 2, 10000])
+@pytest.mark.parametrize("kind", ["implicit", "pd"])
+def test_solve_goes_on_after_giving_up(kind, iterations):
+    """Limits from one look to more than a wait takes, from the first exchange on and on the last one
+    alone (a solve that ends after one or two iterations): there, some workgroups see all values and end
+    with a result while others give up."""
+    dims = (20, 20, 80)
+
+    def step(s):
+        if kind == "implicit":
+            return s.implicit_step(params=P.implicit_params(cg_max_iterations=iterations)).cg_iterations
+        return s.pd_step(params=P.pd_params(cg_max_iterations=iterations, iterations=1)).cg_iterations
+
+    ref = solver(dims)
+    ref.set_profiling(1)
+    its = step(ref)
+    want = bits(ref)
+    ref.close()
+    for start in (0, 2 * its - 1):
+        loops = {}
+        for polls in (1, 2, 4, 8, 12, 16, 24, 64):
+            s = solver(dims)
+            s.set_resident_polls(polls, start)
+            say("solve gives up", kind, iterations, start, polls)
+            got_its = step(s)
+            loops[polls] = s.last_loops()[1]
+            assert got_its == its
+            for p, q in zip(bits(s), want):
+                assert np.array_equal(p, q)
+            s.close()
+        say("loops", loops)
+        assert loops[1] == P.LOOP_GAVE_UP
