@@ -393,9 +393,9 @@ __device__ __forceinline__ f32x4 bf4(bf16x4 v) {
 }
 // SiLU and its derivative from one exponential: s = 1 / (1 + e^-z), refined to the last bit or two
 // (e^-z capped where s is no longer a normal number).
-__device__ __forceinline__ void silu_both(float z, float &v, float &dv) {
+__device__ __forceinline__ void silu_both(float z, float &s, float &v, float &dv) {
   const float d = 1.0f + fminf(expf(-z), 1e37f);
-  float s = __builtin_amdgcn_rcpf(d);
+  s = __builtin_amdgcn_rcpf(d);
   s = fmaf(fmaf(-d, s, 1.0f), s, s);
   v = z * s;
   v = fmaf(fmaf(-v, d, z), s, v);  // the quotient z / d to the last bit: it is rounded to BF16 next
@@ -403,14 +403,18 @@ __device__ __forceinline__ void silu_both(float z, float &v, float &dv) {
 }
 
 // Whether a hidden activation v = SiLU(z), z = z0 + z1 + z2 + z3, is as near to the middle of two BF16
-// values as its own rounding error (about 1 in 2000).  One rounded to the other neighbour of an exact
-// evaluation's changes the sample's gradient in the third digit, far more than FP32 rounding does, so
-// those are formed again in FP64, by the whole wave (each by its own lane alone: 28 instead of 23 us a
-// batch; without it 20).  Relative error of the gradient against 64 bits, 30 seeds each of 65 to 30,000
-// samples: at most 1.7e-7, without it up to 7e-5; a bound of 1e-7 instead of 1.5e-7 misses a few.
-__device__ __forceinline__ bool near_middle(float v, float z0, float z1, float z2, float z3) {
+// values as its own rounding error: z's, 1.5e-7 of the sum of |z_i|, times SiLU's slope, and the
+// exponential's, which reaches 1 - s of v (about 1 in 2000 are, saturated units among them; without the
+// slope nine in ten are at z = -10, and a batch of such units takes 11 times as long as a usual one).  One
+// rounded to the other neighbour of an exact evaluation's changes the sample's gradient in the third
+// digit, far more than FP32 rounding does, so those are formed again in FP64, by the whole wave (each by
+// its own lane alone: 28 instead of 23 us a batch; without it 20).  Relative error of the gradient
+// against 64 bits, 30 seeds each of 65 to 30,000 samples: at most 1.7e-7, without it up to 7e-5; a bound
+// of 1e-7 instead of 1.5e-7 misses a few.
+__device__ __forceinline__ bool near_middle(float s, float v, float dv, float z0, float z1, float z2, float z3) {
   const float mid = __builtin_bit_cast(float, (__builtin_bit_cast(unsigned, v) & 0xffff0000u) | 0x8000u);
-  return fabsf(v - mid) <= 1.5e-7f * (fabsf(z0) + fabsf(z1) + fabsf(z2) + fabsf(z3));
+  const float sum = fabsf(z0) + fabsf(z1) + fabsf(z2) + fabsf(z3);
+  return fabsf(v - mid) <= 1.5e-7f * fmaf(fabsf(dv), sum, 2.0f * (1.0f - s) * fabsf(v));
 }
 
 __global__ void __launch_bounds__(256) k_mlp_train(MlpDev net, const float *__restrict__ ds_x,
@@ -502,11 +506,11 @@ __global__ void __launch_bounds__(256) k_mlp_train(MlpDev net, const float *__re
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          float v, dv;
-          silu_both((c[0][i] + c[1][i]) + (c[2][i] + c[3][i]), v, dv);
+          float s, v, dv;
+          silu_both((c[0][i] + c[1][i]) + (c[2][i] + c[3][i]), s, v, dv);
           ds[l][mt][i] = dv;
           hn[mt][i] = (short)f2bf(v);
-          again |= (near_middle(v, c[0][i], c[1][i], c[2][i], c[3][i]) ? 1u : 0u) << (4 * mt + i);
+          again |= (near_middle(s, v, dv, c[0][i], c[1][i], c[2][i], c[3][i]) ? 1u : 0u) << (4 * mt + i);
           S.h[l][16 * mt + 4 * q + i][16 * w + r] = (unsigned short)hn[mt][i];
         }
       }
