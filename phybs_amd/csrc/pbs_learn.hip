@@ -391,14 +391,16 @@ __device__ __forceinline__ f32x4 bf4(bf16x4 v) {
   for (int i = 0; i < 4; ++i) f[i] = bf2f((unsigned short)v[i]);
   return f;
 }
-// SiLU and its derivative from one exponential: s = 1 / (1 + e^-z), refined to the last bit or two
-// (e^-z capped where s is no longer a normal number).
+// SiLU and its derivative from one exponential: s = 1 / (1 + e^-z), refined to the last bit or two.  Zero
+// below -85, where s leaves the normal numbers (e^-z is capped there), so that any finite z gives 0 and
+// 0; above 17, s is 1 and the quotient needs no refinement, which infinity would not survive.
 __device__ __forceinline__ void silu_both(float z, float &s, float &v, float &dv) {
   const float d = 1.0f + fminf(expf(-z), 1e37f);
   s = __builtin_amdgcn_rcpf(d);
   s = fmaf(fmaf(-d, s, 1.0f), s, s);
+  s = z < -85.0f ? 0.0f : s;
   v = z * s;
-  v = fmaf(fmaf(-v, d, z), s, v);  // the quotient z / d to the last bit: it is rounded to BF16 next
+  if (d > 1.0f) v = fmaf(fmaf(-v, d, z), s, v);  // the quotient z / d to the last bit: it is rounded to BF16 next
   dv = s * fmaf(z, 1.0f - s, 1.0f);
 }
 

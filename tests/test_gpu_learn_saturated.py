@@ -81,3 +81,19 @@ def test_saturated_units_cost_no_more():
         s.close()
     say("saturated units, us a call", {b: round(1e6 * v, 1) for b, v in times.items()})
     assert max(times.values()) <= 2 * times[0.0]
+
+
+@pytest.mark.parametrize("z", [-80.0, -84.9, -85.1, -90.0, -1e4, -1e20, -1e36, 20.0, 120.0])
+def test_units_at_the_ends_of_the_range(z):
+    """One unit of the first layer with a bias of z, the others usual: loss and gradient against 64 bits
+    (SiLU and its slope are 0 for any large negative z).  Tolerance as above."""
+    s, model, f, t = setup(0.0, 3, 257)
+    model[1152 + 5] = z
+    s.learn_set_model(model, SCALES)
+    loss, g = s.learn_loss_grad(f, t)
+    with np.errstate(over="ignore"):
+        lref, gref = loss_grad_64(model, f, t)
+    err = np.linalg.norm(g - gref) / np.linalg.norm(gref)
+    say("a unit at", z, "loss", loss, lref, "grad rel err %.2e" % err)
+    assert loss == pytest.approx(lref, rel=1e-6) and err <= 2e-6
+    s.close()
