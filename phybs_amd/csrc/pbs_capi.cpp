@@ -266,8 +266,10 @@ template <typename R> static int alloc_impl(pbs_solver *s) {
   return rc ? PBS_ERR_HIP : PBS_OK;
 }
 
-// The resident descent loop (pbs_persist.hip) of a single mesh with the default tile size and graph
-// length: plan, device arrays and exchange buffers, where the mesh fits it.  Parts of at least 21
+// The resident descent loop (pbs_persist.hip) of a single mesh with the default tile size: plan, device
+// arrays and exchange buffers, where the mesh fits it.  Made by the first step that can take it, so that a
+// handle for the material calls, training or the implicit steps does not pay for it (creating one of
+// 43 K tets takes 8.8 ms, with it 12.7).  Parts of at least 21
 // nodes (one wave's; 16 or 12 are no faster, 32 take 6 to 14 % more per pass at 1.5 K tets), at most
 // one per CU, at most 168 nodes each (8 waves of 21), so 43,000 nodes at most.  It is the faster path
 // up to there: us per pass of a step, resident against launches, FP32 96 passes (FP64 rel-grad in
@@ -535,10 +537,7 @@ static int create_impl(int ninst, const int *node_off, const int *tet_off, const
   if (rc) return fail(rc);
   rc = p->precision == PBS_FP64 ? setup_impl<double>(s, mask) : setup_impl<float>(s, mask);
   if (rc) return fail(rc);
-  if (tile_tets == 0 && !inst_tiles) {
-    rc = p->precision == PBS_FP64 ? persist_setup<double>(s) : persist_setup<float>(s);
-    if (rc) return fail(rc);
-  }
+  s->persist_tried = tile_tets != 0 || inst_tiles;
   if (nodes) {
     rc = p->precision == PBS_FP64 ? set_positions_impl<double>(s, nodes) : set_positions_impl<float>(s, nodes);
     if (rc) return fail(rc);
@@ -1011,6 +1010,21 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
   const int G = s->p.graph_passes == 0 ? 32 : s->p.graph_passes;
   const bool use_graph = G > 0;
   const int period = s->prof_period;
+  // the resident loop: the default graph length, no timing of single kernels, no mixed mode
+  const bool relg = s->dp.relgrad_tol > 0;
+  const bool mixed = use_graph && relg && s->p.mixed_switch > 0 && sizeof(R) == 8;
+  const bool resident = s->p.graph_passes == 0 && !period && !mixed;
+  if (resident && !s->persist_tried) {
+    s->persist_tried = true;
+    int dev = s->device;  // (the calling thread's may be another)
+    (void)hipGetDevice(&dev);
+    if (dev != s->device) HIPCHK(hipSetDevice(s->device));
+    if (persist_setup<R>(s)) {  // no memory for it: the launches
+      (void)hipGetLastError();
+      s->persist = PersistDev{};
+    }
+    if (dev != s->device) HIPCHK(hipSetDevice(dev));
+  }
   s->dp.f32math = 0;  // step start, warm start and eager passes: FP64 arithmetic
   HIPCHK(hipEventRecord(s->ev0, s->st));
   int i = -1;
@@ -1032,7 +1046,6 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
     int rc = begin_step();
     if (rc) return rc;
   }
-  const bool relg = s->dp.relgrad_tol > 0;
   const long cap = relg ? (long)s->p.max_iterations + 256 : (long)s->p.iterations + 256;
   s->descent_loop = PBS_LOOP_LAUNCHES;
   long launched = 0;
@@ -1062,7 +1075,6 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
   // resolve the remaining gradient: the step goes on in FP64 from the restored iterate, with the
   // step length the step started with.
   constexpr double kMixedNoise = 2e-4;
-  const bool mixed = use_graph && relg && s->p.mixed_switch > 0 && sizeof(R) == 8;
   bool fp64_phase = !mixed;
   std::vector<float> alpha0;
   std::vector<int> rb0;
@@ -1075,8 +1087,7 @@ template <typename R> static int step_impl(pbs_solver *s, const float *ext, floa
     }
   }
   while (true) {
-    // the resident loop: the default graph length, no timing of single kernels, no mixed mode
-    if (s->persist.nparts > 0 && !s->descent_gave_up && s->p.graph_passes == 0 && !period && !mixed) {
+    if (resident && s->persist.nparts > 0 && !s->descent_gave_up) {
       s->persist.polls = s->resident_polls;
       s->persist.from = s->resident_from;
       // one launch runs the step (at most 4096 passes at a time)

@@ -55,6 +55,7 @@ struct pbs_solver {
   TilePlan plan;
   size_t lds_budget = 65536;
   PersistDev persist{};       // resident descent loop of a small mesh (nparts 0: not used)
+  bool persist_tried = false; // it is made by the first step that can take it
   // The resident loops' bounded waits, and how the last descent loop and CG solve ran (PBS_LOOP_*); one
   // that gave up once leaves its loop to the launches from then on.
   int resident_polls = kPolls, resident_from = 0;

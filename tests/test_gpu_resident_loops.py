@@ -123,3 +123,27 @@ def test_solve_goes_on_after_giving_up(kind, iterations):
             s.close()
         say("loops", loops)
         assert loops[1] == P.LOOP_GAVE_UP
+
+
+def test_creation_does_not_pay_for_the_resident_loop():
+    """A handle that may never step is created in the time of one that cannot run the resident loop (the
+    same tiles, by an explicit size); the first step makes what the loop needs."""
+    import time
+
+    rest, tets = M.bar(12, 12, 50, 0.05)
+    mask = M.clamp_x0(rest)
+    s = P.Solver(rest, tets, mask, P.default_params())
+    tile = int(s.get_params().tile_tets)
+    s.step()
+    assert s.last_loops()[0] == P.LOOP_RESIDENT
+    s.close()
+    times = {0: [], tile: []}
+    for _ in range(15):
+        for k in times:
+            t0 = time.perf_counter()
+            s = P.Solver(rest, tets, mask, P.default_params(tile_tets=k))
+            times[k].append(time.perf_counter() - t0)
+            s.close()
+    med = {k: 1e3 * float(np.median(v[3:])) for k, v in times.items()}
+    say("creation, ms by tile size", med)
+    assert med[0] <= 1.2 * med[tile]
