@@ -8,17 +8,20 @@ namespace pbs {
 void build_block_rows(const TilePlan &P, BlockRows &B) {
   B = BlockRows();
   const int N = P.nn;
-  std::vector<int> row_off(N + 1, 0), cols, tmp;
+  std::vector<int> row_off(N + 1, 0), cols, tmp, last(N, -1);  // last: the last row that took a column
   cols.reserve((size_t)N * 16);
   for (int n = 0; n < N; ++n) {
-    tmp.clear();
+    tmp.assign(1, n);
+    last[n] = n;
     for (int e = P.inc_off[n]; e < P.inc_off[n + 1]; ++e) {
-      const int t = P.inc[e] >> 2;
-      for (int c = 0; c < 4; ++c) tmp.push_back(P.tets_new[4 * (size_t)t + c]);
+      const int *q = &P.tets_new[4 * (size_t)(P.inc[e] >> 2)];
+      for (int c = 0; c < 4; ++c)
+        if (last[q[c]] != n) {
+          last[q[c]] = n;
+          tmp.push_back(q[c]);
+        }
     }
-    tmp.push_back(n);
     std::sort(tmp.begin(), tmp.end());
-    tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
     cols.insert(cols.end(), tmp.begin(), tmp.end());
     row_off[n + 1] = (int)cols.size();
   }
