@@ -72,8 +72,10 @@ typedef struct pbs_params {
   int tile_tets;        /* max tets per workgroup of the tile pass (16..4096); 0 = chosen from mesh size and
                            LDS; -1 = autotuned at creation (64, 128, 256, 512 timed on 32 passes) */
   int graph_passes;     /* descent passes per captured HIP graph replay: 0 = 32 (a single mesh of at most
-                           40,000 nodes with default tile_tets: the whole loop in one launch instead,
-                           the same iterates), -1 = no graph (kernels launched one by one) */
+                           40,000 nodes with default tile_tets: the whole loop in one launch instead;
+                           the same iterates bit for bit while the loop decides alike -- the energies
+                           and gradient norms it compares are sums in another order, equal to within
+                           their last bits), -1 = no graph (kernels launched one by one) */
   double mixed_switch;  /* PBS_FP64 with graphs only (no reference counterpart): while |g|/|g_0| of
                            the last graph replay is above this, the tile pass forms F in FP64 and
                            evaluates the per-tet forces in FP32 (neo-Hookean: from H = F - I) with
@@ -215,8 +217,8 @@ int pbs_reset_kernel_times(pbs_solver *s);
  * every n-th graph replay (every n-th pass without graphs) are timed, the timed replay's passes
  * being launched one by one instead of from the graph.  Launches that run after the loop has
  * stopped within a replay are not counted.  Any period > 0 times every CG replay.  A timed solver
- * launches its kernels one by one where an untimed one of its size runs a resident loop; the iterates
- * are the same. */
+ * launches its kernels one by one where an untimed one of its size runs a resident loop (CG: the same
+ * bits; descent: see graph_passes). */
 int pbs_set_profiling(pbs_solver *s, int period);
 /* How the last step's descent loop and the last CG solve ran: kernel by kernel, as one resident launch,
  * or as a resident launch of which some workgroup gave up waiting for another, and then kernel by kernel

@@ -412,7 +412,7 @@ __device__ __forceinline__ double sqrt_ratio(double v, double w) {
 // after one of at most 2e-4 (FP32) / 1e-8 (FP64): 3 steps at up to 25 % stretch in FP32, 4 in FP64, 5 at
 // kappa = 20.  Largest entry's error over 2e5 random F of kappa <= 20: 1.8e-7 / 3.1e-16 (the fixed 4 /
 // 5 scaled steps above: 4.0e-7 / 1.7e-14).  Bound by its vector instructions: the tile pass on 6.3 M
-// tets takes 102 us instead of 128 in FP32, 206 instead of 245 in FP64.
+// tets twisted by 30 degrees takes 101 us instead of 130 in FP32, 208 instead of 257 in FP64.
 template <typename R> __device__ __forceinline__ bool polar_rotation_fast(const R *F, R *Rot) {
   constexpr R kLast = sizeof(R) == 4 ? (R)2e-4 : (R)1e-8;
   R X[9];

@@ -309,8 +309,8 @@ __device__ __forceinline__ void tile_body(const DevParams &p, int chk, const R *
   float4 *srest = (float4 *)(smem + tile_rest_offset<R>(td));
   const int nthr = blockDim.x;
   // neo-Hookean: tet tid's local ids and slots, loaded before the staging so that they arrive with
-  // it.  The stretch material's kernel would lose a wave per SIMD to the 4 registers it holds across
-  // the staging (FP32 137 -> 147 us), so it loads them after the barrier.
+  // it.  The FP64 stretch kernel would lose waves to the 4 registers it holds across the staging (6.3 M
+  // tets, 208 -> 261 us; FP32 101 -> 98), so the stretch material loads them after the barrier.
   constexpr bool PRE = MAT == 0;
   const uint4 lp0 = PRE && tid < ti.tet_cnt ? td.tet_lp[(size_t)ti.tet_start + tid] : make_uint4(0, 0, 0, 0);
   const C mu = (C)td.inst_mu[ti.inst], lam = (C)td.inst_lam[ti.inst];
@@ -373,13 +373,15 @@ __device__ __forceinline__ void tile_body(const DevParams &p, int chk, const R *
 
 // F32M (FP64 state only): the per-tet arithmetic in FP32 after F (the mixed mode's early passes).
 //
-// Bound: the staging's scattered halo reads and the LDS traffic of contributions, not the arithmetic
-// (forces with a third fewer FP32 instructions left its time as it was).  So node data is node-major
+// Bound (neo-Hookean): the staging's scattered halo reads and the LDS, busy in 77 % (FP32) and 68 %
+// (FP64) of the cycles, half of that with bank conflicts.  The vector units issue in 86 % and 53 %, but
+// forces with a third fewer FP32 instructions left the time as it was.  So node data is node-major
 // (the three components of a node in one cache line, its rest position one 16-byte read, instead of
 // three lines each), the first lstride ids and the thread's contribution run are read with the
-// descriptor instead of after it, and the neo-Hookean force takes one 3x3 product (neo_force).  Per
-// launch on 6.3 M tets (64x64x256 cells), before -> now: FP32 73 -> 69 us, FP64 139 -> 115, stretch
-// FP32 121 -> 122.  The FP64 neo-Hookean kernel is held to 5 waves per SIMD (at most 102 VGPRs, no
+// descriptor instead of after it, and the neo-Hookean force takes one 3x3 product (neo_force).  Average
+// of a 64-pass step's launches on 6.3 M tets (64x64x256 cells, twisted by 30 degrees), with planes and
+// three products -> now: FP32 78 -> 76 us, FP64 133 -> 123; stretch FP32 134 -> 130, FP64 259 -> 257,
+// with polar_rotation_fast 101 and 208 (bound by its vector instructions).  The FP64 neo-Hookean kernel is held to 5 waves per SIMD (at most 102 VGPRs, no
 // spilling), as many as the LDS of 256-tet tiles allows (30.8 KB: 5 workgroups per CU).  6 waves with
 // 224-tet tiles spill (130 us), 4 waves 114 us.
 template <typename R, int MAT, bool F32M>

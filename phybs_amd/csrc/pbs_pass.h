@@ -1,7 +1,7 @@
 // pbs_pass.h -- device code shared by the kernels of the descent pass: the rest shape and force of
 // one tet, the Chebyshev schedule and the loop control.  The launches of a pass (pbs_kernels.hip)
 // and the resident descent kernel (pbs_persist.hip) evaluate the same functions, so their iterates
-// agree bitwise.
+// agree bitwise while the loop's decisions do.
 #pragma once
 #include <type_traits>
 

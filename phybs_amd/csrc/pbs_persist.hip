@@ -31,8 +31,10 @@
 // for) are off that chain on all but check passes.  Wall time of a step, three launches -> resident:
 // 1.5 K tets FP32, 96 passes, 876 -> 276 us; 43 K tets FP64, rel-grad 1e-4, 29.4 -> 7.3 ms.
 //
-// Iterates are bitwise those of the three launches (same functions, contributions added in the same
-// groups and order); the energy and |g|^2 are FP64 sums in another fixed order.
+// Iterates are bitwise those of the three launches as long as the loop decides alike (same functions,
+// contributions added in the same groups and order).  The energy and |g|^2 are FP64 sums in another
+// fixed order, so a decision can differ where one of them is within its last bits of the other side of
+// a comparison; from there on alpha, the budget and the iterates do.
 #include <algorithm>
 
 #include "pbs_exchange.h"
